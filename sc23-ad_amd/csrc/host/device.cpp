@@ -323,6 +323,162 @@ int order_by_level(const std::vector<int>& lev, const std::vector<int>& chain_be
   return maxlev_all;
 }
 
+// Row-parallel layout of an integer smoother factor (k_tri_chain_rp).
+//
+// A level is cut into pieces of at most 64 waves / lanes rows (rows of a level
+// are independent, so any cut is valid), and a piece takes about
+//   70 + 7.5 e + 10 log2(lanes) + (waves - 1) (2 + 4.5 e) ns,
+// e entries per lane: fitted to a sweep of the kernel on synthetic chains (40
+// chains of 256 levels; one wave of 4 / 10 entries 145 / 190 ns of which 45
+// are the launch's, each further wave 20 / 47 ns for its barrier and its share
+// of the CU's load bandwidth).  The layout with the least total over the
+// longest chain wins; so narrow levels get one wave, which needs no barrier,
+// and wide ones several.  With one chain, levels of more than single_wg_max
+// rows are otherwise launched one by one (about 4.4 us each, and 0.6 us per
+// narrow level): the row-parallel kernel takes the factor when its total is
+// below that.
+void plan_rp(TriPlan& plan, int n, const std::vector<int>& lbeg, const std::vector<int>& lpos,
+             const std::vector<int32_t>& lval, const std::vector<int>& lev_ptr,
+             const std::vector<int>& chain_lev, long long span, int single_wg_max) {
+  const char* env_rp = std::getenv("SC23AD_TRI_RP");
+  if ((env_rp && env_rp[0] == '0') || n <= 0 || n >= (1 << 29)) return;
+  const bool one_lane = env_rp && env_rp[0] == '1';
+  const bool force_groups = env_rp && env_rp[0] == '2';  // lanes per row even for short rows
+  const bool pow2 = std::getenv("SC23AD_RP_POW2") != nullptr;
+  // SC23AD_RP_LANES / SC23AD_RP_WAVES (tests): only layouts of so many lanes
+  // per row / waves
+  auto forced = [](const char* name) {
+    const char* e = std::getenv(name);
+    return e ? std::atoi(e) : 0;
+  };
+  const int only_lanes = forced("SC23AD_RP_LANES"), only_waves = forced("SC23AD_RP_WAVES");
+  const int nlev = static_cast<int>(lev_ptr.size()) - 1;
+  // the kernel keeps negated values
+  for (int32_t v : lval)
+    if (v == INT32_MIN) return;
+  // LDS ring: a dependency is read from it when no later position of its
+  // level's end has overwritten it, else (at least kEpFarLevels levels back)
+  // from global memory
+  int ring = 2;
+  while (ring < 32768 && ring < span) ring *= 2;
+  std::vector<int> lev_of(static_cast<size_t>(n));
+  for (int Lv = 0; Lv < nlev; ++Lv)
+    for (int idx = lev_ptr[Lv]; idx < lev_ptr[Lv + 1]; ++idx) lev_of[idx] = Lv;
+  auto is_far = [&](int idx, int dpos) {
+    return static_cast<long long>(lev_ptr[lev_of[idx] + 1]) - dpos > ring;
+  };
+  int md = 0, farq = 0, far_dist = 1 << 30;
+  for (int idx = 0; idx < n; ++idx) {
+    md = std::max(md, lbeg[idx + 1] - lbeg[idx]);
+    int c = 0;
+    for (int q = lbeg[idx]; q < lbeg[idx + 1]; ++q)
+      if (is_far(idx, lpos[q])) {
+        far_dist = std::min(far_dist, lev_of[idx] - lev_of[lpos[q]]);
+        ++c;
+      }
+    farq = std::max(farq, c);
+  }
+  if (farq > 0 && far_dist < dev::kEpFarLevels) return;
+  auto pieces_of = [&](size_t chain, int cap) {
+    long long k = 0;
+    for (int Lv = chain_lev[2 * chain]; Lv < chain_lev[2 * chain + 1]; ++Lv)
+      k += (lev_ptr[Lv + 1] - lev_ptr[Lv] + cap - 1) / cap;
+    return k;
+  };
+  const size_t nchain = chain_lev.size() / 2;
+  double best = 0;
+  int best_g = 0, best_e = 0, best_w = 0;
+  long long best_pieces = 0;
+  for (int lg = 0; (1 << lg) <= (one_lane || farq > 0 ? 1 : dev::kRpMaxLanes); ++lg)
+    for (int e : {4, 6, 8, 10, 12}) {
+      const int g = 1 << lg;
+      if (g * e < md || (g == 1 && e == 6) ||
+          static_cast<uint64_t>(n) * (g * e * 8) > UINT32_MAX)
+        continue;
+      if (g == 1 && force_groups && farq == 0 && md > 4) continue;
+      if (only_lanes > 0 && g != only_lanes) continue;
+      for (int w = 1; w <= dev::kRpMaxWaves; w = pow2 ? 2 * w : w + 1) {
+        if (w > 8 && (g > 1 || e > 4)) break;
+        const int cap = 64 * w / g;
+        if (only_waves > 0 && w != only_waves) continue;
+        long long most = 0;
+        for (size_t c = 0; c < nchain; ++c) most = std::max(most, pieces_of(c, cap));
+        if (dev::rp_lds_bytes(ring, static_cast<int>(std::min<long long>(most, 1 << 20))) >
+            dev::kTriBlockedMaxLds)
+          continue;
+        const double cost =
+            static_cast<double>(most) * (70 + 7.5 * e + 10 * lg + (w - 1) * (2 + 4.5 * e));
+        if (best_w == 0 || cost < best) {
+          best = cost;
+          best_g = g;
+          best_e = e;
+          best_w = w;
+          best_pieces = most;
+        }
+      }
+    }
+  if (best_w == 0) return;
+  if (nchain == 1) {
+    double segmented = 0;
+    bool wide = false;
+    for (int Lv = 0; Lv < nlev; ++Lv) {
+      const bool own = lev_ptr[Lv + 1] - lev_ptr[Lv] > single_wg_max;
+      wide = wide || own;
+      segmented += own ? 4400 : 600;
+    }
+    if (wide && segmented <= best) return;
+  }
+  const int cap = 64 * best_w / best_g;
+  std::vector<int> piece_ptr(1, 0), piece_chain;
+  for (size_t c = 0; c < nchain; ++c) {
+    piece_chain.push_back(static_cast<int>(piece_ptr.size()) - 1);
+    for (int Lv = chain_lev[2 * c]; Lv < chain_lev[2 * c + 1]; ++Lv)
+      for (int p = lev_ptr[Lv]; p < lev_ptr[Lv + 1]; p += cap)
+        piece_ptr.push_back(std::min(p + cap, lev_ptr[Lv + 1]));
+    piece_chain.push_back(static_cast<int>(piece_ptr.size()) - 1);
+  }
+  std::vector<int> rent(static_cast<size_t>(n) * best_g * best_e * 2, 0);
+  std::vector<int> ord;
+  for (int idx = 0; idx < n; ++idx) {
+    // far entries first (a row's integer sum is order-free), so the kernel
+    // loads far values for the first farq slots only
+    ord.clear();
+    for (int pass = 0; pass < 2; ++pass)
+      for (int q = lbeg[idx]; q < lbeg[idx + 1]; ++q)
+        if (is_far(idx, lpos[q]) == (pass == 0)) ord.push_back(q);
+    for (int m = 0; m < static_cast<int>(ord.size()); ++m) {
+      const size_t at =
+          ((static_cast<size_t>(idx) * best_g + m % best_g) * best_e + m / best_g) * 2;
+      const int dpos = lpos[ord[m]];
+      rent[at] = is_far(idx, dpos) ? ~(4 * dpos) : 4 * (dpos & (ring - 1));
+      rent[at + 1] = -lval[ord[m]];
+    }
+  }
+  plan.rent.alloc(sizeof(int) * rent.size());
+  plan.rent.upload(rent.data(), sizeof(int) * rent.size());
+  plan.rp_lev.alloc(sizeof(int) * piece_ptr.size());
+  plan.rp_lev.upload(piece_ptr.data(), sizeof(int) * piece_ptr.size());
+  plan.rp_chain.alloc(sizeof(int) * piece_chain.size());
+  plan.rp_chain.upload(piece_chain.data(), sizeof(int) * piece_chain.size());
+  dev::TriLayout& L = plan.layout;
+  L.rent = plan.rent.get();
+  L.rp_lev = plan.rp_lev.as<int>();
+  L.rp_chain = plan.rp_chain.as<int>();
+  L.rp_nchain = static_cast<int>(nchain);
+  L.rp_maxlev = static_cast<int>(best_pieces);
+  L.rp_ring = ring;
+  // a value is fenced before a load kRpMaxAhead levels ahead of its use, at
+  // least far_dist levels (so at least as many pieces) after its store
+  L.rp_fence = 32;
+  while (farq > 0 && 2 * L.rp_fence + dev::kRpMaxAhead <= far_dist) L.rp_fence *= 2;
+  L.rp_e = best_e;
+  L.rp_rows = 1;
+  L.rp_lanes = best_g;
+  L.rp_waves = best_w;
+  L.rp_farq = farq;
+  plan.nlaunch = 1;
+}
+
 // Level schedule of a triangular factor.  `chain_begin` (nchain + 1 row
 // boundaries) splits rows into independent contiguous chains (the BlockSOR
 // partition), each walked by one workgroup in a single launch; with one
@@ -589,75 +745,6 @@ void build_plan(TriPlan& plan, TriKind kind, int n, const std::vector<int>& rptr
       // every row of a level and about as many entries.
       L.ep_narrow = (maxlev_rows <= static_cast<size_t>(w) * 64 && overflowing(w, 4) * 16 <= nlev)
                         ? 1 : 0;
-      // Row-parallel mode for smoother factors with short rows: one lane per
-      // row for at most kRpMaxEntries dependencies, else (no far entries)
-      // 2-16 lanes of 8, 10 or 12 entries per row; no LDS accumulators.
-      // SC23AD_TRI_RP=0 keeps the entry-parallel kernel, SC23AD_TRI_RP=1
-      // uses one lane per row only; SC23AD_RP_ROWS=2 puts two rows on each
-      // lane of the 4-entry layout (default one: at 128^3 level 0 took 157 us
-      // with 8 waves of one row per lane, 174 us with 4 waves of two).
-      int md = 0;
-      for (int idx = 0; idx < n; ++idx) md = std::max(md, lbeg[idx + 1] - lbeg[idx]);
-      const char* env_rp = std::getenv("SC23AD_TRI_RP");
-      int e = 0, lanes = 1, rows = 1;
-      const bool force_groups = env_rp && env_rp[0] == '2';  // tuning: lanes per row even for short rows
-      if (md <= dev::kRpMaxEntries && !(force_groups && !any_far && md > 4)) {
-        e = md <= 4 ? 4 : md <= 8 ? 8 : md <= 10 ? 10 : 12;
-        if (const char* r = std::getenv("SC23AD_RP_ROWS"); r && e == 4 && r[0] == '2') rows = 2;
-      } else if (!any_far && !(env_rp && env_rp[0] == '1')) {
-        // the fewest waves, then the fewest entries per row
-        size_t best = 0;
-        for (int g = 2; g <= dev::kRpMaxLanes; g *= 2)
-          for (int ge : {8, 10, 12}) {
-            if (g * ge < md) continue;
-            const size_t w = (maxlev_rows * g + 63) / 64;
-            const size_t key = w * 4096 + static_cast<size_t>(g * ge);
-            if (w <= 8 && (best == 0 || key < best)) {
-              best = key;
-              lanes = g;
-              e = ge;
-            }
-          }
-      }
-      if (kind != TriKind::kLD || (env_rp && env_rp[0] == '0') ||
-          dev::rp_lds_bytes(ep_ring, maxlev_chain) > dev::kTriBlockedMaxLds)
-        e = 0;
-      const size_t lanes_needed = (maxlev_rows + rows - 1) / rows * lanes;
-      // the fewest waves, 1 to 8 (SC23AD_RP_POW2=1: powers of two; at 128^3
-      // three waves instead of four took levels 1 and 3 from 94 and 109 us
-      // to 87 and 95 us per solve)
-      const bool pow2 = std::getenv("SC23AD_RP_POW2") != nullptr;
-      int rw = 1;
-      while (rw < 8 && static_cast<size_t>(rw) * 64 < lanes_needed) rw = pow2 ? rw * 2 : rw + 1;
-      if (e > 0 && static_cast<size_t>(rw) * 64 >= lanes_needed) {
-        std::vector<int> rent(static_cast<size_t>(std::max(n, 1)) * lanes * e * 2, 0);
-        int farq = 0;
-        for (int idx = 0; idx < n; ++idx) {
-          // far entries first (a row's integer sum is order-free), so the
-          // kernel loads far values for the first farq slots only
-          std::vector<int> ord;
-          for (int q = lbeg[idx]; q < lbeg[idx + 1]; ++q)
-            if (lent[4 * static_cast<size_t>(q)] < 0) ord.push_back(q);
-          farq = std::max(farq, static_cast<int>(ord.size()));
-          for (int q = lbeg[idx]; q < lbeg[idx + 1]; ++q)
-            if (lent[4 * static_cast<size_t>(q)] >= 0) ord.push_back(q);
-          for (int m = 0; m < static_cast<int>(ord.size()); ++m) {
-            const int q = ord[m];
-            const size_t at =
-                ((static_cast<size_t>(idx) * lanes + m % lanes) * e + m / lanes) * 2;
-            rent[at] = lent[4 * static_cast<size_t>(q)];
-            rent[at + 1] = lent[4 * static_cast<size_t>(q) + 1];
-          }
-        }
-        plan.rent.alloc(sizeof(int) * rent.size());
-        plan.rent.upload(rent.data(), sizeof(int) * rent.size());
-        L.rent = plan.rent.get();
-        L.rp_e = e;
-        L.rp_rows = rows;
-        L.rp_lanes = lanes;
-        L.rp_waves = rw;
-        L.rp_farq = farq;
-      }
       // The block kernel's layout (four right-hand sides per workgroup,
       // block.hip), chosen on its own: its ring keeps four values per slot,
       // so it is at most kTriBlockedMaxLds / 16 slots, and it reads
@@ -776,6 +863,14 @@ void build_plan(TriPlan& plan, TriKind kind, int n, const std::vector<int>& rptr
           L.ep_maxlev = maxlev_chain;
         }
       }
+    }
+  }
+  // Row-parallel mode (integer smoother factors): lanes per row, entries per
+  // lane and waves chosen by plan_rp; SC23AD_TRI_RP=0 keeps the other kernels.
+  if constexpr (std::is_same_v<V, int32_t>) {
+    if (kind == TriKind::kLD && plan.identity) {
+      std::vector<int> chains = chain_lev;
+      plan_rp(plan, n, lbeg, lpos, lval, lev_ptr, chains, span, single_wg_max);
     }
   }
   // FP smoother factors (solvers 0 and 1): the row-parallel kernel with one
@@ -949,11 +1044,13 @@ void build_plan(TriPlan& plan, TriKind kind, int n, const std::vector<int>& rptr
                  "[sc23ad plan] kind %d n %d nnz %zu chains %d levels(max chain) %d "
                  "max level rows %zu launches %d ring %d span %lld max deps %d ep waves %d far %d "
                  "narrow %d copies %d rp waves %d entries %d rows %d lanes %d identity %d "
-                 "| block: waves %d entries %d rows %d lanes %d ring %d far %d\n",
+                 "| block: waves %d entries %d rows %d lanes %d ring %d far %d "
+                 "| rp: pieces %d far %d fence %d\n",
                  static_cast<int>(kind), n, cind.size(), nchain, plan.nlevels, maxlev_rows,
                  plan.nlaunch, L.ring, span, maxdeps, L.ep_waves, L.ep_far, L.ep_narrow,
                  L.ep_copies, L.rp_waves, L.rp_e, L.rp_rows, L.rp_lanes, plan.identity ? 1 : 0,
-                 L.waves_blk, L.e_blk, L.rows_blk, L.lanes_blk, L.ring_blk, L.farq_blk);
+                 L.waves_blk, L.e_blk, L.rows_blk, L.lanes_blk, L.ring_blk, L.farq_blk, L.rp_maxlev,
+                 L.rp_farq, L.rp_fence);
   }
 }
 
@@ -1417,8 +1514,8 @@ void DevAmg::spmv(const DevMat& m, SpmvMode mode, const void* x, const void* z,
 // Whether trsv() solves the factor with one launch that binds armed
 // dispatch events (the row- and entry-parallel integer kernels).
 bool DevAmg::trsv_timing_aware(const TriPlan& plan) const {
-  return elem == Elem::kI32 && !plan.dense && !plan.blocked && plan.segs.size() == 1 &&
-         (plan.layout.rp_waves > 0 || plan.layout.ep_waves > 0);
+  return elem == Elem::kI32 && !plan.dense && !plan.blocked &&
+         (plan.layout.rp_waves > 0 || (plan.segs.size() == 1 && plan.layout.ep_waves > 0));
 }
 
 void DevAmg::trsv(const TriPlan& plan, const DevMat& m, const void* in, void* out,
@@ -1447,9 +1544,8 @@ void DevAmg::trsv(const TriPlan& plan, const DevMat& m, const void* in, void* ou
               "trsv blocked");
     return;
   }
-  if (plan.layout.rp_waves > 0 && elem == Elem::kI32 && plan.segs.size() == 1) {
-    hip_check(dev::launch_trsv_rp(plan.layout, plan.segs[0], m.d.bit, m.d.dbit, in, out,
-                                  lib_stream()),
+  if (plan.layout.rp_waves > 0 && elem == Elem::kI32) {
+    hip_check(dev::launch_trsv_rp(plan.layout, m.d.bit, m.d.dbit, in, out, lib_stream()),
               "trsv rp");
     return;
   }

@@ -107,10 +107,17 @@ struct TriLayout {
   int ep_copies = 1; // accumulator copies per row (1 or kEpCopies)
   int ep_acc = 0;    // accumulator slots in LDS
   // row-parallel mode (LD factors with short rows): rp_lanes lanes per row,
-  // each holding rp_e entries (int2 {dep, val}, padded) of its row, rp_rows
-  // rows per lane (one lane per row only), rp_waves waves per chain; same
-  // chains, ring and far rule as the entry-parallel mode
+  // each holding rp_e entries (int2 {code, -val}, padded, see k_tri_chain_rp)
+  // of its row, rp_rows rows per lane (FP, one lane per row only), rp_waves
+  // waves per chain; its own levels (pieces of the level schedule's), chains
+  // and ring, and the far rule of the entry-parallel mode
   const void* rent = nullptr;
+  const int* rp_lev = nullptr;
+  const int* rp_chain = nullptr;
+  int rp_nchain = 0;
+  int rp_maxlev = 0;  // most pieces in one chain
+  int rp_ring = 0;
+  int rp_fence = 1;   // levels between full fences (power of two; far entries only)
   int rp_waves = 0;  // > 0: use the row-parallel kernel
   int rp_e = 0;
   int rp_rows = 0;
@@ -146,16 +153,18 @@ constexpr int kEpMaxRows = 1024;  // most rows in one level of one chain
 constexpr int kEpCopies = 8;
 hipError_t launch_trsv_ep(TriKind kind, const TriLayout& L, const TriSegment& seg, int bit,
                           int dbit, const void* in, void* out, hipStream_t s);
-// Row-parallel integer LD solve (one workgroup per chain, 1-16 lanes per row).
-constexpr int kRpMaxEntries = 12;  // one lane per row
-constexpr int kRpMaxLanes = 16;    // several lanes per row: 8 or 12 entries each
-hipError_t launch_trsv_rp(const TriLayout& L, const TriSegment& seg, int bit, int dbit,
-                          const void* in, void* out, hipStream_t s);
+// Row-parallel integer LD solve (one workgroup per chain, 1-64 lanes per row).
+constexpr int kRpMaxLanes = 64;   // lanes per row, 4 to 12 entries each
+constexpr int kRpMaxWaves = 16;   // more than 8: one lane of 4 entries per row
+constexpr int kRpMaxAhead = 4;    // far values are loaded at most this many levels ahead
+constexpr int kRpPadLevels = 12;  // level offsets past a chain's last one
+hipError_t launch_trsv_rp(const TriLayout& L, int bit, int dbit, const void* in, void* out,
+                          hipStream_t s);
 hipError_t launch_trsv_rpf(Elem e, const TriLayout& L, const TriSegment& seg, const void* in,
                            void* out, hipStream_t s);
 inline size_t rp_lds_bytes(int ring, int maxlev) {
   return sizeof(int32_t) * static_cast<size_t>(ring) +
-         sizeof(int) * (static_cast<size_t>(maxlev) + 1);
+         sizeof(int) * (static_cast<size_t>(maxlev) + 1 + kRpPadLevels);
 }
 // ---- block kernels (block.hip): several right-hand sides of one hierarchy --
 // A block vector of n rows and `groups` groups of four right-hand sides holds

@@ -1289,255 +1289,355 @@ hipError_t tri_ep_launch(const TriLayout& L, const TriSegment& seg, int bit, int
 // ---------------------------------------------------------------------------
 // Row-parallel integer LD solve: the chains, levels, LDS ring and far
 // dependencies of k_tri_chain_ep, for factors whose rows hold at most kG * kE
-// dependency entries.  kG lanes serve one row (kG = 1: each lane serves kR
-// rows t, t + kThreads, ...); each lane keeps kE entries of its row, padded
-// with zero values, in registers.  A level costs one round of ring reads, the
-// products in registers, a sum over the row's kG lanes (DPP moves),
-// the ring writes and one barrier: no accumulators, no atomics.  The integer
-// sum is order-free (wrap-around), so the result equals the sequential one
-// bit for bit.  Entries are stored by position as kG * kE int2 {dep, val}
-// pairs, lane j's kE contiguous (a row's entry m goes to lane m % kG); dep is
-// encoded as in k_tri_chain_ep and padding is {0, 0}.
-template <int kE, int kR>
+// dependency entries.  kG lanes serve one row; each lane keeps kE entries of
+// its row, padded with zero values, in registers.  The integer sum is
+// order-free (wrap-around), so the result equals the sequential one bit for
+// bit.
+//
+// What bounds it: a chain is one workgroup of 1-8 waves that walks its levels
+// one after another, so a level costs the instructions its waves issue (one
+// per four cycles and wave) plus one LDS round trip, whatever the bandwidth.
+// Everything that does not depend on the previous level is therefore computed
+// once on the host or kept off the vector unit:
+//  * an entry {code, val} holds the byte offset of its ring slot (no masking,
+//    no address arithmetic) and the negated value, so a row's sum starts from
+//    in * 2^bit and only adds products; a far entry (the first kFq slots of a
+//    row at most) holds ~(4 * position) instead;
+//  * entries, inverse diagonals, right-hand sides and results are buffers
+//    addressed by a scalar offset per level plus a lane offset that never
+//    changes; lanes past a level's end load what follows (past the buffer's
+//    end: 0) and never store;
+//  * the loads of level L + kD - 1 are issued into the buffer that level L - 1
+//    has freed, between this level's ring reads and their first use;
+//  * shifts by bit and dbit (0..30) are single 32-bit funnel shifts, and the
+//    finish takes one 32 x 32 product and one low product.
+// Measured per solve against the form that masked ring positions and computed
+// addresses per level (128^3 BlockSOR, levels 1-4: 83 / 78 / 92 / 43 us, now
+// 80 / 64 / 62 / 29 us; level 0: 87 -> 82 us) and against the entry-parallel
+// kernel and one launch per wide level (63^3 SOR, whole V-cycle: 5.27 -> 2.61 ms).
+using RpWord4 = __attribute__((ext_vector_type(4))) unsigned;
+template <int kE, int kFq>
 struct RpPre {
-  int lo, hi;             // the level's position bounds
-  int4 ent[kR][kE / 2];   // {dep, val, dep, val}
-  int32_t xfar[kR][kE];
-  int32_t dinv[kR];
-  int32_t in[kR];
+  int lo, cnt;            // first position and rows of the level (scalars)
+  RpWord4 ent[kE / 2];    // {code, -val, code, -val}
+  int32_t xfar[kFq > 0 ? kFq : 1];
+  int32_t dinv, in;
 };
 
-template <int kThreads, int kG, int kE, int kR>
-__device__ __forceinline__ void rp_load(RpPre<kE, kR>& r, int lo, int hi,
-                                        const int4* __restrict__ rent,
-                                        const int32_t* __restrict__ dinv,
-                                        const int32_t* __restrict__ in) {
-  const int t = threadIdx.x;
+struct RpArgs {
+  __amdgpu_buffer_rsrc_t rent, dinv, in, out;
+  unsigned ring_mask;     // ring size in bytes - 1
+  int bit, dbit;
+  int fence_mask;
+};
+
+// Constants of a lane.
+struct RpLane {
+  int ent_off;            // its entries' byte offset from the level's first row's
+  int row4;               // 4 * its row in the level
+  int owner;              // its row for the row's first lane, else INT32_MAX
+  int32_t scale;          // 2^bit for the row's first lane, else 0
+};
+
+// A buffer of `bytes` bytes; loads past its end return 0.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t rp_buffer(const void* p, unsigned bytes) {
+  constexpr int kRaw32 = 0x00020000;  // untyped, 32-bit elements
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, static_cast<int>(bytes),
+                                           kRaw32);
+}
+
+// LDS word at a byte offset: the ring begins the kernel's only LDS array, at
+// address 0.
+using LdsWord = __attribute__((address_space(3))) int32_t;
+__device__ __forceinline__ LdsWord* rp_lds(unsigned off) {
+  return reinterpret_cast<LdsWord*>(off);
+}
+
+template <int kG, int kE, int kFq>
+__device__ __forceinline__ void rp_load(RpPre<kE, kFq>& r, int lo, int hi, const RpArgs& a,
+                                        const RpLane& ln) {
   r.lo = lo;
-  r.hi = hi;
+  r.cnt = hi - lo;
+  const int lo4 = 4 * lo, loe = static_cast<int>(static_cast<unsigned>(lo) * (kG * kE * 8));
 #pragma unroll
-  for (int q = 0; q < kR; ++q) {
-    const int idx = lo + t / kG + q * (kThreads / kG);
-    const int id = idx < hi ? idx : 0;  // lanes past the level's end load position 0
-    const size_t base = (static_cast<size_t>(id) * kG + t % kG) * (kE / 2);
-#pragma unroll
-    for (int h = 0; h < kE / 2; ++h) r.ent[q][h] = rent[base + h];
-    r.dinv[q] = dinv[id];
-    r.in[q] = in[id];
-  }
+  for (int h = 0; h < kE / 2; ++h)
+    r.ent[h] = __builtin_amdgcn_raw_buffer_load_b128(a.rent, ln.ent_off + 16 * h, loe, 0);
+  r.dinv = static_cast<int>(__builtin_amdgcn_raw_buffer_load_b32(a.dinv, ln.row4, lo4, 0));
+  r.in = static_cast<int>(__builtin_amdgcn_raw_buffer_load_b32(a.in, ln.row4, lo4, 0));
 }
 
-// Far values of the first kFq entries of each row (the plan puts a row's far
-// entries first; kFq bounds their number).
-template <int kThreads, int kG, int kE, int kR, int kFq = kE>
-__device__ __forceinline__ void rp_far(RpPre<kE, kR>& r, const int32_t* out) {
-  const int t = threadIdx.x;
-#pragma unroll
-  for (int q = 0; q < kR; ++q) {
-    const bool ok = r.lo + t / kG + q * (kThreads / kG) < r.hi;
-#pragma unroll
-    for (int h = 0; h < kE / 2; ++h) {
-      const int d0 = r.ent[q][h].x, d1 = r.ent[q][h].z;
-      if (2 * h < kFq) r.xfar[q][2 * h] = out[(ok && d0 < 0) ? -d0 - 1 : 0];
-      if (2 * h + 1 < kFq) r.xfar[q][2 * h + 1] = out[(ok && d1 < 0) ? -d1 - 1 : 0];
-    }
+// acc + dpp(acc) on 64-bit values, one stage of a group sum: the low words'
+// sum sets the carry that the high words' takes.  A DPP operand written by
+// the two instructions before it needs two wait states.
+#define SC23AD_DPP_ADD64(NAME, CTRL)                                                    \
+  __device__ __forceinline__ uint64_t NAME(uint64_t v) {                                \
+    unsigned lo, hi;                                                                    \
+    asm("s_nop 1\n\t"                                                                   \
+        "v_add_co_u32_dpp %0, vcc, %2, %2 " CTRL " row_mask:0xf bank_mask:0xf\n\t"      \
+        "v_addc_co_u32_dpp %1, vcc, %3, %3, vcc " CTRL " row_mask:0xf bank_mask:0xf"    \
+        : "=&v"(lo), "=&v"(hi)                                                          \
+        : "v"(static_cast<unsigned>(v)), "v"(static_cast<unsigned>(v >> 32))            \
+        : "vcc");                                                                       \
+    return (static_cast<uint64_t>(hi) << 32) | lo;                                      \
   }
+SC23AD_DPP_ADD64(dpp_add_swap1, "quad_perm:[1,0,3,2]")
+SC23AD_DPP_ADD64(dpp_add_swap2, "quad_perm:[2,3,0,1]")
+SC23AD_DPP_ADD64(dpp_add_half_mirror, "row_half_mirror")
+SC23AD_DPP_ADD64(dpp_add_mirror, "row_mirror")
+#undef SC23AD_DPP_ADD64
+
+// Sum over aligned groups of kG lanes, every lane ending with its group's;
+// all lanes must be active.  Groups of 32 and 64 exchange rows of 16 and
+// halves of the wave with gfx950's permlane swaps: two equal inputs come back
+// as the two parts side by side.
+__device__ __forceinline__ uint64_t permlane_add(uint64_t v, bool halves) {
+  const unsigned lo = static_cast<unsigned>(v), hi = static_cast<unsigned>(v >> 32);
+  auto l = halves ? __builtin_amdgcn_permlane32_swap(lo, lo, false, false)
+                  : __builtin_amdgcn_permlane16_swap(lo, lo, false, false);
+  auto h = halves ? __builtin_amdgcn_permlane32_swap(hi, hi, false, false)
+                  : __builtin_amdgcn_permlane16_swap(hi, hi, false, false);
+  return ((static_cast<uint64_t>(h[0]) << 32) | l[0]) +
+         ((static_cast<uint64_t>(h[1]) << 32) | l[1]);
+}
+template <int kG>
+__device__ __forceinline__ uint64_t group_sum_dpp(uint64_t v) {
+  static_assert(kG >= 1 && kG <= 64 && (kG & (kG - 1)) == 0, "groups of 1-64 lanes");
+  if (kG >= 2) v = dpp_add_swap1(v);
+  if (kG >= 4) v = dpp_add_swap2(v);
+  if (kG >= 8) v = dpp_add_half_mirror(v);
+  if (kG >= 16) v = dpp_add_mirror(v);
+  if (kG >= 32) v = permlane_add(v, false);
+  if (kG >= 64) v = permlane_add(v, true);
+  return v;
 }
 
+// low32(mul_wrap(t >> bit, dinv) >> dbit) for shifts 0..31.  With q = t >> bit
+// as words qhi:qlo and dinv read as unsigned u = dinv + 2^32 [dinv < 0], the
+// low 64 bits of q dinv are qlo u plus, in the high word, qhi u - qlo
+// [dinv < 0]; the two products and the correction do not wait for each other.
+__device__ __forceinline__ int32_t rp_finish(uint64_t t, int32_t dinv, int bit, int dbit) {
+  const unsigned lo = static_cast<unsigned>(t), hi = static_cast<unsigned>(t >> 32);
+  const unsigned neg = static_cast<unsigned>(dinv >> 31);
+  const unsigned qlo = __builtin_amdgcn_alignbit(hi, lo, static_cast<unsigned>(bit));
+  const unsigned qhi = static_cast<unsigned>(static_cast<int>(hi) >> bit);
+  unsigned m;  // opaque: folded into the other product it would wait for it
+  asm("v_mul_lo_u32 %0, %1, %2" : "=v"(m) : "v"(qhi), "v"(dinv));
+  const uint64_t p = static_cast<uint64_t>(qlo) * static_cast<unsigned>(dinv);
+  const unsigned ph = static_cast<unsigned>(p >> 32) + m + ((0u - qlo) & neg);
+  return static_cast<int32_t>(
+      __builtin_amdgcn_alignbit(ph, static_cast<unsigned>(p), static_cast<unsigned>(dbit)));
+}
 
-template <TriKind K, int kWaves, bool kFar, int kG, int kE, int kR, int kD, int kA, int kFq>
-__device__ __forceinline__ void rp_level(RpPre<kE, kR>& cur, RpPre<kE, kR>& ahead, int L, int nl,
-                                         const int* lvo, int32_t* ring, int rmask,
-                                         const int4* __restrict__ rent,
-                                         const int32_t* __restrict__ dinv,
-                                         const int32_t* __restrict__ in, int32_t* out, int bit,
-                                         int dbit) {
-  constexpr int kThreads = 64 * kWaves;
-  const int t = threadIdx.x;
-  const int s = cur.lo, e = cur.hi;
-  // bounds of the level prefetched at the end of this one
-  const int Lp = min(L + kD, nl);
-  const int plo = lvo[Lp], phi = lvo[min(Lp + 1, nl)];
-  if (kFar) rp_far<kThreads, kG, kE, kR, kFq>(ahead, out);
-  int32_t xv[kR][kE];
+// Level L (buffer cur).  nxt: the buffer level L - 1 has freed, filled for
+// level L + kD - 1, whose bounds `pend` holds; `ahead`: level L + kA's buffer.
+template <bool kTail, int kMaxWaves, bool kFar, int kG, int kE, int kD, int kA, int kFq>
+__device__ __forceinline__ void rp_level(RpPre<kE, kFq>& cur, RpPre<kE, kFq>& nxt,
+                                         RpPre<kE, kFq>& ahead, int L, int2& pend,
+                                         const int* lvo, const RpArgs& a,
+                                         const RpLane& ln) {
+  int32_t xv[kE];
 #pragma unroll
-  for (int q = 0; q < kR; ++q)
-#pragma unroll
-    for (int h = 0; h < kE / 2; ++h) {
-      xv[q][2 * h] = ring[cur.ent[q][h].x & rmask];
-      xv[q][2 * h + 1] = ring[cur.ent[q][h].z & rmask];
-    }
-  // rows of 8-12 entries: every ring read is issued before the first
-  // product, so the level pays one LDS round trip (left to itself the
-  // scheduler splits them in two: 4-5 % slower; with 4 entries the barrier
-  // measured 2 % slower)
-  if constexpr (kE >= 8) __builtin_amdgcn_sched_barrier(0);
+  for (int q = 0; q < kE; ++q) {
+    int c = static_cast<int>(q % 2 ? cur.ent[q / 2].z : cur.ent[q / 2].x);
+    if (kFar && q < kFq) c = max(c, 0);
+    xv[q] = *rp_lds(static_cast<unsigned>(c));
+  }
+  int plo = 0, phi = 0;
+  if (!kTail) {
+    plo = __builtin_amdgcn_readfirstlane(pend.x);
+    phi = __builtin_amdgcn_readfirstlane(pend.y);
+  }
+  // every ring read is issued before the loads and the first product, so the
+  // level pays one LDS round trip, covered in part by issuing the loads
+  __builtin_amdgcn_sched_barrier(0);
+  if (!kTail) rp_load<kG, kE, kFq>(nxt, plo, phi, a, ln);
   if (kFar) {
 #pragma unroll
-    for (int q = 0; q < kR; ++q)
-#pragma unroll
-      for (int h = 0; h < kE / 2; ++h) {
-        const int d0 = cur.ent[q][h].x, d1 = cur.ent[q][h].z;
-        if (2 * h < kFq && __any(d0 < 0))
-          xv[q][2 * h] = d0 < 0 ? cur.xfar[q][2 * h] : xv[q][2 * h];
-        if (2 * h + 1 < kFq && __any(d1 < 0))
-          xv[q][2 * h + 1] = d1 < 0 ? cur.xfar[q][2 * h + 1] : xv[q][2 * h + 1];
-      }
-  }
-#pragma unroll
-  for (int q = 0; q < kR; ++q) {
-    uint64_t acc = 0, acc2 = 0;  // two chains of multiply-adds
-#pragma unroll
-    for (int h = 0; h < kE / 2; ++h) {
-      acc += prod64(cur.ent[q][h].y, xv[q][2 * h]);
-      acc2 += prod64(cur.ent[q][h].w, xv[q][2 * h + 1]);
-    }
-    // opaque ends keep the two chains apart (the compiler would otherwise
-    // fold them into one chain of dependent multiply-adds)
-    asm volatile("" : "+v"(acc));
-    asm volatile("" : "+v"(acc2));
-    acc = group_sum<kG>(acc + acc2);
-    const int k = s + t / kG + q * (kThreads / kG);
-    if (k < e && t % kG == 0) {
-      const uint64_t tt = (static_cast<uint64_t>(static_cast<int64_t>(cur.in[q])) << bit) - acc;
-      const int32_t v = acc_final<int32_t, K>(tt, cur.dinv[q], bit, dbit);
-      ring[k & rmask] = v;
-      out[k] = v;
+    for (int q = 0; q < kFq; ++q) {
+      // ~code is 4 * position for a far entry, else past the buffer's end
+      const unsigned c = q % 2 ? ahead.ent[q / 2].z : ahead.ent[q / 2].x;
+      ahead.xfar[q] = static_cast<int>(
+          __builtin_amdgcn_raw_buffer_load_b32(a.out, static_cast<int>(~c), 0, 0));
     }
   }
-  if (kFar && (L % kEpFence) == kEpFence - 1)
-    __syncthreads();  // full fence: global results visible to later loads
+  if (!kTail) {
+    pend.x = lvo[L + kD];
+    pend.y = lvo[L + kD + 1];
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  if (kFar) {
+    // waits for a far value only where a lane of the wave has one
+#pragma unroll
+    for (int q = 0; q < kFq; ++q) {
+      const int c = static_cast<int>(q % 2 ? cur.ent[q / 2].z : cur.ent[q / 2].x);
+      if (__any(c < 0)) xv[q] = c < 0 ? cur.xfar[q] : xv[q];
+    }
+  }
+  uint64_t acc = prod64(cur.in, ln.scale), acc2 = 0;  // two chains of multiply-adds
+#pragma unroll
+  for (int h = 0; h < kE / 2; ++h) {
+    acc += prod64(static_cast<int>(cur.ent[h].y), xv[2 * h]);
+    acc2 += prod64(static_cast<int>(cur.ent[h].w), xv[2 * h + 1]);
+  }
+  // opaque ends keep the two chains apart (the compiler would otherwise
+  // fold them into one chain of dependent multiply-adds)
+  asm volatile("" : "+v"(acc));
+  asm volatile("" : "+v"(acc2));
+  acc = group_sum_dpp<kG>(acc + acc2);
+  const int32_t v = rp_finish(acc, cur.dinv, a.bit, a.dbit);
+  if (ln.owner < cur.cnt) {
+    const int lo4 = 4 * cur.lo;
+    *rp_lds(static_cast<unsigned>(lo4 + ln.row4) & a.ring_mask) = v;
+    __builtin_amdgcn_raw_buffer_store_b32(static_cast<unsigned>(v), a.out, ln.row4, lo4, 0);
+  }
+  // a full fence every fence_mask + 1 levels makes far values visible before
+  // any load of them; it also drains the loads in flight, so the plan makes
+  // the period as long as the nearest far dependency allows
+  if (kFar && (L & a.fence_mask) == a.fence_mask)
+    __syncthreads();
   else
-    ep_sync<kWaves>();
-  rp_load<kThreads, kG>(cur, plo, phi, rent, dinv, in);
+    ep_sync<kMaxWaves>();
 }
 
-// LDS: the ring, then the chain's level offsets (max_levels + 1 ints).
-// Far values of level L + kA are loaded at the start of level L, from entries
-// loaded kD - kA levels before that.
-template <TriKind K, int kWaves, bool kFar, int kG, int kE, int kR, int kD, int kA, int kFq = kE>
-__global__ __launch_bounds__(64 * kWaves) void k_tri_chain_rp(
-    const int4* __restrict__ rent, const int32_t* __restrict__ dinv,
-    const int* __restrict__ lev_ptr, const int* __restrict__ chain_lev, int rmask, int bit,
-    int dbit, const int32_t* __restrict__ in, int32_t* out) {
-  constexpr int kThreads = 64 * kWaves;
-  static_assert(kG == 1 || kR == 1, "several lanes per row serve one row each");
-  static_assert(kA >= 1 && kA < kD, "far values need their entries loaded first");
-  static_assert(kEpFarLevels >= kA + kEpFence,
-                "far dependencies must be fenced before their values are loaded");
+// The last nl - L0 < kD levels, nested so that no paths join between them.
+template <int kFirst, int kMaxWaves, bool kFar, int kG, int kE, int kD, int kA, int kFq>
+__device__ __forceinline__ void rp_tail(RpPre<kE, kFq> (&buf)[kD], int L0, int nl, int2& pend,
+                                        const int* lvo, const RpArgs& a, const RpLane& ln) {
+  if constexpr (kFirst < kD - 1) {
+    if (L0 + kFirst < nl) {
+      rp_level<true, kMaxWaves, kFar, kG, kE, kD, kA, kFq>(
+          buf[kFirst], buf[(kFirst + kD - 1) % kD], buf[(kFirst + kA) % kD], L0 + kFirst, pend,
+          lvo, a, ln);
+      rp_tail<kFirst + 1, kMaxWaves, kFar, kG, kE, kD, kA, kFq>(buf, L0, nl, pend, lvo, a, ln);
+    }
+  }
+}
+
+// LDS: the ring, then the chain's level offsets (max_levels + 1 ints and
+// kRpPadLevels more that repeat the last one).  Far values of level L + kA
+// are loaded in level L, from entries loaded kD - 1 - kA levels before that.
+template <int kMaxWaves, bool kFar, int kG, int kE, int kD, int kA, int kFq>
+__global__ __launch_bounds__(64 * kMaxWaves) void k_tri_chain_rp(
+    const void* __restrict__ rent, const int32_t* __restrict__ dinv,
+    const int* __restrict__ lev_ptr, const int* __restrict__ chain_lev, int n, int ring4, int bit,
+    int dbit, int fence, const int32_t* __restrict__ in, int32_t* out) {
+  static_assert(!kFar || (kA >= 1 && kA < kD - 1), "far values need their entries loaded first");
+  static_assert(kA <= kRpMaxAhead, "the plan's fence period allows for kRpMaxAhead");
+  static_assert(kD + 1 <= kRpPadLevels, "level offsets are read kD + 1 past the end");
   extern __shared__ __align__(16) unsigned char smem_r[];
-  int32_t* ring = reinterpret_cast<int32_t*>(smem_r);
-  int* lvo = ring + rmask + 1;
+  int* lvo = reinterpret_cast<int*>(smem_r + ring4);
   const int t = threadIdx.x;
+  const int threads = kMaxWaves == 1 ? 64 : static_cast<int>(blockDim.x);
   const int lb = chain_lev[2 * blockIdx.x], le = chain_lev[2 * blockIdx.x + 1];
   const int nl = le - lb;
-  for (int k = t; k <= nl; k += kThreads) lvo[k] = lev_ptr[lb + k];
+  for (int k = t; k <= nl + kD + 1; k += threads) lvo[k] = lev_ptr[lb + min(k, nl)];
   __syncthreads();
-  RpPre<kE, kR> buf[kD];
+  const unsigned n4 = 4u * static_cast<unsigned>(n);
+  const RpArgs a{rp_buffer(rent, n4 * (kG * kE * 2)), rp_buffer(dinv, n4), rp_buffer(in, n4),
+                 rp_buffer(out, n4), static_cast<unsigned>(ring4) - 1u, bit, dbit, fence - 1};
+  RpLane ln;
+  ln.ent_off = t * (kE * 8);
+  ln.row4 = 4 * (t / kG);
+  ln.owner = t % kG == 0 ? t / kG : INT32_MAX;
+  ln.scale = t % kG == 0 ? 1 << bit : 0;
+  RpPre<kE, kFq> buf[kD];
 #pragma unroll
-  for (int d = 0; d < kD; ++d) {
-    const int Lc = min(d, nl);
-    rp_load<kThreads, kG>(buf[d], lvo[Lc], lvo[min(Lc + 1, nl)], rent, dinv, in);
-  }
-  // Whole rounds of kD levels, then the tail in a copy of the body.  (One
-  // body for all levels measured slower: with a test around each level the
-  // compiler waits for every outstanding load where the paths join, and
-  // without one the last round runs up to kD - 1 empty levels.)
+  for (int d = 0; d < kD - 1; ++d)
+    rp_load<kG, kE, kFq>(buf[d], __builtin_amdgcn_readfirstlane(lvo[d]),
+                         __builtin_amdgcn_readfirstlane(lvo[d + 1]), a, ln);
+  int2 pend = make_int2(lvo[kD - 1], lvo[kD]);
+  // Whole rounds of kD levels, then the tail, which loads nothing ahead, in a
+  // copy of the body.  (One body for all levels measured slower: with a test
+  // around each level the compiler waits for every outstanding load where the
+  // paths join, and without one the last round runs up to kD - 1 empty levels.)
   int L0 = 0;
   for (; L0 + kD <= nl; L0 += kD) {
 #pragma unroll
     for (int d = 0; d < kD; ++d)
-      rp_level<K, kWaves, kFar, kG, kE, kR, kD, kA, kFq>(buf[d], buf[(d + kA) % kD], L0 + d, nl,
-                                                         lvo, ring, rmask, rent, dinv, in, out,
-                                                         bit, dbit);
+      rp_level<false, kMaxWaves, kFar, kG, kE, kD, kA, kFq>(buf[d], buf[(d + kD - 1) % kD],
+                                                       buf[(d + kA) % kD], L0 + d, pend, lvo, a,
+                                                       ln);
   }
-#pragma unroll
-  for (int d = 0; d < kD; ++d)
-    if (L0 + d < nl)
-      rp_level<K, kWaves, kFar, kG, kE, kR, kD, kA, kFq>(buf[d], buf[(d + kA) % kD], L0 + d, nl,
-                                                         lvo, ring, rmask, rent, dinv, in, out,
-                                                         bit, dbit);
+  rp_tail<0, kMaxWaves, kFar, kG, kE, kD, kA, kFq>(buf, L0, nl, pend, lvo, a, ln);
 }
 
-template <int kWaves, bool kFar, int kG, int kE, int kR, int kD, int kA, int kFq = kE>
-hipError_t tri_rp_go(const TriLayout& L, const TriSegment& seg, int bit, int dbit,
-                     const int32_t* in, int32_t* out, hipStream_t s) {
-  constexpr TriKind K = TriKind::kLD;
-  const size_t lds = rp_lds_bytes(L.ring, L.ep_maxlev);
-  if (lds > static_cast<size_t>(kTriBlockedMaxLds)) return hipErrorInvalidValue;
+template <int kMaxWaves, bool kFar, int kG, int kE, int kD, int kA, int kFq = kFar ? kE : 0>
+hipError_t tri_rp_go(const TriLayout& L, int bit, int dbit, const int32_t* in, int32_t* out, hipStream_t s) {
+  const size_t lds = rp_lds_bytes(L.rp_ring, L.rp_maxlev);
+  if (lds > static_cast<size_t>(kTriBlockedMaxLds) || L.n <= 0 || bit < 0 || bit > 30 ||
+      dbit < 0 || dbit > 30 || L.rp_fence < 1 || static_cast<uint64_t>(L.n) * (kG * kE * 8) > UINT32_MAX)
+    return hipErrorInvalidValue;
   static bool attr = false;
   if (!attr) {
     hipError_t e = hipFuncSetAttribute(
-        reinterpret_cast<const void*>(&k_tri_chain_rp<K, kWaves, kFar, kG, kE, kR, kD, kA, kFq>),
+        reinterpret_cast<const void*>(&k_tri_chain_rp<kMaxWaves, kFar, kG, kE, kD, kA, kFq>),
         hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(kTriBlockedMaxLds));
     if (e != hipSuccess) return e;
     attr = true;
   }
-  launch_timed(&k_tri_chain_rp<K, kWaves, kFar, kG, kE, kR, kD, kA, kFq>, dim3(seg.nchain),
-               dim3(64 * kWaves), static_cast<uint32_t>(lds), s,
-               reinterpret_cast<const int4*>(L.rent), static_cast<const int32_t*>(L.ldiag),
-               L.lev_ptr, seg.chain_lev, L.ring - 1, bit, dbit, in, out);
+  launch_timed(&k_tri_chain_rp<kMaxWaves, kFar, kG, kE, kD, kA, kFq>, dim3(L.rp_nchain),
+               dim3(64 * L.rp_waves), static_cast<uint32_t>(lds), s,
+               L.rent, static_cast<const int32_t*>(L.ldiag), L.rp_lev, L.rp_chain, L.n,
+               4 * L.rp_ring, bit, dbit, L.rp_fence, in, out);
   return hipGetLastError();
 }
 
-// Register layouts.  4 entries and 1 row per lane: prefetch distance 8
-// levels and far values 4 levels ahead (a level takes less than one
-// global-load latency, and a far value waits for two: at 128^3 the finest
-// level's solve took 116 us, against 157 us at distance 4); 2 rows per lane:
-// distance 6, far values 3 ahead (the registers of 8 levels spill).  One lane with 8,
-// 10 or 12 entries, or 2, 4, 8 or 16 lanes of 8, 10 or 12 entries per row (factors
-// without far dependencies): distance 4, far values 2 ahead (distance 8
-// measured no faster there).
-template <int kWaves, bool kFar>
-hipError_t tri_rp_layout(const TriLayout& L, const TriSegment& seg, int bit, int dbit,
-                         const int32_t* in, int32_t* out, hipStream_t s) {
+// Register layouts and prefetch distances: a level takes 0.1-0.3 us and its
+// entries come from HBM, so the loads run several levels ahead, as far as the
+// 256 registers of a lane allow.
+template <int kMaxWaves, bool kFar>
+hipError_t tri_rp_layout(const TriLayout& L, int bit, int dbit, const int32_t* in, int32_t* out, hipStream_t s) {
+  constexpr int kD8 = kFar ? 6 : 8, kD10 = kFar ? 5 : 8, kD12 = kFar ? 5 : 6;
+  constexpr int kA8 = kFar ? 3 : 1, kA10 = kFar ? 2 : 1;
   if (L.rp_lanes <= 1) {
-    if (L.rp_e == 4 && L.rp_rows == 1) {
+    if (L.rp_e == 4) {
       if (kFar && L.rp_farq == 1)  // one far entry at most, stored first
-        return tri_rp_go<kWaves, kFar, 1, 4, 1, 8, 4, 1>(L, seg, bit, dbit, in, out, s);
-      return tri_rp_go<kWaves, kFar, 1, 4, 1, 8, 4>(L, seg, bit, dbit, in, out, s);
+        return tri_rp_go<kMaxWaves, kFar, 1, 4, 10, 4, 1>(L, bit, dbit, in, out, s);
+      return tri_rp_go<kMaxWaves, kFar, 1, 4, 10, 4>(L, bit, dbit, in, out, s);
     }
-    if (L.rp_e == 4 && L.rp_rows == 2)
-      return tri_rp_go<kWaves, kFar, 1, 4, 2, 6, 3>(L, seg, bit, dbit, in, out, s);
-    if (L.rp_e == 8 && L.rp_rows == 1)
-      return tri_rp_go<kWaves, kFar, 1, 8, 1, 4, 2>(L, seg, bit, dbit, in, out, s);
-    if (L.rp_e == 10 && L.rp_rows == 1)
-      return tri_rp_go<kWaves, kFar, 1, 10, 1, 4, 2>(L, seg, bit, dbit, in, out, s);
-    if (L.rp_e == 12 && L.rp_rows == 1)
-      return tri_rp_go<kWaves, kFar, 1, 12, 1, 4, 2>(L, seg, bit, dbit, in, out, s);
+    if (L.rp_e == 8) return tri_rp_go<kMaxWaves, kFar, 1, 8, kD8, kA8>(L, bit, dbit, in, out, s);
+    if (L.rp_e == 10)
+      return tri_rp_go<kMaxWaves, kFar, 1, 10, kD10, kA10>(L, bit, dbit, in, out, s);
+    if (L.rp_e == 12)
+      return tri_rp_go<kMaxWaves, kFar, 1, 12, kD12, kA10>(L, bit, dbit, in, out, s);
     return hipErrorInvalidValue;
   }
   if constexpr (!kFar) {
-    if (L.rp_e == 10 && L.rp_rows == 1) {
-      if (L.rp_lanes == 2) return tri_rp_go<kWaves, false, 2, 10, 1, 4, 2>(L, seg, bit, dbit, in, out, s);
-      if (L.rp_lanes == 4) return tri_rp_go<kWaves, false, 4, 10, 1, 4, 2>(L, seg, bit, dbit, in, out, s);
-      if (L.rp_lanes == 8) return tri_rp_go<kWaves, false, 8, 10, 1, 4, 2>(L, seg, bit, dbit, in, out, s);
-      if (L.rp_lanes == 16)
-        return tri_rp_go<kWaves, false, 16, 10, 1, 4, 2>(L, seg, bit, dbit, in, out, s);
-    }
-    if (L.rp_e == 12 && L.rp_rows == 1) {
-      if (L.rp_lanes == 2) return tri_rp_go<kWaves, false, 2, 12, 1, 4, 2>(L, seg, bit, dbit, in, out, s);
-      if (L.rp_lanes == 4) return tri_rp_go<kWaves, false, 4, 12, 1, 4, 2>(L, seg, bit, dbit, in, out, s);
-      if (L.rp_lanes == 8) return tri_rp_go<kWaves, false, 8, 12, 1, 4, 2>(L, seg, bit, dbit, in, out, s);
-      if (L.rp_lanes == 16)
-        return tri_rp_go<kWaves, false, 16, 12, 1, 4, 2>(L, seg, bit, dbit, in, out, s);
-    }
-    if (L.rp_e == 8 && L.rp_rows == 1) {
-      if (L.rp_lanes == 2) return tri_rp_go<kWaves, false, 2, 8, 1, 4, 2>(L, seg, bit, dbit, in, out, s);
-      if (L.rp_lanes == 4) return tri_rp_go<kWaves, false, 4, 8, 1, 4, 2>(L, seg, bit, dbit, in, out, s);
-      if (L.rp_lanes == 8) return tri_rp_go<kWaves, false, 8, 8, 1, 4, 2>(L, seg, bit, dbit, in, out, s);
-      if (L.rp_lanes == 16)
-        return tri_rp_go<kWaves, false, 16, 8, 1, 4, 2>(L, seg, bit, dbit, in, out, s);
-    }
+    auto lanes = [&](auto e_tag, auto d_tag) -> hipError_t {
+      constexpr int E = decltype(e_tag)::value, D = decltype(d_tag)::value;
+      switch (L.rp_lanes) {
+        case 2: return tri_rp_go<kMaxWaves, false, 2, E, D, 1>(L, bit, dbit, in, out, s);
+        case 4: return tri_rp_go<kMaxWaves, false, 4, E, D, 1>(L, bit, dbit, in, out, s);
+        case 8: return tri_rp_go<kMaxWaves, false, 8, E, D, 1>(L, bit, dbit, in, out, s);
+        case 16: return tri_rp_go<kMaxWaves, false, 16, E, D, 1>(L, bit, dbit, in, out, s);
+        case 32: return tri_rp_go<kMaxWaves, false, 32, E, D, 1>(L, bit, dbit, in, out, s);
+        case 64: return tri_rp_go<kMaxWaves, false, 64, E, D, 1>(L, bit, dbit, in, out, s);
+        default: return hipErrorInvalidValue;
+      }
+    };
+    using std::integral_constant;
+    if (L.rp_e == 4) return lanes(integral_constant<int, 4>{}, integral_constant<int, 10>{});
+    if (L.rp_e == 6) return lanes(integral_constant<int, 6>{}, integral_constant<int, 8>{});
+    if (L.rp_e == 8) return lanes(integral_constant<int, 8>{}, integral_constant<int, 8>{});
+    if (L.rp_e == 10) return lanes(integral_constant<int, 10>{}, integral_constant<int, 8>{});
+    if (L.rp_e == 12) return lanes(integral_constant<int, 12>{}, integral_constant<int, 6>{});
   }
   return hipErrorInvalidValue;
 }
 
-template <int kWaves>
-hipError_t tri_rp_far(const TriLayout& L, const TriSegment& seg, int bit, int dbit,
-                      const int32_t* in, int32_t* out, hipStream_t s) {
-  if (L.ep_far) return tri_rp_layout<kWaves, true>(L, seg, bit, dbit, in, out, s);
-  return tri_rp_layout<kWaves, false>(L, seg, bit, dbit, in, out, s);
+template <int kMaxWaves>
+hipError_t tri_rp_far(const TriLayout& L, int bit, int dbit, const int32_t* in, int32_t* out, hipStream_t s) {
+  if (L.rp_farq > 0) return tri_rp_layout<kMaxWaves, true>(L, bit, dbit, in, out, s);
+  return tri_rp_layout<kMaxWaves, false>(L, bit, dbit, in, out, s);
+}
+
+// 9-16 waves (128 registers per lane): one lane of 4 entries per row.
+inline hipError_t tri_rp_wide(const TriLayout& L, int bit, int dbit, const int32_t* in,
+                              int32_t* out, hipStream_t s) {
+  if (L.rp_lanes != 1 || L.rp_e != 4) return hipErrorInvalidValue;
+  if (L.rp_farq == 0) return tri_rp_go<16, false, 1, 4, 8, 1>(L, bit, dbit, in, out, s);
+  if (L.rp_farq == 1) return tri_rp_go<16, true, 1, 4, 8, 4, 1>(L, bit, dbit, in, out, s);
+  return tri_rp_go<16, true, 1, 4, 6, 2>(L, bit, dbit, in, out, s);
 }
 
 // Row-parallel FP LD solve (solvers 0 and 1): the chains, levels, LDS ring and
@@ -2255,19 +2355,13 @@ hipError_t launch_trsv_ep(TriKind kind, const TriLayout& L, const TriSegment& se
   return tri_ep_launch<TriKind::kDU, 8>(L, seg, bit, dbit, in, o, s);
 }
 
-hipError_t launch_trsv_rp(const TriLayout& L, const TriSegment& seg, int bit, int dbit,
-                          const void* in_v, void* out_v, hipStream_t s) {
+hipError_t launch_trsv_rp(const TriLayout& L, int bit, int dbit, const void* in_v, void* out_v,
+                          hipStream_t s) {
   const int32_t* in = static_cast<const int32_t*>(in_v);
   int32_t* o = static_cast<int32_t*>(out_v);
-  const int w = L.rp_waves;
-  if (w <= 1) return tri_rp_far<1>(L, seg, bit, dbit, in, o, s);
-  if (w <= 2) return tri_rp_far<2>(L, seg, bit, dbit, in, o, s);
-  if (w <= 3) return tri_rp_far<3>(L, seg, bit, dbit, in, o, s);
-  if (w <= 4) return tri_rp_far<4>(L, seg, bit, dbit, in, o, s);
-  if (w <= 5) return tri_rp_far<5>(L, seg, bit, dbit, in, o, s);
-  if (w <= 6) return tri_rp_far<6>(L, seg, bit, dbit, in, o, s);
-  if (w <= 7) return tri_rp_far<7>(L, seg, bit, dbit, in, o, s);
-  return tri_rp_far<8>(L, seg, bit, dbit, in, o, s);
+  if (L.rp_waves <= 1) return tri_rp_far<1>(L, bit, dbit, in, o, s);
+  if (L.rp_waves <= 8) return tri_rp_far<8>(L, bit, dbit, in, o, s);
+  return tri_rp_wide(L, bit, dbit, in, o, s);
 }
 
 hipError_t launch_trsv_rpf(Elem e, const TriLayout& L, const TriSegment& seg, const void* in,

@@ -1,0 +1,71 @@
+"""The row-parallel integer LD solve (k_tri_chain_rp) in the layouts that the
+plan picks at the ends of its range: one wave and 9-16 waves, 1-64 lanes per
+row, levels cut into pieces, a single chain with levels of more than 1,024
+rows, odd sizes.  Every LD solve equals the oracle's bit for bit (whole
+numbers: no tolerance)."""
+from __future__ import annotations
+
+import os
+import re
+
+import numpy as np
+import pytest
+
+import oracle as O
+import sc23ad as S
+from helpers import export
+
+pytestmark = pytest.mark.gpu
+
+LAYOUT = re.compile(r"\[sc23ad plan\] kind 0 n (\d+) .*rp waves (\d+) entries (\d+) rows \d+ "
+                    r"lanes (\d+) .*rp: pieces (\d+)")
+
+
+
+def _check(a, smoother, monkeypatch, capfd):
+    """LD solves of every level against the oracle; the layouts picked."""
+    monkeypatch.setenv("SC23AD_VERBOSE", "1")
+    a.lmax1_scaling(np.zeros(a.n))
+    h = S.Hierarchy(a, S.INT, S.amg_param(smoother))
+    capfd.readouterr()
+    amg = S.Amg(h)
+    plans = [tuple(map(int, m.groups())) for m in LAYOUT.finditer(capfd.readouterr().err)]
+    print("[ld layouts] (n, waves, entries, lanes, pieces):", plans, flush=True)
+    path = export(h)
+    try:
+        oh = O.OracleHier(path)
+    finally:
+        os.unlink(path)
+    rng = np.random.default_rng(7)
+    for lv in range(amg.depth):
+        n = oh.level_n(lv)
+        x = rng.integers(-2**29, 2**29, n).astype(np.int32)
+        assert np.array_equal(amg.level_op(lv, S.OP_TRSV_LD, x, n),
+                              oh.level_op(lv, S.OP_TRSV_LD, x, n)), lv
+    return plans
+
+
+@pytest.mark.parametrize("kind,params,smoother,waves,lanes", [
+    (S.GEN_POISSON2D, (3,), S.SOR, 1, 1),
+    (S.GEN_LAPLACE3D, (61,), S.SOR, 9, 32),
+    (S.GEN_DIFFUSION27, (33, 5, 1.0, 1.0, 1e-3, 3), S.BLOCK_SOR, 1, 8),
+], ids=["poisson2d_3", "laplace3d_61_sor", "diffusion27_33_block"])
+def test_layouts_of_the_plan(kind, params, smoother, waves, lanes, monkeypatch, capfd):
+    plans = _check(S.CsrMat.generate(kind, *params), smoother, monkeypatch, capfd)
+    assert max(p[1] for p in plans) >= waves and max(p[3] for p in plans) >= lanes
+
+
+@pytest.mark.parametrize("lanes", [1, 2, 4, 8, 16, 32, 64])
+@pytest.mark.parametrize("waves", [1, 3])
+def test_forced_layouts(lanes, waves, monkeypatch, capfd):
+    monkeypatch.setenv("SC23AD_RP_LANES", str(lanes))
+    monkeypatch.setenv("SC23AD_RP_WAVES", str(waves))
+    plans = _check(S.CsrMat.generate(S.GEN_DIFFUSION27, 17, 5, 1.0, 1.0, 1e-3, 3), S.SOR,
+                   monkeypatch, capfd)
+    assert any(p[1] == waves and p[3] == lanes for p in plans) or lanes == 1
+
+
+def test_sixteen_waves(monkeypatch, capfd):
+    monkeypatch.setenv("SC23AD_RP_WAVES", "16")
+    plans = _check(S.CsrMat.generate(S.GEN_POISSON2D, 67), S.SOR, monkeypatch, capfd)
+    assert any(p[1] == 16 for p in plans)
