@@ -54,7 +54,7 @@ std::unique_ptr<DevAmg::BlockWork> DevAmg::make_block_work(int groups) const {
 bool DevAmg::block_native() const {
   for (int l = 0; l < depth; ++l) {
     const TriPlan& p = lv[l].ld_plan;
-    if (!(p.segs.size() == 1 && dev::trsv_rp_blk_supported(p.layout))) return false;
+    if (!dev::trsv_rp_blk_supported(p.layout)) return false;
   }
   return lc_plan.dense && uc_plan.dense;
 }
@@ -77,9 +77,9 @@ void DevAmg::trsv_blk(const TriPlan& plan, const DevMat& m, const void* in, void
               "trsv tiles block");
     return;
   }
-  if (plan.segs.size() == 1 && dev::trsv_rp_blk_supported(plan.layout)) {
-    hip_check(dev::launch_trsv_rp_blk(plan.layout, plan.segs[0], groups, m.d.bit, m.d.dbit, in,
-                                      out, lib_stream()),
+  if (dev::trsv_rp_blk_supported(plan.layout)) {
+    hip_check(dev::launch_trsv_rp_blk(plan.layout, groups, m.d.bit, m.d.dbit, in, out,
+                                      lib_stream()),
               "trsv rp block");
     return;
   }

@@ -389,12 +389,14 @@ void plan_rp(TriPlan& plan, int n, const std::vector<int>& lbeg, const std::vect
   double best = 0;
   int best_g = 0, best_e = 0, best_w = 0;
   long long best_pieces = 0;
-  for (int lg = 0; (1 << lg) <= (one_lane || farq > 0 ? 1 : dev::kRpMaxLanes); ++lg)
+  for (int lg = 0; (1 << lg) <= (one_lane ? 1 : farq > 0 ? 8 : dev::kRpMaxLanes); ++lg)
     for (int e : {4, 6, 8, 10, 12}) {
       const int g = 1 << lg;
       if (g * e < md || (g == 1 && e == 6) ||
           static_cast<uint64_t>(n) * (g * e * 8) > UINT32_MAX)
         continue;
+      // far entries over several lanes: 8 entries or more, kRpFarSlots far ones
+      if (farq > 0 && g > 1 && (e < 8 || farq > dev::kRpFarSlots * g)) continue;
       if (g == 1 && force_groups && farq == 0 && md > 4) continue;
       if (only_lanes > 0 && g != only_lanes) continue;
       for (int w = 1; w <= dev::kRpMaxWaves; w = pow2 ? 2 * w : w + 1) {
@@ -656,6 +658,14 @@ void build_plan(TriPlan& plan, TriKind kind, int n, const std::vector<int>& rptr
         span = std::max<long long>(span, static_cast<long long>(lev_ptr[Lv + 1]) - lpos[q]);
   L.ring = (one_launch_chains && span <= ring) ? ring : 0;
   L.n = n;
+  // Row-parallel mode (integer smoother factors): lanes per row, entries per
+  // lane and waves chosen by plan_rp; SC23AD_TRI_RP=0 keeps the other kernels.
+  if constexpr (std::is_same_v<V, int32_t>) {
+    if (kind == TriKind::kLD && plan.identity) {
+      std::vector<int> chains = chain_lev;
+      plan_rp(plan, n, lbeg, lpos, lval, lev_ptr, chains, span, single_wg_max);
+    }
+  }
   // Entry-parallel mode (integer factors): a dependency is read from the LDS
   // ring when the ring holds it, else from global memory, which needs it at
   // least kEpFarLevels levels back.  The ring is the smallest power of two
@@ -686,7 +696,7 @@ void build_plan(TriPlan& plan, TriKind kind, int n, const std::vector<int>& rptr
                     dev::kTriBlockedMaxLds)
     copies = false;
   const int ep_acc = copies ? acc_rows * dev::kEpCopies : dev::kEpMaxRows;
-  if (std::is_same_v<V, int32_t> && plan.identity && one_launch_chains &&
+  if (std::is_same_v<V, int32_t> && L.rp_waves == 0 && plan.identity && one_launch_chains &&
       maxlev_rows <= static_cast<size_t>(dev::kEpMaxRows) &&
       dev::ep_lds_bytes(ep_ring, maxlev_chain, ep_acc) <= dev::kTriBlockedMaxLds) {
     std::vector<int> lev_of(static_cast<size_t>(std::max(n, 1)), 0);
@@ -745,132 +755,6 @@ void build_plan(TriPlan& plan, TriKind kind, int n, const std::vector<int>& rptr
       // every row of a level and about as many entries.
       L.ep_narrow = (maxlev_rows <= static_cast<size_t>(w) * 64 && overflowing(w, 4) * 16 <= nlev)
                         ? 1 : 0;
-      // The block kernel's layout (four right-hand sides per workgroup,
-      // block.hip), chosen on its own: its ring keeps four values per slot,
-      // so it is at most kTriBlockedMaxLds / 16 slots, and it reads
-      // dependencies at least kRpbFarLevels levels back from global memory;
-      // one or two rows per lane, so that wide levels fit in 8 waves.
-      if (kind == TriKind::kLD) {
-        int md_b = 0;
-        for (int idx = 0; idx < n; ++idx) md_b = std::max(md_b, lbeg[idx + 1] - lbeg[idx]);
-        long long span_near = 0, span_all = 0;
-        for (size_t Lv = 0; Lv + 1 < lev_ptr.size(); ++Lv)
-          for (int idx = lev_ptr[Lv]; idx < lev_ptr[Lv + 1]; ++idx)
-            for (int q = lbeg[idx]; q < lbeg[idx + 1]; ++q) {
-              const long long d = static_cast<long long>(lev_ptr[Lv + 1]) - lpos[q];
-              span_all = std::max(span_all, d);
-              if (lev_of[idx] - lev_of[lpos[q]] < dev::kRpbFarLevels)
-                span_near = std::max(span_near, d);
-            }
-        auto pow2 = [](long long v) {
-          int r = 2;
-          while (r < v) r *= 2;
-          return r;
-        };
-        // far entries per row for a ring of rb slots (one-lane layouts)
-        auto far_count = [&](int rb) {
-          int mx = 0;
-          for (size_t Lv = 0; Lv + 1 < lev_ptr.size(); ++Lv)
-            for (int idx = lev_ptr[Lv]; idx < lev_ptr[Lv + 1]; ++idx) {
-              int c = 0;
-              for (int q = lbeg[idx]; q < lbeg[idx + 1]; ++q)
-                if (static_cast<long long>(lev_ptr[Lv + 1]) - lpos[q] > rb) ++c;
-              mx = std::max(mx, c);
-            }
-          return mx;
-        };
-        int best_e = 0, best_g = 0, best_r = 0, best_w = 0, best_ring = 0, best_fq = 0;
-        size_t best_key = 0;
-        for (int g : {1, 2, 4, 8, 16})
-          for (int ge : {4, 8, 10, 12}) {
-            if ((g > 1 && ge == 4) || g * ge < md_b) continue;
-            // the whole span in the ring when it fits, else the largest ring
-            // that fits (at least the near span), the rest read as far
-            // dependencies
-            int rb = pow2(span_all);
-            if (dev::rpb_lds_bytes(rb, maxlev_chain) > dev::kTriBlockedMaxLds) {
-              rb = pow2(span_near);
-              while (dev::rpb_lds_bytes(2 * rb, maxlev_chain) <= dev::kTriBlockedMaxLds) rb *= 2;
-            }
-            if (dev::rpb_lds_bytes(rb, maxlev_chain) > dev::kTriBlockedMaxLds) continue;
-            int fq = 0;
-            if (span_all > rb) {
-              fq = far_count(rb);
-              // one lane: any number of far slots; g lanes: up to four per
-              // lane (eight with 10 or 12 entries)
-              if (fq > (g == 1 ? ge : (ge >= 10 ? 8 : 4) * g)) continue;
-            }
-            for (int rows_b : {1, 2}) {
-              if (rows_b == 2 && g > 1 && ge > 8) continue;  // no such block kernel
-              // two rows per lane: 1 (4 entries) or 2 far slots, one lane
-              if (rows_b == 2 && fq > 0 && (g > 1 || fq > (ge == 4 ? 1 : 2))) continue;
-              const size_t lanes = (maxlev_rows + rows_b - 1) / rows_b * g;
-              const size_t w = (lanes + 63) / 64;
-              if (w > 8) continue;
-              const size_t key = (w * 4096 + static_cast<size_t>(g * ge)) * 4 + rows_b;
-              if (best_e == 0 || key < best_key) {
-                best_key = key;
-                best_e = ge;
-                best_g = g;
-                best_r = rows_b;
-                best_w = static_cast<int>(w);
-                best_ring = rb;
-                best_fq = fq;
-              }
-            }
-          }
-        if (best_e == 0 && std::getenv("SC23AD_VERBOSE")) {
-          int rb_near = pow2(span_near);
-          while (dev::rpb_lds_bytes(2 * rb_near, maxlev_chain) <= dev::kTriBlockedMaxLds)
-            rb_near *= 2;
-          std::fprintf(stderr,
-                       "[sc23ad plan] no block layout: max deps %d, span %lld (near %lld), "
-                       "max level rows %d, far entries per row %d at ring %d\n",
-                       md_b, span_all, span_near, static_cast<int>(maxlev_rows),
-                       far_count(rb_near), rb_near);
-        }
-        if (best_e > 0) {
-          const int e_b = best_e, g_b = best_g;
-          std::vector<int> rb(static_cast<size_t>(std::max(n, 1)) * g_b * e_b * 2, 0);
-          for (size_t Lv = 0; Lv + 1 < lev_ptr.size(); ++Lv)
-            for (int idx = lev_ptr[Lv]; idx < lev_ptr[Lv + 1]; ++idx) {
-              std::vector<int> code, vals;  // far entries first (one-lane layouts)
-              for (int pass = 0; pass < 2; ++pass)
-                for (int q = lbeg[idx]; q < lbeg[idx + 1]; ++q) {
-                  const bool far =
-                      static_cast<long long>(lev_ptr[Lv + 1]) - lpos[q] > best_ring;
-                  if (far != (pass == 0)) continue;
-                  code.push_back(far ? -(lcol[q] + 1) : lpos[q]);
-                  vals.push_back(static_cast<int>(lval[q]));
-                }
-              for (size_t mm = 0; mm < code.size(); ++mm) {
-                const size_t at =
-                    ((static_cast<size_t>(idx) * g_b + mm % g_b) * e_b + mm / g_b) * 2;
-                rb[at] = code[mm];
-                rb[at + 1] = vals[mm];
-              }
-            }
-          plan.rent_blk.alloc(sizeof(int) * rb.size());
-          plan.rent_blk.upload(rb.data(), sizeof(int) * rb.size());
-          L.rent_blk = plan.rent_blk.get();
-          L.ring_blk = best_ring;
-          L.far_blk = best_fq > 0 ? 1 : 0;
-          L.farq_blk = best_fq;
-          L.e_blk = e_b;
-          L.lanes_blk = g_b;
-          L.rows_blk = best_r;
-          L.waves_blk = best_w;
-          L.ep_maxlev = maxlev_chain;
-        }
-      }
-    }
-  }
-  // Row-parallel mode (integer smoother factors): lanes per row, entries per
-  // lane and waves chosen by plan_rp; SC23AD_TRI_RP=0 keeps the other kernels.
-  if constexpr (std::is_same_v<V, int32_t>) {
-    if (kind == TriKind::kLD && plan.identity) {
-      std::vector<int> chains = chain_lev;
-      plan_rp(plan, n, lbeg, lpos, lval, lev_ptr, chains, span, single_wg_max);
     }
   }
   // FP smoother factors (solvers 0 and 1): the row-parallel kernel with one
@@ -1044,13 +928,11 @@ void build_plan(TriPlan& plan, TriKind kind, int n, const std::vector<int>& rptr
                  "[sc23ad plan] kind %d n %d nnz %zu chains %d levels(max chain) %d "
                  "max level rows %zu launches %d ring %d span %lld max deps %d ep waves %d far %d "
                  "narrow %d copies %d rp waves %d entries %d rows %d lanes %d identity %d "
-                 "| block: waves %d entries %d rows %d lanes %d ring %d far %d "
                  "| rp: pieces %d far %d fence %d\n",
                  static_cast<int>(kind), n, cind.size(), nchain, plan.nlevels, maxlev_rows,
                  plan.nlaunch, L.ring, span, maxdeps, L.ep_waves, L.ep_far, L.ep_narrow,
                  L.ep_copies, L.rp_waves, L.rp_e, L.rp_rows, L.rp_lanes, plan.identity ? 1 : 0,
-                 L.waves_blk, L.e_blk, L.rows_blk, L.lanes_blk, L.ring_blk, L.farq_blk, L.rp_maxlev,
-                 L.rp_farq, L.rp_fence);
+                 L.rp_maxlev, L.rp_farq, L.rp_fence);
   }
 }
 

@@ -108,7 +108,6 @@ struct TriPlan {
   DevBuf lrow, lbeg, lcol, lval, ldiag, ecol, eval, lpos, epos, lent, lev_eptr, rent;
   DevBuf rp_lev, rp_chain;           // row-parallel mode: its levels and chains
   DevBuf rpf_dep, rpf_val, rpf_cnt;  // FP row-parallel layout
-  DevBuf rent_blk;                    // row-parallel entries for the block kernel's ring
   dev::TriLayout layout;
 };
 

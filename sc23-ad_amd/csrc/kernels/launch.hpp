@@ -124,18 +124,6 @@ struct TriLayout {
   int rp_lanes = 1;
   int rp_farq = 0;   // most far entries in one row (stored first; one-lane layouts)
   int rp_stage = 0;  // FP rows over several lanes: products staged in LDS (else shuffled)
-  // the block kernel's own row-parallel layout (four right-hand sides per
-  // workgroup, four values per ring slot): entries as rent, ring slots, far
-  // flag and most far entries per row, entries per lane, lanes per row,
-  // rows per lane, waves
-  const void* rent_blk = nullptr;
-  int ring_blk = 0;
-  int far_blk = 0;
-  int farq_blk = 0;
-  int e_blk = 0;
-  int lanes_blk = 1;
-  int rows_blk = 1;
-  int waves_blk = 0;
   // FP row-parallel mode (one lane per row, rp_e entries in stored order):
   // dependency codes and values by position, and each row's entry count
   const int* rpf_dep = nullptr;
@@ -156,6 +144,7 @@ hipError_t launch_trsv_ep(TriKind kind, const TriLayout& L, const TriSegment& se
 // Row-parallel integer LD solve (one workgroup per chain, 1-64 lanes per row).
 constexpr int kRpMaxLanes = 64;   // lanes per row, 4 to 12 entries each
 constexpr int kRpMaxWaves = 16;   // more than 8: one lane of 4 entries per row
+constexpr int kRpFarSlots = 4;    // far entries per lane of layouts over several lanes
 constexpr int kRpMaxAhead = 4;    // far values are loaded at most this many levels ahead
 constexpr int kRpPadLevels = 12;  // level offsets past a chain's last one
 hipError_t launch_trsv_rp(const TriLayout& L, int bit, int dbit, const void* in, void* out,
@@ -169,18 +158,11 @@ inline size_t rp_lds_bytes(int ring, int maxlev) {
 // ---- block kernels (block.hip): several right-hand sides of one hierarchy --
 // A block vector of n rows and `groups` groups of four right-hand sides holds
 // element (row i, right-hand side r) at ((r / 4) * n + i) * 4 + r % 4.
-// Least level distance of a dependency the block kernel reads from global
-// memory (it fences every 8 levels; its far values are loaded at most 4
-// levels ahead).
-constexpr int kRpbFarLevels = 12;
 // LDS of the FP several-lanes-per-row LD solve: the ring, each thread's e
 // products (staged for the row's ordered subtraction), the level offsets.
 inline size_t rpg_lds_bytes(size_t elem, int ring, int waves, int e, int maxlev, bool stage) {
   return elem * (static_cast<size_t>(ring) + (stage ? static_cast<size_t>(waves) * 64 * e : 0)) +
          sizeof(int) * (static_cast<size_t>(maxlev) + 1);
-}
-inline size_t rpb_lds_bytes(int ring, int maxlev) {
-  return 16 * static_cast<size_t>(ring) + sizeof(int) * (static_cast<size_t>(maxlev) + 1);
 }
 hipError_t launch_permute_blk(int n, int groups, const int* perm, const void* src, void* dst,
                               bool gather, hipStream_t s);
@@ -190,11 +172,11 @@ hipError_t launch_blk_column(int n, int r, void* blk, void* col, bool get, hipSt
 // y = spmv(x) | z - spmv(x) | z + spmv(x) for every right-hand side (y may alias z)
 hipError_t launch_spmv_blk(const DCsr& a, int groups, SpmvMode mode, const void* x,
                            const void* z, void* y, hipStream_t s);
-// Row-parallel LD solve of a block (the layouts of launch_trsv_rp that the
-// block kernel has; see trsv_rp_blk_supported).
+// Row-parallel LD solve of a block: one workgroup per chain and right-hand
+// side (launch_trsv_rp's kernel on 16-byte-strided vectors).
 bool trsv_rp_blk_supported(const TriLayout& L);
-hipError_t launch_trsv_rp_blk(const TriLayout& L, const TriSegment& seg, int groups, int bit,
-                              int dbit, const void* in, void* out, hipStream_t s);
+hipError_t launch_trsv_rp_blk(const TriLayout& L, int groups, int bit, int dbit, const void* in,
+                              void* out, hipStream_t s);
 // Tiled coarse solve of a block: xp holds groups * n * 4 words, tickets two
 // zero-initialised counters that the kernel leaves at zero.
 hipError_t launch_trsv_tiles_blk(TriKind kind, int n, int nb, int groups, const int32_t* tiles,

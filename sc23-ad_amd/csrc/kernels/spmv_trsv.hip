@@ -1315,6 +1315,11 @@ hipError_t tri_ep_launch(const TriLayout& L, const TriSegment& seg, int bit, int
 // addresses per level (128^3 BlockSOR, levels 1-4: 83 / 78 / 92 / 43 us, now
 // 80 / 64 / 62 / 29 us; level 0: 87 -> 82 us) and against the entry-parallel
 // kernel and one launch per wide level (63^3 SOR, whole V-cycle: 5.27 -> 2.61 ms).
+// A block of right-hand sides runs one workgroup per chain and right-hand side
+// (a chain leaves most of the chip idle: 40 chains, 256 CUs), all of one chain
+// on one XCD when the chain count is a multiple of 8; four right-hand sides
+// per workgroup, which loads each entry once, took 1.9 ms of LD solves per
+// 16-vector V-cycle of the 96^3 inclusions system, against 1.1 ms.
 using RpWord4 = __attribute__((ext_vector_type(4))) unsigned;
 template <int kE, int kFq>
 struct RpPre {
@@ -1335,6 +1340,7 @@ struct RpArgs {
 struct RpLane {
   int ent_off;            // its entries' byte offset from the level's first row's
   int row4;               // 4 * its row in the level
+  int vec_off;            // its row's byte offset in the vectors (stride 4 or 16)
   int owner;              // its row for the row's first lane, else INT32_MAX
   int32_t scale;          // 2^bit for the row's first lane, else 0
 };
@@ -1353,7 +1359,7 @@ __device__ __forceinline__ LdsWord* rp_lds(unsigned off) {
   return reinterpret_cast<LdsWord*>(off);
 }
 
-template <int kG, int kE, int kFq>
+template <int kG, int kE, int kS, int kFq>
 __device__ __forceinline__ void rp_load(RpPre<kE, kFq>& r, int lo, int hi, const RpArgs& a,
                                         const RpLane& ln) {
   r.lo = lo;
@@ -1363,7 +1369,7 @@ __device__ __forceinline__ void rp_load(RpPre<kE, kFq>& r, int lo, int hi, const
   for (int h = 0; h < kE / 2; ++h)
     r.ent[h] = __builtin_amdgcn_raw_buffer_load_b128(a.rent, ln.ent_off + 16 * h, loe, 0);
   r.dinv = static_cast<int>(__builtin_amdgcn_raw_buffer_load_b32(a.dinv, ln.row4, lo4, 0));
-  r.in = static_cast<int>(__builtin_amdgcn_raw_buffer_load_b32(a.in, ln.row4, lo4, 0));
+  r.in = static_cast<int>(__builtin_amdgcn_raw_buffer_load_b32(a.in, ln.vec_off, kS * lo4, 0));
 }
 
 // acc + dpp(acc) on 64-bit values, one stage of a group sum: the low words'
@@ -1430,7 +1436,7 @@ __device__ __forceinline__ int32_t rp_finish(uint64_t t, int32_t dinv, int bit, 
 
 // Level L (buffer cur).  nxt: the buffer level L - 1 has freed, filled for
 // level L + kD - 1, whose bounds `pend` holds; `ahead`: level L + kA's buffer.
-template <bool kTail, int kMaxWaves, bool kFar, int kG, int kE, int kD, int kA, int kFq>
+template <bool kTail, int kMaxWaves, bool kFar, int kG, int kE, int kS, int kD, int kA, int kFq>
 __device__ __forceinline__ void rp_level(RpPre<kE, kFq>& cur, RpPre<kE, kFq>& nxt,
                                          RpPre<kE, kFq>& ahead, int L, int2& pend,
                                          const int* lvo, const RpArgs& a,
@@ -1450,14 +1456,14 @@ __device__ __forceinline__ void rp_level(RpPre<kE, kFq>& cur, RpPre<kE, kFq>& nx
   // every ring read is issued before the loads and the first product, so the
   // level pays one LDS round trip, covered in part by issuing the loads
   __builtin_amdgcn_sched_barrier(0);
-  if (!kTail) rp_load<kG, kE, kFq>(nxt, plo, phi, a, ln);
+  if (!kTail) rp_load<kG, kE, kS, kFq>(nxt, plo, phi, a, ln);
   if (kFar) {
 #pragma unroll
     for (int q = 0; q < kFq; ++q) {
       // ~code is 4 * position for a far entry, else past the buffer's end
       const unsigned c = q % 2 ? ahead.ent[q / 2].z : ahead.ent[q / 2].x;
       ahead.xfar[q] = static_cast<int>(
-          __builtin_amdgcn_raw_buffer_load_b32(a.out, static_cast<int>(~c), 0, 0));
+          __builtin_amdgcn_raw_buffer_load_b32(a.out, static_cast<int>(kS * ~c), 0, 0));
     }
   }
   if (!kTail) {
@@ -1488,7 +1494,8 @@ __device__ __forceinline__ void rp_level(RpPre<kE, kFq>& cur, RpPre<kE, kFq>& nx
   if (ln.owner < cur.cnt) {
     const int lo4 = 4 * cur.lo;
     *rp_lds(static_cast<unsigned>(lo4 + ln.row4) & a.ring_mask) = v;
-    __builtin_amdgcn_raw_buffer_store_b32(static_cast<unsigned>(v), a.out, ln.row4, lo4, 0);
+    __builtin_amdgcn_raw_buffer_store_b32(static_cast<unsigned>(v), a.out, ln.vec_off, kS * lo4,
+                                          0);
   }
   // a full fence every fence_mask + 1 levels makes far values visible before
   // any load of them; it also drains the loads in flight, so the plan makes
@@ -1500,15 +1507,15 @@ __device__ __forceinline__ void rp_level(RpPre<kE, kFq>& cur, RpPre<kE, kFq>& nx
 }
 
 // The last nl - L0 < kD levels, nested so that no paths join between them.
-template <int kFirst, int kMaxWaves, bool kFar, int kG, int kE, int kD, int kA, int kFq>
+template <int kFirst, int kMaxWaves, bool kFar, int kG, int kE, int kS, int kD, int kA, int kFq>
 __device__ __forceinline__ void rp_tail(RpPre<kE, kFq> (&buf)[kD], int L0, int nl, int2& pend,
                                         const int* lvo, const RpArgs& a, const RpLane& ln) {
   if constexpr (kFirst < kD - 1) {
     if (L0 + kFirst < nl) {
-      rp_level<true, kMaxWaves, kFar, kG, kE, kD, kA, kFq>(
+      rp_level<true, kMaxWaves, kFar, kG, kE, kS, kD, kA, kFq>(
           buf[kFirst], buf[(kFirst + kD - 1) % kD], buf[(kFirst + kA) % kD], L0 + kFirst, pend,
           lvo, a, ln);
-      rp_tail<kFirst + 1, kMaxWaves, kFar, kG, kE, kD, kA, kFq>(buf, L0, nl, pend, lvo, a, ln);
+      rp_tail<kFirst + 1, kMaxWaves, kFar, kG, kE, kS, kD, kA, kFq>(buf, L0, nl, pend, lvo, a, ln);
     }
   }
 }
@@ -1516,7 +1523,7 @@ __device__ __forceinline__ void rp_tail(RpPre<kE, kFq> (&buf)[kD], int L0, int n
 // LDS: the ring, then the chain's level offsets (max_levels + 1 ints and
 // kRpPadLevels more that repeat the last one).  Far values of level L + kA
 // are loaded in level L, from entries loaded kD - 1 - kA levels before that.
-template <int kMaxWaves, bool kFar, int kG, int kE, int kD, int kA, int kFq>
+template <int kMaxWaves, bool kFar, int kG, int kE, int kS, int kD, int kA, int kFq>
 __global__ __launch_bounds__(64 * kMaxWaves) void k_tri_chain_rp(
     const void* __restrict__ rent, const int32_t* __restrict__ dinv,
     const int* __restrict__ lev_ptr, const int* __restrict__ chain_lev, int n, int ring4, int bit,
@@ -1533,17 +1540,23 @@ __global__ __launch_bounds__(64 * kMaxWaves) void k_tri_chain_rp(
   for (int k = t; k <= nl + kD + 1; k += threads) lvo[k] = lev_ptr[lb + min(k, nl)];
   __syncthreads();
   const unsigned n4 = 4u * static_cast<unsigned>(n);
-  const RpArgs a{rp_buffer(rent, n4 * (kG * kE * 2)), rp_buffer(dinv, n4), rp_buffer(in, n4),
-                 rp_buffer(out, n4), static_cast<unsigned>(ring4) - 1u, bit, dbit, fence - 1};
+  // kS = 1: a plain vector.  kS = 4: right-hand side blockIdx.y of a block
+  // (four values of a row in one 16-byte word, groups of four one after another)
+  const unsigned r = kS == 1 ? 0u : blockIdx.y & 3u;
+  const size_t off = kS == 1 ? 0 : static_cast<size_t>(blockIdx.y >> 2) * n * 4 + r;
+  const unsigned vec_bytes = kS * n4 - 4u * r;
+  const RpArgs a{rp_buffer(rent, n4 * (kG * kE * 2)), rp_buffer(dinv, n4),
+                 rp_buffer(in + off, vec_bytes), rp_buffer(out + off, vec_bytes), static_cast<unsigned>(ring4) - 1u, bit, dbit, fence - 1};
   RpLane ln;
   ln.ent_off = t * (kE * 8);
   ln.row4 = 4 * (t / kG);
+  ln.vec_off = kS * ln.row4;
   ln.owner = t % kG == 0 ? t / kG : INT32_MAX;
   ln.scale = t % kG == 0 ? 1 << bit : 0;
   RpPre<kE, kFq> buf[kD];
 #pragma unroll
   for (int d = 0; d < kD - 1; ++d)
-    rp_load<kG, kE, kFq>(buf[d], __builtin_amdgcn_readfirstlane(lvo[d]),
+    rp_load<kG, kE, kS, kFq>(buf[d], __builtin_amdgcn_readfirstlane(lvo[d]),
                          __builtin_amdgcn_readfirstlane(lvo[d + 1]), a, ln);
   int2 pend = make_int2(lvo[kD - 1], lvo[kD]);
   // Whole rounds of kD levels, then the tail, which loads nothing ahead, in a
@@ -1554,15 +1567,16 @@ __global__ __launch_bounds__(64 * kMaxWaves) void k_tri_chain_rp(
   for (; L0 + kD <= nl; L0 += kD) {
 #pragma unroll
     for (int d = 0; d < kD; ++d)
-      rp_level<false, kMaxWaves, kFar, kG, kE, kD, kA, kFq>(buf[d], buf[(d + kD - 1) % kD],
+      rp_level<false, kMaxWaves, kFar, kG, kE, kS, kD, kA, kFq>(buf[d], buf[(d + kD - 1) % kD],
                                                        buf[(d + kA) % kD], L0 + d, pend, lvo, a,
                                                        ln);
   }
-  rp_tail<0, kMaxWaves, kFar, kG, kE, kD, kA, kFq>(buf, L0, nl, pend, lvo, a, ln);
+  rp_tail<0, kMaxWaves, kFar, kG, kE, kS, kD, kA, kFq>(buf, L0, nl, pend, lvo, a, ln);
 }
 
-template <int kMaxWaves, bool kFar, int kG, int kE, int kD, int kA, int kFq = kFar ? kE : 0>
-hipError_t tri_rp_go(const TriLayout& L, int bit, int dbit, const int32_t* in, int32_t* out, hipStream_t s) {
+template <int kMaxWaves, bool kFar, int kG, int kE, int kS, int kD, int kA, int kFq = kFar ? kE : 0>
+hipError_t tri_rp_go(const TriLayout& L, int nrhs, int bit, int dbit, const int32_t* in,
+                     int32_t* out, hipStream_t s) {
   const size_t lds = rp_lds_bytes(L.rp_ring, L.rp_maxlev);
   if (lds > static_cast<size_t>(kTriBlockedMaxLds) || L.n <= 0 || bit < 0 || bit > 30 ||
       dbit < 0 || dbit > 30 || L.rp_fence < 1 || static_cast<uint64_t>(L.n) * (kG * kE * 8) > UINT32_MAX)
@@ -1570,12 +1584,12 @@ hipError_t tri_rp_go(const TriLayout& L, int bit, int dbit, const int32_t* in, i
   static bool attr = false;
   if (!attr) {
     hipError_t e = hipFuncSetAttribute(
-        reinterpret_cast<const void*>(&k_tri_chain_rp<kMaxWaves, kFar, kG, kE, kD, kA, kFq>),
+        reinterpret_cast<const void*>(&k_tri_chain_rp<kMaxWaves, kFar, kG, kE, kS, kD, kA, kFq>),
         hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(kTriBlockedMaxLds));
     if (e != hipSuccess) return e;
     attr = true;
   }
-  launch_timed(&k_tri_chain_rp<kMaxWaves, kFar, kG, kE, kD, kA, kFq>, dim3(L.rp_nchain),
+  launch_timed(&k_tri_chain_rp<kMaxWaves, kFar, kG, kE, kS, kD, kA, kFq>, dim3(L.rp_nchain, nrhs),
                dim3(64 * L.rp_waves), static_cast<uint32_t>(lds), s,
                L.rent, static_cast<const int32_t*>(L.ldiag), L.rp_lev, L.rp_chain, L.n,
                4 * L.rp_ring, bit, dbit, L.rp_fence, in, out);
@@ -1585,33 +1599,51 @@ hipError_t tri_rp_go(const TriLayout& L, int bit, int dbit, const int32_t* in, i
 // Register layouts and prefetch distances: a level takes 0.1-0.3 us and its
 // entries come from HBM, so the loads run several levels ahead, as far as the
 // 256 registers of a lane allow.
-template <int kMaxWaves, bool kFar>
-hipError_t tri_rp_layout(const TriLayout& L, int bit, int dbit, const int32_t* in, int32_t* out, hipStream_t s) {
+template <int kMaxWaves, int kS, bool kFar>
+hipError_t tri_rp_layout(const TriLayout& L, int nrhs, int bit, int dbit, const int32_t* in,
+                         int32_t* out, hipStream_t s) {
   constexpr int kD8 = kFar ? 6 : 8, kD10 = kFar ? 5 : 8, kD12 = kFar ? 5 : 6;
   constexpr int kA8 = kFar ? 3 : 1, kA10 = kFar ? 2 : 1;
   if (L.rp_lanes <= 1) {
     if (L.rp_e == 4) {
       if (kFar && L.rp_farq == 1)  // one far entry at most, stored first
-        return tri_rp_go<kMaxWaves, kFar, 1, 4, 10, 4, 1>(L, bit, dbit, in, out, s);
-      return tri_rp_go<kMaxWaves, kFar, 1, 4, 10, 4>(L, bit, dbit, in, out, s);
+        return tri_rp_go<kMaxWaves, kFar, 1, 4, kS, 10, 4, 1>(L, nrhs, bit, dbit, in, out, s);
+      return tri_rp_go<kMaxWaves, kFar, 1, 4, kS, 10, 4>(L, nrhs, bit, dbit, in, out, s);
     }
-    if (L.rp_e == 8) return tri_rp_go<kMaxWaves, kFar, 1, 8, kD8, kA8>(L, bit, dbit, in, out, s);
+    if (L.rp_e == 8) return tri_rp_go<kMaxWaves, kFar, 1, 8, kS, kD8, kA8>(L, nrhs, bit, dbit, in, out, s);
     if (L.rp_e == 10)
-      return tri_rp_go<kMaxWaves, kFar, 1, 10, kD10, kA10>(L, bit, dbit, in, out, s);
+      return tri_rp_go<kMaxWaves, kFar, 1, 10, kS, kD10, kA10>(L, nrhs, bit, dbit, in, out, s);
     if (L.rp_e == 12)
-      return tri_rp_go<kMaxWaves, kFar, 1, 12, kD12, kA10>(L, bit, dbit, in, out, s);
+      return tri_rp_go<kMaxWaves, kFar, 1, 12, kS, kD12, kA10>(L, nrhs, bit, dbit, in, out, s);
     return hipErrorInvalidValue;
+  }
+  if constexpr (kFar) {
+    // far entries dealt over the lanes, slot 0 of each lane first: up to
+    // kRpFarSlots per lane
+    auto lanes = [&](auto e_tag) -> hipError_t {
+      constexpr int E = decltype(e_tag)::value, Q = kRpFarSlots;
+      switch (L.rp_lanes) {
+        case 2: return tri_rp_go<kMaxWaves, true, 2, E, kS, 5, 2, Q>(L, nrhs, bit, dbit, in, out, s);
+        case 4: return tri_rp_go<kMaxWaves, true, 4, E, kS, 5, 2, Q>(L, nrhs, bit, dbit, in, out, s);
+        case 8: return tri_rp_go<kMaxWaves, true, 8, E, kS, 5, 2, Q>(L, nrhs, bit, dbit, in, out, s);
+        default: return hipErrorInvalidValue;
+      }
+    };
+    using std::integral_constant;
+    if (L.rp_e == 8) return lanes(integral_constant<int, 8>{});
+    if (L.rp_e == 10) return lanes(integral_constant<int, 10>{});
+    if (L.rp_e == 12) return lanes(integral_constant<int, 12>{});
   }
   if constexpr (!kFar) {
     auto lanes = [&](auto e_tag, auto d_tag) -> hipError_t {
       constexpr int E = decltype(e_tag)::value, D = decltype(d_tag)::value;
       switch (L.rp_lanes) {
-        case 2: return tri_rp_go<kMaxWaves, false, 2, E, D, 1>(L, bit, dbit, in, out, s);
-        case 4: return tri_rp_go<kMaxWaves, false, 4, E, D, 1>(L, bit, dbit, in, out, s);
-        case 8: return tri_rp_go<kMaxWaves, false, 8, E, D, 1>(L, bit, dbit, in, out, s);
-        case 16: return tri_rp_go<kMaxWaves, false, 16, E, D, 1>(L, bit, dbit, in, out, s);
-        case 32: return tri_rp_go<kMaxWaves, false, 32, E, D, 1>(L, bit, dbit, in, out, s);
-        case 64: return tri_rp_go<kMaxWaves, false, 64, E, D, 1>(L, bit, dbit, in, out, s);
+        case 2: return tri_rp_go<kMaxWaves, false, 2, E, kS, D, 1>(L, nrhs, bit, dbit, in, out, s);
+        case 4: return tri_rp_go<kMaxWaves, false, 4, E, kS, D, 1>(L, nrhs, bit, dbit, in, out, s);
+        case 8: return tri_rp_go<kMaxWaves, false, 8, E, kS, D, 1>(L, nrhs, bit, dbit, in, out, s);
+        case 16: return tri_rp_go<kMaxWaves, false, 16, E, kS, D, 1>(L, nrhs, bit, dbit, in, out, s);
+        case 32: return tri_rp_go<kMaxWaves, false, 32, E, kS, D, 1>(L, nrhs, bit, dbit, in, out, s);
+        case 64: return tri_rp_go<kMaxWaves, false, 64, E, kS, D, 1>(L, nrhs, bit, dbit, in, out, s);
         default: return hipErrorInvalidValue;
       }
     };
@@ -1625,19 +1657,21 @@ hipError_t tri_rp_layout(const TriLayout& L, int bit, int dbit, const int32_t* i
   return hipErrorInvalidValue;
 }
 
-template <int kMaxWaves>
-hipError_t tri_rp_far(const TriLayout& L, int bit, int dbit, const int32_t* in, int32_t* out, hipStream_t s) {
-  if (L.rp_farq > 0) return tri_rp_layout<kMaxWaves, true>(L, bit, dbit, in, out, s);
-  return tri_rp_layout<kMaxWaves, false>(L, bit, dbit, in, out, s);
+template <int kMaxWaves, int kS>
+hipError_t tri_rp_far(const TriLayout& L, int nrhs, int bit, int dbit, const int32_t* in,
+                         int32_t* out, hipStream_t s) {
+  if (L.rp_farq > 0) return tri_rp_layout<kMaxWaves, kS, true>(L, nrhs, bit, dbit, in, out, s);
+  return tri_rp_layout<kMaxWaves, kS, false>(L, nrhs, bit, dbit, in, out, s);
 }
 
 // 9-16 waves (128 registers per lane): one lane of 4 entries per row.
-inline hipError_t tri_rp_wide(const TriLayout& L, int bit, int dbit, const int32_t* in,
-                              int32_t* out, hipStream_t s) {
+template <int kS>
+hipError_t tri_rp_wide(const TriLayout& L, int nrhs, int bit, int dbit, const int32_t* in,
+                         int32_t* out, hipStream_t s) {
   if (L.rp_lanes != 1 || L.rp_e != 4) return hipErrorInvalidValue;
-  if (L.rp_farq == 0) return tri_rp_go<16, false, 1, 4, 8, 1>(L, bit, dbit, in, out, s);
-  if (L.rp_farq == 1) return tri_rp_go<16, true, 1, 4, 8, 4, 1>(L, bit, dbit, in, out, s);
-  return tri_rp_go<16, true, 1, 4, 6, 2>(L, bit, dbit, in, out, s);
+  if (L.rp_farq == 0) return tri_rp_go<16, false, 1, 4, kS, 8, 1>(L, nrhs, bit, dbit, in, out, s);
+  if (L.rp_farq == 1) return tri_rp_go<16, true, 1, 4, kS, 8, 4, 1>(L, nrhs, bit, dbit, in, out, s);
+  return tri_rp_go<16, true, 1, 4, kS, 6, 2>(L, nrhs, bit, dbit, in, out, s);
 }
 
 // Row-parallel FP LD solve (solvers 0 and 1): the chains, levels, LDS ring and
@@ -2355,13 +2389,29 @@ hipError_t launch_trsv_ep(TriKind kind, const TriLayout& L, const TriSegment& se
   return tri_ep_launch<TriKind::kDU, 8>(L, seg, bit, dbit, in, o, s);
 }
 
-hipError_t launch_trsv_rp(const TriLayout& L, int bit, int dbit, const void* in_v, void* out_v,
+template <int kS>
+static hipError_t trsv_rp_waves(const TriLayout& L, int nrhs, int bit, int dbit,
+                                const int32_t* in, int32_t* out, hipStream_t s) {
+  if (L.rp_waves <= 1) return tri_rp_far<1, kS>(L, nrhs, bit, dbit, in, out, s);
+  if (L.rp_waves <= 8) return tri_rp_far<8, kS>(L, nrhs, bit, dbit, in, out, s);
+  return tri_rp_wide<kS>(L, nrhs, bit, dbit, in, out, s);
+}
+
+hipError_t launch_trsv_rp(const TriLayout& L, int bit, int dbit, const void* in, void* out,
                           hipStream_t s) {
-  const int32_t* in = static_cast<const int32_t*>(in_v);
-  int32_t* o = static_cast<int32_t*>(out_v);
-  if (L.rp_waves <= 1) return tri_rp_far<1>(L, bit, dbit, in, o, s);
-  if (L.rp_waves <= 8) return tri_rp_far<8>(L, bit, dbit, in, o, s);
-  return tri_rp_wide(L, bit, dbit, in, o, s);
+  return trsv_rp_waves<1>(L, 1, bit, dbit, static_cast<const int32_t*>(in),
+                          static_cast<int32_t*>(out), s);
+}
+
+bool trsv_rp_blk_supported(const TriLayout& L) {
+  return L.rp_waves > 0 && L.n < (1 << 27);  // 32-bit byte offsets into 16 n bytes
+}
+
+hipError_t launch_trsv_rp_blk(const TriLayout& L, int groups, int bit, int dbit, const void* in,
+                              void* out, hipStream_t s) {
+  if (!trsv_rp_blk_supported(L)) return hipErrorInvalidValue;
+  return trsv_rp_waves<4>(L, 4 * groups, bit, dbit, static_cast<const int32_t*>(in),
+                          static_cast<int32_t*>(out), s);
 }
 
 hipError_t launch_trsv_rpf(Elem e, const TriLayout& L, const TriSegment& seg, const void* in,
