@@ -148,15 +148,30 @@ void DevAmg::vcycle_lo_blk(const void* in, void* out, BlockWork& w) const {
 }
 
 void DevAmg::check_errors(BlockWork& w) const {
-  int e = 0;
-  hip_check(hipMemcpyAsync(&e, w.err.get(), sizeof(int), hipMemcpyDeviceToHost, lib_stream()),
+  hip_check(hipMemcpyAsync(w.host_err.get(), w.err.get(), sizeof(int), hipMemcpyDeviceToHost,
+                           lib_stream()),
             "error flag");
   hip_check(hipStreamSynchronize(lib_stream()), "sync");
-  if (e != 0) {
+  if (*w.host_err.get() != 0) {
     hip_check(dev::launch_fill_zero(sizeof(int), w.err.get(), lib_stream()), "error reset");
     hip_check(hipStreamSynchronize(lib_stream()), "sync");
     throw DevError{5, "coarse solve: a block waited too long for its dependencies"};
   }
+}
+
+std::unique_ptr<DevAmg::BlockWork> DevAmg::take_block_work(int groups) {
+  {
+    std::lock_guard<std::mutex> lock(idle_mutex_);
+    if (idle_ && idle_->groups == groups) return std::move(idle_);
+  }
+  return make_block_work(groups);
+}
+
+void DevAmg::give_block_work(std::unique_ptr<BlockWork> w) {
+  std::unique_ptr<BlockWork> old;  // freed after the lock is dropped
+  std::lock_guard<std::mutex> lock(idle_mutex_);
+  old = std::move(idle_);
+  idle_ = std::move(w);
 }
 
 // ---------------------------------------------------------------------------

@@ -185,7 +185,6 @@ int sc23ad_amg_precondition(sc23ad_amg* m, const void* in, void* out, int on_dev
       a.vcycle(di.get(), dout.get(), a.own_work());
       dout.download(out, bytes);
     }
-    hip_check(hipStreamSynchronize(lib_stream()), "sync");
     a.check_errors(a.own_work());
     return SC23AD_OK;
   });
@@ -381,7 +380,7 @@ int sc23ad_amg_precondition_block(sc23ad_amg* m, int nrhs, const int32_t* in, in
     DevAmg& a = *m->d;
     const int groups = (nrhs + 3) / 4;
     const size_t bytes = 16 * static_cast<size_t>(groups) * a.n0();
-    auto w = a.make_block_work(groups);
+    auto w = a.take_block_work(groups);
     if (on_device) {
       a.vcycle_blk(in, out, *w);
     } else {
@@ -390,8 +389,8 @@ int sc23ad_amg_precondition_block(sc23ad_amg* m, int nrhs, const int32_t* in, in
       a.vcycle_blk(di.get(), dout.get(), *w);
       dout.download(out, bytes);
     }
-    hip_check(hipStreamSynchronize(lib_stream()), "sync");
-    a.check_errors(*w);
+    a.check_errors(*w);  // waits for the stream
+    a.give_block_work(std::move(w));
     return SC23AD_OK;
   });
 }

@@ -68,6 +68,17 @@ void DevBuf::download(void* dst, size_t bytes, size_t off) const {
   hip_check(hipStreamSynchronize(lib_stream()), "download sync");
 }
 
+PinnedInt::PinnedInt() {
+  lib_stream();
+  hip_check(hipHostMalloc(reinterpret_cast<void**>(&p_), sizeof(int), hipHostMallocDefault),
+            "hipHostMalloc");
+  *p_ = 0;
+}
+
+PinnedInt::~PinnedInt() {
+  if (p_) (void)hipHostFree(p_);
+}
+
 size_t DevMat::algo_bytes_spmv(size_t elem) const {
   // values + column indices + row pointers + gathered x (one read per column)
   // + y written once.
@@ -1477,17 +1488,15 @@ void DevAmg::smooth(int l, const void* in, void* out, bool inited, Work& w) cons
 }
 
 void DevAmg::check_errors(Work& w) const {
-  if (!lc_plan.dense && !uc_plan.dense && !lc_plan.dense_fp && !uc_plan.dense_fp) return;
-  int e = 0;
-  hip_check(hipMemcpyAsync(&e, w.err.get(), sizeof(int), hipMemcpyDeviceToHost, lib_stream()),
-            "error flag");
-  hip_check(hipStreamSynchronize(lib_stream()), "sync");
-  if (e != 0) {
-    // clear the word so that later calls on this work context start clean
-    const int zero = 0;
-    hip_check(hipMemcpyAsync(w.err.get(), &zero, sizeof(int), hipMemcpyHostToDevice,
+  const bool waits = lc_plan.dense || uc_plan.dense || lc_plan.dense_fp || uc_plan.dense_fp;
+  if (waits)
+    hip_check(hipMemcpyAsync(w.host_err.get(), w.err.get(), sizeof(int), hipMemcpyDeviceToHost,
                              lib_stream()),
-              "error flag reset");
+              "error flag");
+  hip_check(hipStreamSynchronize(lib_stream()), "sync");
+  if (waits && *w.host_err.get() != 0) {
+    // clear the word so that later calls on this work context start clean
+    hip_check(dev::launch_fill_zero(sizeof(int), w.err.get(), lib_stream()), "error flag reset");
     hip_check(hipStreamSynchronize(lib_stream()), "sync");
     throw DevError{5, "coarse solve: a block waited too long for its dependencies"};
   }
