@@ -23,7 +23,10 @@ struct sc23ad_amg_s {
 };
 
 struct sc23ad_mlp_s {
-  DevBuf P, G, M, V, loss;
+  DevBuf P, M, V;
+  DevBuf G;  // the gradient, the loss, then the gradient's partial sums
+  float* loss() const { return G.as<float>() + kMlpParams; }
+  float* part() const { return loss() + 1; }
   int step = 0;
 };
 
@@ -682,11 +685,11 @@ int sc23ad_mlp_create(uint64_t seed, sc23ad_mlp** out) {
     auto m = std::make_unique<sc23ad_mlp>();
     std::vector<float> p(kMlpParams), z(kMlpParams, 0.0f);
     mlp_init(seed, p.data());
-    for (DevBuf* b : {&m->P, &m->G, &m->M, &m->V}) b->alloc(sizeof(float) * kMlpParams);
+    for (DevBuf* b : {&m->P, &m->M, &m->V}) b->alloc(sizeof(float) * kMlpParams);
+    m->G.alloc(sizeof(float) * (kMlpParams + 1) + dev::mlp_part_bytes());
     m->P.upload(p.data(), sizeof(float) * kMlpParams);
     m->M.upload(z.data(), sizeof(float) * kMlpParams);
     m->V.upload(z.data(), sizeof(float) * kMlpParams);
-    m->loss.alloc(sizeof(float));
     *out = m.release();
     return SC23AD_OK;
   });
@@ -737,9 +740,9 @@ int sc23ad_mlp_grad(sc23ad_mlp* m, const float* x, const float* t, int batch, fl
     dx.upload(x, sizeof(float) * batch * kMlpIn);
     dt.upload(t, sizeof(float) * batch * kMlpOut);
     hip_check(dev::launch_mlp_grad(batch, dx.as<float>(), dt.as<float>(), m->P.as<float>(),
-                                   m->G.as<float>(), m->loss.as<float>(), lib_stream()),
+                                   m->G.as<float>(), m->loss(), m->part(), lib_stream()),
               "mlp grad");
-    if (loss) m->loss.download(loss, sizeof(float));
+    if (loss) m->G.download(loss, sizeof(float), sizeof(float) * kMlpParams);
     if (grad) m->G.download(grad, sizeof(float) * kMlpParams);
     return SC23AD_OK;
   });
@@ -755,7 +758,7 @@ int sc23ad_mlp_train(sc23ad_mlp* m, const float* x, const float* t, int batch, i
     dt.upload(t, sizeof(float) * batch * kMlpOut);
     for (int k = 0; k < steps; ++k) {
       hip_check(dev::launch_mlp_grad(batch, dx.as<float>(), dt.as<float>(), m->P.as<float>(),
-                                     m->G.as<float>(), m->loss.as<float>(), lib_stream()),
+                                     m->G.as<float>(), m->loss(), m->part(), lib_stream()),
                 "mlp grad");
       hip_check(dev::launch_adam(kMlpParams, m->P.as<float>(), m->G.as<float>(),
                                  m->M.as<float>(), m->V.as<float>(), lr, ++m->step,
@@ -764,9 +767,9 @@ int sc23ad_mlp_train(sc23ad_mlp* m, const float* x, const float* t, int batch, i
     }
     if (loss) {  // loss at the final parameters
       hip_check(dev::launch_mlp_grad(batch, dx.as<float>(), dt.as<float>(), m->P.as<float>(),
-                                     m->G.as<float>(), m->loss.as<float>(), lib_stream()),
+                                     m->G.as<float>(), m->loss(), m->part(), lib_stream()),
                 "mlp grad");
-      m->loss.download(loss, sizeof(float));
+      m->G.download(loss, sizeof(float), sizeof(float) * kMlpParams);
     }
     return SC23AD_OK;
   });

@@ -357,8 +357,10 @@ hipError_t launch_fill_zero(size_t bytes, void* dst, hipStream_t s);
 // floats), inputs X (B x 8), targets T and outputs Y (B x 2).
 int mlp_param_count();
 hipError_t launch_mlp_forward(int B, const float* X, const float* P, float* Y, hipStream_t s);
+// part: mlp_part_bytes() of scratch
+size_t mlp_part_bytes();
 hipError_t launch_mlp_grad(int B, const float* X, const float* T, const float* P, float* G,
-                           float* loss, hipStream_t s);
+                           float* loss, float* part, hipStream_t s);
 hipError_t launch_adam(int n, float* P, const float* G, float* M, float* V, float lr, int step,
                        hipStream_t s);
 

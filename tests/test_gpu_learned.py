@@ -29,6 +29,23 @@ def test_forward_and_gradient_match_oracle():
     np.testing.assert_allclose(g, go, rtol=1e-3, atol=1e-6 * np.abs(go).max())
 
 
+@pytest.mark.parametrize("batch", [1, 31, 32, 33, 1220, 128 * 32 + 7])
+def test_gradient_at_tile_edges(batch):
+    """Tiles of 32 samples, at most 128 workgroups: one sample, remainders,
+    and more tiles than workgroups.  A sum of `batch` 32-bit terms in any order
+    is within batch * 2^-24 of its absolute sum; the terms themselves carry
+    a few roundings of tanh and products, 1e-5 of the largest gradient."""
+    m = S.Mlp(seed=11)
+    rng = np.random.default_rng(batch)
+    x = rng.uniform(0.0, 1.5, (batch, 8)).astype(np.float32)
+    t = rng.random((batch, 2)).astype(np.float32)
+    lo, go = MO.loss_grad(m.params(), x, t)
+    for _ in range(2):  # the second call finds the first one's partial sums
+        loss, g = m.grad(x, t)
+        assert abs(loss - lo) <= 1e-5 * lo
+        np.testing.assert_allclose(g, go, rtol=1e-4, atol=1e-5 * np.abs(go).max())
+
+
 def test_training_fits_a_smooth_target():
     rng = np.random.default_rng(2)
     x = rng.random((512, 8)).astype(np.float32)
