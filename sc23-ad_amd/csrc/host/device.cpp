@@ -1205,6 +1205,13 @@ void tune_spmv(DevMat& m, Elem e, SpmvMode mode) {
       csr.group = g;
       cands.push_back(csr);
     }
+    // streamed through LDS: one to four tiles of 2048 entries per workgroup
+    for (int r = 16; r <= 256; r *= 2)
+      if (r * avg >= 1024 && r * avg <= 8192) {
+        dev::DCsr st = csr;
+        st.stream = r;
+        cands.push_back(st);
+      }
   } else {
     cands.push_back(csr);
   }
@@ -1228,7 +1235,8 @@ void tune_spmv(DevMat& m, Elem e, SpmvMode mode) {
     const std::string want(f);
     std::vector<dev::DCsr> keep;
     for (const auto& c : cands) {
-      const char* k = !c.soff                            ? "csr"
+      const char* k = c.stream                           ? "stream"
+                      : !c.soff                          ? "csr"
                       : c.scol16                         ? "sell16"
                       : (m.has2 && c.soff == m.d2.soff) ? "sellcol"
                                                          : "sell";
@@ -1255,12 +1263,13 @@ void tune_spmv(DevMat& m, Elem e, SpmvMode mode) {
     hip_check(hipEventElapsedTime(&ms, e0, e1), "elapsed");
     if (std::getenv("SC23AD_VERBOSE"))
       std::fprintf(stderr, "[sc23ad spmv tune] n %d nnz %d %s%s%s%s lanes %d: %.2f us\n",
-                   m.d.n, m.d.nnz, cands[i].soff ? "SELL" : "CSR",
+                   m.d.n, m.d.nnz,
+                   cands[i].soff ? "SELL" : cands[i].stream ? "streamed CSR" : "CSR",
                    (m.has2 && cands[i].soff == m.d2.soff) ? " column-ordered"
                    : cands[i].srow                        ? " sorted"
                                                           : "",
                    cands[i].scol16 ? " 16-bit" : "", cands[i].remap == 1 ? " XCD rows" : "",
-                   cands[i].group, ms * 1000.0f / 5);
+                   cands[i].stream ? cands[i].stream : cands[i].group, ms * 1000.0f / 5);
     if (ms < best) {
       best = ms;
       best_i = i;

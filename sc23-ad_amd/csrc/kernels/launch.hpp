@@ -25,6 +25,9 @@ struct DCsr {
   const int* cind = nullptr;
   const void* val = nullptr;
   int group = 8;  // lanes per row for the integer SpMV (power of two <= 64)
+  // integer CSR: rows per workgroup of the LDS-streamed kernel (16, 32, 64,
+  // 128 or 256), 0: `group` lanes per row
+  int stream = 0;
   // SELL-64 copy (rows with near-uniform lengths): slices of 64 rows, entry k
   // of row r of slice s at soff[s] + 64 k + r, padded with column -1 / value 0.
   // srow (optional): the slices hold rows srow[0], srow[1], ... (rows sorted

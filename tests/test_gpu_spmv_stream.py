@@ -1,0 +1,58 @@
+"""The integer CSR product streamed through LDS (k_spmv_stream_int): every row
+count per workgroup, rows shorter and longer than a tile of 2,048 entries,
+empty rows and workgroups without entries, sizes off the workgroup's.  Whole
+numbers: no tolerance."""
+from __future__ import annotations
+
+import os
+
+import numpy as np
+import pytest
+
+import oracle as O
+import sc23ad as S
+from helpers import export
+
+pytestmark = pytest.mark.gpu
+
+
+def _reference(rptr, cind, val, bit, x):
+    with np.errstate(over="ignore"):  # 64-bit sums wrap
+        p = np.concatenate([[0], np.cumsum(val.astype(np.int64) * x[cind].astype(np.int64))])
+        return ((p[rptr[1:]] - p[rptr[:-1]]) >> bit).astype(np.int32)
+
+
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 32 * 512 - 1, 32 * 512, 128 * 512, 128 * 512 + 77])
+def test_rows_per_workgroup(n):
+    """16, 32 and 128 rows per workgroup, by the number of rows."""
+    rng = np.random.default_rng(n)
+    lens = rng.integers(0, 12, n)
+    lens[rng.integers(0, n, 3)] = [2047, 2048, 5001]
+    lens[n // 3:n // 3 + 300] = 0
+    rptr = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    m = 3001
+    cind = rng.integers(0, m, rptr[-1]).astype(np.int32)
+    val = rng.integers(-2**31, 2**31, rptr[-1]).astype(np.int32)
+    x = rng.integers(-2**31, 2**31, m).astype(np.int32)
+    for bit in (0, 30):
+        assert np.array_equal(S.spmv_int(rptr, cind, val, bit, x),
+                              _reference(rptr, cind, val, bit, x)), bit
+
+
+def test_fused_modes_on_a_hierarchy(monkeypatch):
+    """Forced on every matrix that has a streamed candidate: each level's
+    products and one V-cycle, whose residuals and corrections are fused."""
+    monkeypatch.setenv("SC23AD_SPMV_FORMAT", "stream")
+    sy = S.make_system(S.GEN_INCLUSIONS3D, (24, 8, 2.0, 4.0, 1e4, 3), 5)
+    h = S.Hierarchy(sy.a, S.INT, S.amg_param(S.BLOCK_SOR))
+    path = export(h)
+    amg, oh = S.Amg(h), O.OracleHier(path)
+    os.unlink(path)
+    rng = np.random.default_rng(31)
+    for lv in range(amg.depth):
+        n = oh.level_n(lv)
+        x = rng.integers(-2**29, 2**29, n).astype(np.int32)
+        for op in (S.OP_SPMV_A, S.OP_SPMV_U):
+            assert np.array_equal(amg.level_op(lv, op, x, n), oh.level_op(lv, op, x, n)), lv
+    v = rng.integers(-2**20, 2**20, sy.a.n).astype(np.int32)
+    assert np.array_equal(amg.precondition(v), oh.vcycle(v))
