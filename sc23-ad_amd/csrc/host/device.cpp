@@ -334,6 +334,42 @@ int order_by_level(const std::vector<int>& lev, const std::vector<int>& chain_be
   return maxlev_all;
 }
 
+// Cuts every level of every chain into pieces of at most `cap` rows and
+// uploads their positions; returns them.
+std::vector<int> put_pieces(TriPlan& plan, const std::vector<int>& lev_ptr,
+                            const std::vector<int>& chain_lev, int cap) {
+  std::vector<int> ptr(1, 0), chain;
+  for (size_t c = 0; c + 1 < chain_lev.size(); c += 2) {
+    chain.push_back(static_cast<int>(ptr.size()) - 1);
+    for (int Lv = chain_lev[c]; Lv < chain_lev[c + 1]; ++Lv)
+      for (int p = lev_ptr[Lv]; p < lev_ptr[Lv + 1]; p += cap)
+        ptr.push_back(std::min(p + cap, lev_ptr[Lv + 1]));
+    chain.push_back(static_cast<int>(ptr.size()) - 1);
+  }
+  plan.rp_lev.alloc(sizeof(int) * ptr.size());
+  plan.rp_lev.upload(ptr.data(), sizeof(int) * ptr.size());
+  plan.rp_chain.alloc(sizeof(int) * std::max<size_t>(chain.size(), 2));
+  plan.rp_chain.upload(chain.data(), sizeof(int) * chain.size());
+  plan.layout.rp_lev = plan.rp_lev.as<int>();
+  plan.layout.rp_chain = plan.rp_chain.as<int>();
+  plan.layout.rp_nchain = static_cast<int>(chain_lev.size() / 2);
+  return ptr;
+}
+
+// Whether a single chain whose levels of more than single_wg_max rows would
+// be launched one by one (about 4.4 us each, 0.6 us per narrow level) is
+// better left to those launches than to a row-parallel solve of `cost` ns.
+bool segmented_wins(const std::vector<int>& lev_ptr, int single_wg_max, double cost) {
+  double segmented = 0;
+  bool wide = false;
+  for (size_t Lv = 0; Lv + 1 < lev_ptr.size(); ++Lv) {
+    const bool own = lev_ptr[Lv + 1] - lev_ptr[Lv] > single_wg_max;
+    wide = wide || own;
+    segmented += own ? 4400 : 600;
+  }
+  return wide && segmented <= cost;
+}
+
 // Row-parallel layout of an integer smoother factor (k_tri_chain_rp).
 //
 // A level is cut into pieces of at most 64 waves / lanes rows (rows of a level
@@ -344,10 +380,7 @@ int order_by_level(const std::vector<int>& lev, const std::vector<int>& chain_be
 // are the launch's, each further wave 20 / 47 ns for its barrier and its share
 // of the CU's load bandwidth).  The layout with the least total over the
 // longest chain wins; so narrow levels get one wave, which needs no barrier,
-// and wide ones several.  With one chain, levels of more than single_wg_max
-// rows are otherwise launched one by one (about 4.4 us each, and 0.6 us per
-// narrow level): the row-parallel kernel takes the factor when its total is
-// below that.
+// and wide ones several.
 void plan_rp(TriPlan& plan, int n, const std::vector<int>& lbeg, const std::vector<int>& lpos,
              const std::vector<int32_t>& lval, const std::vector<int>& lev_ptr,
              const std::vector<int>& chain_lev, long long span, int single_wg_max) {
@@ -431,25 +464,8 @@ void plan_rp(TriPlan& plan, int n, const std::vector<int>& lbeg, const std::vect
       }
     }
   if (best_w == 0) return;
-  if (nchain == 1) {
-    double segmented = 0;
-    bool wide = false;
-    for (int Lv = 0; Lv < nlev; ++Lv) {
-      const bool own = lev_ptr[Lv + 1] - lev_ptr[Lv] > single_wg_max;
-      wide = wide || own;
-      segmented += own ? 4400 : 600;
-    }
-    if (wide && segmented <= best) return;
-  }
-  const int cap = 64 * best_w / best_g;
-  std::vector<int> piece_ptr(1, 0), piece_chain;
-  for (size_t c = 0; c < nchain; ++c) {
-    piece_chain.push_back(static_cast<int>(piece_ptr.size()) - 1);
-    for (int Lv = chain_lev[2 * c]; Lv < chain_lev[2 * c + 1]; ++Lv)
-      for (int p = lev_ptr[Lv]; p < lev_ptr[Lv + 1]; p += cap)
-        piece_ptr.push_back(std::min(p + cap, lev_ptr[Lv + 1]));
-    piece_chain.push_back(static_cast<int>(piece_ptr.size()) - 1);
-  }
+  if (nchain == 1 && segmented_wins(lev_ptr, single_wg_max, best)) return;
+  const std::vector<int> piece_ptr = put_pieces(plan, lev_ptr, chain_lev, 64 * best_w / best_g);
   std::vector<int> rent(static_cast<size_t>(n) * best_g * best_e * 2, 0);
   std::vector<int> ord;
   for (int idx = 0; idx < n; ++idx) {
@@ -469,15 +485,8 @@ void plan_rp(TriPlan& plan, int n, const std::vector<int>& lbeg, const std::vect
   }
   plan.rent.alloc(sizeof(int) * rent.size());
   plan.rent.upload(rent.data(), sizeof(int) * rent.size());
-  plan.rp_lev.alloc(sizeof(int) * piece_ptr.size());
-  plan.rp_lev.upload(piece_ptr.data(), sizeof(int) * piece_ptr.size());
-  plan.rp_chain.alloc(sizeof(int) * piece_chain.size());
-  plan.rp_chain.upload(piece_chain.data(), sizeof(int) * piece_chain.size());
   dev::TriLayout& L = plan.layout;
   L.rent = plan.rent.get();
-  L.rp_lev = plan.rp_lev.as<int>();
-  L.rp_chain = plan.rp_chain.as<int>();
-  L.rp_nchain = static_cast<int>(nchain);
   L.rp_maxlev = static_cast<int>(best_pieces);
   L.rp_ring = ring;
   // a value is fenced before a load kRpMaxAhead levels ahead of its use, at
@@ -485,10 +494,139 @@ void plan_rp(TriPlan& plan, int n, const std::vector<int>& lbeg, const std::vect
   L.rp_fence = 32;
   while (farq > 0 && 2 * L.rp_fence + dev::kRpMaxAhead <= far_dist) L.rp_fence *= 2;
   L.rp_e = best_e;
-  L.rp_rows = 1;
   L.rp_lanes = best_g;
   L.rp_waves = best_w;
   L.rp_farq = farq;
+  plan.nlaunch = 1;
+}
+
+// Row-parallel layout of an FP smoother factor (k_tri_chain_rpf): as plan_rp,
+// with the row's ordered subtractions in the cost of a piece,
+//   70 + 10 e + (waves - 1) (2 + 4.5 e elem / 4)                 one lane
+//   150 + 8 e + 2.5 steps + (waves - 1) (2 + 4.5 e elem / 4)     several
+// ns, steps = the entries of the level's longest row rounded up to 8.
+template <typename V>
+void plan_rpf(TriPlan& plan, int n, const std::vector<int>& lbeg, const std::vector<int>& lpos,
+              const std::vector<V>& lval, const std::vector<int>& lev_ptr,
+              const std::vector<int>& chain_lev, long long span, int single_wg_max) {
+  const char* env_rp = std::getenv("SC23AD_TRI_RP");
+  if ((env_rp && env_rp[0] == '0') || n <= 0 || n >= (1 << 27)) return;
+  auto forced = [](const char* name) {
+    const char* e = std::getenv(name);
+    return e ? std::atoi(e) : 0;
+  };
+  const int only_lanes = forced("SC23AD_RP_LANES"), only_waves = forced("SC23AD_RP_WAVES");
+  const int nlev = static_cast<int>(lev_ptr.size()) - 1;
+  constexpr int kT = sizeof(V);
+  std::vector<int> lev_of(static_cast<size_t>(n)), lev_md(nlev, 0);
+  for (int Lv = 0; Lv < nlev; ++Lv)
+    for (int idx = lev_ptr[Lv]; idx < lev_ptr[Lv + 1]; ++idx) {
+      lev_of[idx] = Lv;
+      lev_md[Lv] = std::max(lev_md[Lv], lbeg[idx + 1] - lbeg[idx]);
+    }
+  const int md = *std::max_element(lev_md.begin(), lev_md.end());
+  // LDS ring of at most 128 KB; further dependencies, at least kEpFarLevels
+  // levels back, come from global memory
+  int ring = 4;
+  while (ring * 2 * kT <= 128 * 1024 && ring < span) ring *= 2;
+  if (std::getenv("SC23AD_FP_RING_FAR") && md > 8) {
+    // (tests) the smallest ring the far rule admits
+    long long need = 1;
+    for (int idx = 0; idx < n; ++idx)
+      for (int q = lbeg[idx]; q < lbeg[idx + 1]; ++q)
+        if (lev_of[idx] - lev_of[lpos[q]] < dev::kEpFarLevels)
+          need = std::max(need, static_cast<long long>(lev_ptr[lev_of[idx] + 1]) - lpos[q]);
+    int r = 4;
+    while (r < need) r *= 2;
+    ring = std::min(ring, r);
+  }
+  auto is_far = [&](int idx, int dpos) {
+    return static_cast<long long>(lev_ptr[lev_of[idx] + 1]) - dpos > ring;
+  };
+  int far_slots = 0, far_dist = 1 << 30;  // leading slots of a row that hold far entries
+  for (int idx = 0; idx < n; ++idx)
+    for (int q = lbeg[idx]; q < lbeg[idx + 1]; ++q)
+      if (is_far(idx, lpos[q])) {
+        far_slots = std::max(far_slots, q - lbeg[idx] + 1);
+        far_dist = std::min(far_dist, lev_of[idx] - lev_of[lpos[q]]);
+      }
+  if (far_slots > 0 && far_dist < dev::kEpFarLevels) return;
+  const size_t nchain = chain_lev.size() / 2;
+  double best = 0;
+  int best_g = 0, best_e = 0, best_w = 0;
+  long long best_pieces = 0;
+  for (int g = 1; g <= 64; g *= 2)
+    for (int e : {4, 8}) {
+      if (g * e < md || (only_lanes > 0 && g != only_lanes) ||
+          static_cast<uint64_t>(n) * g * e * kT > UINT32_MAX)
+        continue;
+      for (int w = 1; w <= 8; ++w) {
+        if (only_waves > 0 && w != only_waves) continue;
+        const int cap = 64 * w / g;
+        if (cap == 0) continue;
+        double most = 0;
+        long long pieces = 0;
+        for (size_t c = 0; c < nchain; ++c) {
+          double t = 0;
+          long long k = 0;
+          for (int Lv = chain_lev[2 * c]; Lv < chain_lev[2 * c + 1]; ++Lv) {
+            const int p = (lev_ptr[Lv + 1] - lev_ptr[Lv] + cap - 1) / cap;
+            const int steps = std::max(8, (lev_md[Lv] + 7) / 8 * 8);
+            const double one = g == 1 ? 70 + 10.0 * e : 150 + 8.0 * e + 2.5 * steps;
+            t += p * (one + (w - 1) * (2 + 4.5 * e * kT / 4));
+            k += p;
+          }
+          most = std::max(most, t);
+          pieces = std::max(pieces, k);
+        }
+        if (pieces > (1 << 20) ||
+            dev::rpf_lds_bytes(kT, ring, w, g, e, static_cast<int>(pieces)) >
+                dev::kTriBlockedMaxLds)
+          continue;
+        if (best_w == 0 || most < best) {
+          best = most;
+          best_g = g;
+          best_e = e;
+          best_w = w;
+          best_pieces = pieces;
+        }
+      }
+    }
+  if (best_w == 0 || (nchain == 1 && segmented_wins(lev_ptr, single_wg_max, best))) return;
+  const std::vector<int> ptr = put_pieces(plan, lev_ptr, chain_lev, 64 * best_w / best_g);
+  std::vector<int> steps(std::max<size_t>(ptr.size() - 1, 1), 8);
+  for (size_t p = 0; p + 1 < ptr.size(); ++p)
+    for (int idx = ptr[p]; idx < ptr[p + 1]; ++idx)
+      steps[p] = std::max(steps[p], (lbeg[idx + 1] - lbeg[idx] + 7) / 8 * 8);
+  // entry m of a row: lane m / e, slot m % e; absent ones name the zero slot
+  const size_t slots = static_cast<size_t>(best_g) * best_e;
+  std::vector<int> dep(static_cast<size_t>(n) * slots, ring * kT);
+  std::vector<V> val(dep.size(), V(0));
+  for (int idx = 0; idx < n; ++idx)
+    for (int q = lbeg[idx]; q < lbeg[idx + 1]; ++q) {
+      const size_t at = static_cast<size_t>(idx) * slots + (q - lbeg[idx]);
+      dep[at] = is_far(idx, lpos[q]) ? ~(lpos[q] * kT) : (lpos[q] & (ring - 1)) * kT;
+      val[at] = lval[q];
+    }
+  plan.rpf_dep.alloc(sizeof(int) * dep.size());
+  plan.rpf_dep.upload(dep.data(), sizeof(int) * dep.size());
+  plan.rpf_val.alloc(sizeof(V) * val.size());
+  plan.rpf_val.upload(val.data(), sizeof(V) * val.size());
+  plan.rp_steps.alloc(sizeof(int) * steps.size());
+  plan.rp_steps.upload(steps.data(), sizeof(int) * steps.size());
+  dev::TriLayout& L = plan.layout;
+  L.rpf_dep = plan.rpf_dep.as<int>();
+  L.rpf_val = plan.rpf_val.get();
+  L.rp_steps = plan.rp_steps.as<int>();
+  L.rp_maxlev = static_cast<int>(best_pieces);
+  L.rp_ring = ring;
+  L.rp_fence = 32;  // as in plan_rp
+  while (far_slots > 0 && 2 * L.rp_fence + dev::kRpMaxAhead <= far_dist) L.rp_fence *= 2;
+  L.rp_e = best_e;
+  L.rp_lanes = best_g;
+  L.rp_waves = best_w;
+  L.rp_farq = far_slots;
+  L.ep_far = far_slots > 0 ? 1 : 0;
   plan.nlaunch = 1;
 }
 
@@ -768,169 +906,11 @@ void build_plan(TriPlan& plan, TriKind kind, int n, const std::vector<int>& rptr
                         ? 1 : 0;
     }
   }
-  // FP smoother factors (solvers 0 and 1): the row-parallel kernel with one
-  // lane per row keeps each row's stored order, so it applies to rows of at
-  // most 8 dependencies, with a ring of at most 128 KB and the same far rule.
-  // SC23AD_TRI_RP=0 keeps the level-pipelined kernel.
+  // FP smoother factors (solvers 0 and 1): plan_rpf; SC23AD_TRI_RP=0 keeps
+  // the level-pipelined kernel.
   if constexpr (!std::is_same_v<V, int32_t>) {
-    int md = 0;
-    for (int idx = 0; idx < n; ++idx) md = std::max(md, lbeg[idx + 1] - lbeg[idx]);
-    const char* env_rp = std::getenv("SC23AD_TRI_RP");
-    int fring = 2;
-    while (fring * 2 * sizeof(V) <= 128 * 1024 && fring < span) fring *= 2;
-    size_t lds = sizeof(V) * static_cast<size_t>(fring) +
-                 sizeof(int) * (static_cast<size_t>(maxlev_chain) + 1);
-    // one row per lane, or two where a level has more than 512 rows
-    // (SC23AD_RP_ROWS=2: two rows per lane wherever the layout applies)
-    const char* env_rows = std::getenv("SC23AD_RP_ROWS");
-    const int fp_rows = (maxlev_rows > 8 * 64 || (env_rows && env_rows[0] == '2')) ? 2 : 1;
-    if (kind == TriKind::kLD && plan.identity && one_launch_chains && md <= 8 &&
-        maxlev_rows <= static_cast<size_t>(fp_rows) * 8 * 64 && lds <= dev::kTriBlockedMaxLds &&
-        !(env_rp && env_rp[0] == '0')) {
-      std::vector<int> lev_of(static_cast<size_t>(std::max(n, 1)), 0);
-      for (size_t Lv = 0; Lv + 1 < lev_ptr.size(); ++Lv)
-        for (int idx = lev_ptr[Lv]; idx < lev_ptr[Lv + 1]; ++idx)
-          lev_of[idx] = static_cast<int>(Lv);
-      const int e = md <= 4 ? 4 : 8;
-      std::vector<int> rdep(static_cast<size_t>(std::max(n, 1)) * e, 0),
-          rcnt(static_cast<size_t>(std::max(n, 1)), 0);
-      std::vector<V> rval(rdep.size(), V(0));
-      bool fits = true, any_far = false;
-      for (size_t Lv = 0; Lv + 1 < lev_ptr.size() && fits; ++Lv)
-        for (int idx = lev_ptr[Lv]; idx < lev_ptr[Lv + 1]; ++idx) {
-          rcnt[idx] = lbeg[idx + 1] - lbeg[idx];
-          for (int q = lbeg[idx]; q < lbeg[idx + 1]; ++q) {
-            const int dpos = lpos[q];
-            const bool in_ring = static_cast<long long>(lev_ptr[Lv + 1]) - dpos <= fring;
-            const bool far = !in_ring && lev_of[idx] - lev_of[dpos] >= dev::kEpFarLevels;
-            if (!in_ring && !far) fits = false;
-            any_far = any_far || far;
-            const size_t at = static_cast<size_t>(idx) * e + (q - lbeg[idx]);
-            rdep[at] = far ? -(lcol[q] + 1) : dpos;
-            rval[at] = lval[q];
-          }
-        }
-      if (fits) {
-        plan.rpf_dep.alloc(sizeof(int) * rdep.size());
-        plan.rpf_dep.upload(rdep.data(), sizeof(int) * rdep.size());
-        plan.rpf_val.alloc(sizeof(V) * rval.size());
-        plan.rpf_val.upload(rval.data(), sizeof(V) * rval.size());
-        plan.rpf_cnt.alloc(sizeof(int) * rcnt.size());
-        plan.rpf_cnt.upload(rcnt.data(), sizeof(int) * rcnt.size());
-        L.rpf_dep = plan.rpf_dep.as<int>();
-        L.rpf_val = plan.rpf_val.get();
-        L.rpf_cnt = plan.rpf_cnt.as<int>();
-        L.ring = fring;
-        L.ep_far = any_far ? 1 : 0;
-        L.ep_maxlev = maxlev_chain;
-        L.rp_e = e;
-        L.rp_rows = fp_rows;
-        int rw = 1;
-        while (rw < 8 && static_cast<size_t>(rw) * 64 * fp_rows < maxlev_rows) rw *= 2;
-        L.rp_waves = rw;
-      }
-    } else if (kind == TriKind::kLD && plan.identity && one_launch_chains && md > 8 &&
-               md <= 16 * 8 && lds <= dev::kTriBlockedMaxLds &&
-               !(env_rp && env_rp[0] == '0')) {
-      // several lanes per row (k_tri_chain_rpg): kG chunks of kE entries, the
-      // fewest waves (at most 8), then the fewest padded slots; every
-      // dependency in the ring, or (rows over 2 or 4 lanes, shuffled) the
-      // far rule of the one-lane kernel
-      // FP32 chunks of 16 entries only where 4 or 8 do not fit in 8 waves
-      // (wide levels of long rows: at 160^3 the FP32 solve went from 0.55 to
-      // 0.43 s, while FP64 rows of 16 measured slower than the
-      // level-pipelined kernel; SC23AD_RP_E16=1, tests: wherever they fit)
-      const bool e16_first = std::getenv("SC23AD_RP_E16") != nullptr;
-      int best_g = 0, best_e = 0;
-      size_t best_key = 0;
-      for (int g = 2; g <= 16; g *= 2)
-        for (int ge : {4, 8, 16}) {
-          if (g * ge < md || (ge == 16 && sizeof(V) == 8)) continue;
-          const size_t w = (maxlev_rows * g + 63) / 64;
-          size_t key = w * 4096 + static_cast<size_t>(g * ge);
-          if ((ge == 16) != e16_first) key += static_cast<size_t>(1) << 30;
-          if (w <= 8 && (best_g == 0 || key < best_key)) {
-            best_key = key;
-            best_g = g;
-            best_e = ge;
-          }
-        }
-      bool fits = best_g > 0;
-      // FP64 rows over 16 lanes stage their products in LDS when the ring
-      // covering the span and the staging area fit together; every other
-      // row shuffles them to its lanes, which measured faster for FP32 rows
-      // (one shuffle per product) and for FP64 rows over at most 8 lanes
-      bool stage = false;
-      if (fits && sizeof(V) == 8 && best_g == 16) {
-        const int w = static_cast<int>((maxlev_rows * best_g + 63) / 64);
-        stage = dev::rpg_lds_bytes(sizeof(V), fring, w, best_e, maxlev_chain, true) <=
-                dev::kTriBlockedMaxLds;
-        // FP64 rows of 16 chunks of 8 spill their registers when shuffled
-        if (!stage && sizeof(V) == 8 && best_g == 16 && best_e == 8) fits = false;
-      }
-      const bool far_ok = !stage && best_g <= 4;
-      std::vector<int> lev_of(static_cast<size_t>(std::max(n, 1)), 0);
-      for (size_t Lv = 0; Lv + 1 < lev_ptr.size(); ++Lv)
-        for (int idx = lev_ptr[Lv]; idx < lev_ptr[Lv + 1]; ++idx)
-          lev_of[idx] = static_cast<int>(Lv);
-      // SC23AD_FP_RING_FAR=1 (tests): the smallest ring the far rule admits,
-      // so that smaller factors take the far path too
-      if (far_ok && std::getenv("SC23AD_FP_RING_FAR")) {
-        long long need = 1;
-        for (int idx = 0; idx < n; ++idx)
-          for (int q = lbeg[idx]; q < lbeg[idx + 1]; ++q)
-            if (lev_of[idx] - lev_of[lpos[q]] < dev::kEpFarLevels)
-              need = std::max(need, static_cast<long long>(lev_ptr[lev_of[idx] + 1]) - lpos[q]);
-        int r = 2;
-        while (r < need) r *= 2;
-        fring = std::min(fring, r);
-      }
-      // a dependency outside the ring is read from global memory when it is
-      // at least kEpFarLevels levels back
-      auto is_far = [&](int idx, int dpos) {
-        return static_cast<long long>(lev_ptr[lev_of[idx] + 1]) - dpos > fring;
-      };
-      bool any_far = false;
-      for (int idx = 0; idx < n && fits; ++idx)
-        for (int q = lbeg[idx]; q < lbeg[idx + 1]; ++q)
-          if (is_far(idx, lpos[q])) {
-            if (far_ok && lev_of[idx] - lev_of[lpos[q]] >= dev::kEpFarLevels)
-              any_far = true;
-            else
-              fits = false;
-          }
-      if (fits) {
-        const size_t slots = static_cast<size_t>(best_g) * best_e;
-        std::vector<int> rdep(static_cast<size_t>(std::max(n, 1)) * slots, 0),
-            rcnt(static_cast<size_t>(std::max(n, 1)), 0);
-        std::vector<V> rval(rdep.size(), V(0));
-        for (int idx = 0; idx < n; ++idx) {
-          rcnt[idx] = lbeg[idx + 1] - lbeg[idx];
-          for (int q = lbeg[idx]; q < lbeg[idx + 1]; ++q) {
-            const size_t at = static_cast<size_t>(idx) * slots + (q - lbeg[idx]);
-            // entry m: lane m / kE, slot m % kE; a far one names -(position + 1)
-            rdep[at] = is_far(idx, lpos[q]) ? -(lpos[q] + 1) : lpos[q];
-            rval[at] = lval[q];
-          }
-        }
-        plan.rpf_dep.alloc(sizeof(int) * rdep.size());
-        plan.rpf_dep.upload(rdep.data(), sizeof(int) * rdep.size());
-        plan.rpf_val.alloc(sizeof(V) * rval.size());
-        plan.rpf_val.upload(rval.data(), sizeof(V) * rval.size());
-        plan.rpf_cnt.alloc(sizeof(int) * rcnt.size());
-        plan.rpf_cnt.upload(rcnt.data(), sizeof(int) * rcnt.size());
-        L.rpf_dep = plan.rpf_dep.as<int>();
-        L.rpf_val = plan.rpf_val.get();
-        L.rpf_cnt = plan.rpf_cnt.as<int>();
-        L.ring = fring;
-        L.ep_far = any_far ? 1 : 0;
-        L.ep_maxlev = maxlev_chain;
-        L.rp_e = best_e;
-        L.rp_lanes = best_g;
-        L.rp_waves = static_cast<int>((maxlev_rows * best_g + 63) / 64);
-        L.rp_stage = stage ? 1 : 0;
-      }
-    }
+    if (kind == TriKind::kLD && plan.identity)
+      plan_rpf(plan, n, lbeg, lpos, lval, lev_ptr, chain_lev, span, single_wg_max);
   }
   int maxdeps = 0;
   for (int idx = 0; idx < n; ++idx) maxdeps = std::max(maxdeps, lbeg[idx + 1] - lbeg[idx]);
@@ -938,11 +918,11 @@ void build_plan(TriPlan& plan, TriKind kind, int n, const std::vector<int>& rptr
     std::fprintf(stderr,
                  "[sc23ad plan] kind %d n %d nnz %zu chains %d levels(max chain) %d "
                  "max level rows %zu launches %d ring %d span %lld max deps %d ep waves %d far %d "
-                 "narrow %d copies %d rp waves %d entries %d rows %d lanes %d identity %d "
+                 "narrow %d copies %d rp waves %d entries %d rows 1 lanes %d identity %d "
                  "| rp: pieces %d far %d fence %d\n",
                  static_cast<int>(kind), n, cind.size(), nchain, plan.nlevels, maxlev_rows,
                  plan.nlaunch, L.ring, span, maxdeps, L.ep_waves, L.ep_far, L.ep_narrow,
-                 L.ep_copies, L.rp_waves, L.rp_e, L.rp_rows, L.rp_lanes, plan.identity ? 1 : 0,
+                 L.ep_copies, L.rp_waves, L.rp_e, L.rp_lanes, plan.identity ? 1 : 0,
                  L.rp_maxlev, L.rp_farq, L.rp_fence);
   }
 }
@@ -1451,8 +1431,8 @@ void DevAmg::trsv(const TriPlan& plan, const DevMat& m, const void* in, void* ou
               "trsv rp");
     return;
   }
-  if (plan.layout.rpf_dep && elem != Elem::kI32 && plan.segs.size() == 1) {
-    hip_check(dev::launch_trsv_rpf(elem, plan.layout, plan.segs[0], in, out, lib_stream()),
+  if (plan.layout.rpf_dep && elem != Elem::kI32) {
+    hip_check(dev::launch_trsv_rpf(elem, plan.layout, in, out, lib_stream()),
               "trsv rp fp");
     return;
   }

@@ -120,8 +120,8 @@ struct TriPlan {
   DevBuf tmask;
   // level-ordered layout used by the level-scheduled kernels
   DevBuf lrow, lbeg, lcol, lval, ldiag, ecol, eval, lpos, epos, lent, lev_eptr, rent;
-  DevBuf rp_lev, rp_chain;           // row-parallel mode: its levels and chains
-  DevBuf rpf_dep, rpf_val, rpf_cnt;  // FP row-parallel layout
+  DevBuf rp_lev, rp_chain, rp_steps;  // row-parallel mode: its pieces and chains
+  DevBuf rpf_dep, rpf_val;            // FP row-parallel layout
   dev::TriLayout layout;
 };
 

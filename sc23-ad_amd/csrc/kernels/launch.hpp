@@ -111,8 +111,7 @@ struct TriLayout {
   int ep_acc = 0;    // accumulator slots in LDS
   // row-parallel mode (LD factors with short rows): rp_lanes lanes per row,
   // each holding rp_e entries (int2 {code, -val}, padded, see k_tri_chain_rp)
-  // of its row, rp_rows rows per lane (FP, one lane per row only), rp_waves
-  // waves per chain; its own levels (pieces of the level schedule's), chains
+  // of its row, rp_waves waves per chain; its own levels (pieces of the level schedule's), chains
   // and ring, and the far rule of the entry-parallel mode
   const void* rent = nullptr;
   const int* rp_lev = nullptr;
@@ -123,15 +122,13 @@ struct TriLayout {
   int rp_fence = 1;   // levels between full fences (power of two; far entries only)
   int rp_waves = 0;  // > 0: use the row-parallel kernel
   int rp_e = 0;
-  int rp_rows = 0;
   int rp_lanes = 1;
-  int rp_farq = 0;   // most far entries in one row (stored first; one-lane layouts)
-  int rp_stage = 0;  // FP rows over several lanes: products staged in LDS (else shuffled)
-  // FP row-parallel mode (one lane per row, rp_e entries in stored order):
-  // dependency codes and values by position, and each row's entry count
+  int rp_farq = 0;   // leading slots per row that can hold a far entry
+  // FP row-parallel mode (rp_lanes lanes of rp_e entries per row, in stored
+  // order): dependency codes and values by position, subtractions per piece
   const int* rpf_dep = nullptr;
   const void* rpf_val = nullptr;
-  const int* rpf_cnt = nullptr;
+  const int* rp_steps = nullptr;
   int n = 0;
 };
 // Entry-parallel integer solve (one workgroup per chain).
@@ -152,8 +149,8 @@ constexpr int kRpMaxAhead = 4;    // far values are loaded at most this many lev
 constexpr int kRpPadLevels = 12;  // level offsets past a chain's last one
 hipError_t launch_trsv_rp(const TriLayout& L, int bit, int dbit, const void* in, void* out,
                           hipStream_t s);
-hipError_t launch_trsv_rpf(Elem e, const TriLayout& L, const TriSegment& seg, const void* in,
-                           void* out, hipStream_t s);
+hipError_t launch_trsv_rpf(Elem e, const TriLayout& L, const void* in, void* out,
+                           hipStream_t s);
 inline size_t rp_lds_bytes(int ring, int maxlev) {
   return sizeof(int32_t) * static_cast<size_t>(ring) +
          sizeof(int) * (static_cast<size_t>(maxlev) + 1 + kRpPadLevels);
@@ -161,11 +158,15 @@ inline size_t rp_lds_bytes(int ring, int maxlev) {
 // ---- block kernels (block.hip): several right-hand sides of one hierarchy --
 // A block vector of n rows and `groups` groups of four right-hand sides holds
 // element (row i, right-hand side r) at ((r / 4) * n + i) * 4 + r % 4.
-// LDS of the FP several-lanes-per-row LD solve: the ring, each thread's e
-// products (staged for the row's ordered subtraction), the level offsets.
-inline size_t rpg_lds_bytes(size_t elem, int ring, int waves, int e, int maxlev, bool stage) {
-  return elem * (static_cast<size_t>(ring) + (stage ? static_cast<size_t>(waves) * 64 * e : 0)) +
-         sizeof(int) * (static_cast<size_t>(maxlev) + 1);
+// LDS of the FP row-parallel LD solve (see k_tri_chain_rpf).
+constexpr int kRpfReadAhead = 3 * 8 * 8;  // bytes read past the last row's products
+inline size_t rpf_lds_bytes(size_t elem, int ring, int waves, int lanes, int e, int maxlev) {
+  const size_t stage = lanes > 1 ? static_cast<size_t>(64 * waves / lanes) *
+                                           (static_cast<size_t>(lanes) * e * elem + 16) +
+                                       kRpfReadAhead
+                                 : 0;
+  return elem * static_cast<size_t>(ring) + 16 + stage +
+         2 * sizeof(int) * (static_cast<size_t>(maxlev) + 1 + kRpPadLevels);
 }
 hipError_t launch_permute_blk(int n, int groups, const int* perm, const void* src, void* dst,
                               bool gather, hipStream_t s);

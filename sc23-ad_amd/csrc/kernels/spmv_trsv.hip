@@ -1753,380 +1753,295 @@ hipError_t tri_rp_wide(const TriLayout& L, int nrhs, int bit, int dbit, const in
   return tri_rp_go<16, true, 1, 4, kS, 6, 2>(L, nrhs, bit, dbit, in, out, s);
 }
 
-// Row-parallel FP LD solve (solvers 0 and 1): the chains, levels, LDS ring and
-// far rule of k_tri_chain_rp with one lane per row.  A row's products are
-// subtracted in stored order, one at a time, as the sequential solve does
-// (entries past the row's count are skipped, not added as zeros), so the
-// result is the reference's bit for bit.  Entries are stored by position:
-// kE dependency codes (as in k_tri_chain_ep) and kE values, and the count.
-template <typename T, int kE, int kR>
+// Row-parallel FP LD solve (solvers 0 and 1): the chains, pieces, LDS ring,
+// far rule and buffer addressing of k_tri_chain_rp, with a row's products
+// subtracted one at a time in stored order, as the sequential solve does, so
+// the result is the reference's bit for bit.
+//
+// 2^lg lanes form the products of a row, kE consecutive entries each.  With
+// one lane they are subtracted as they come.  With several they go through
+// LDS: every lane writes its products to the row's slots and all lanes of the
+// row (one wave, whose LDS accesses stay in order) read them back, 16 bytes
+// at a time, two blocks of 8 ahead of the subtractions; a piece subtracts as
+// many as its longest row has, rounded up to 8.  An absent entry names the
+// zero slot behind the ring and has the value +0, so its product is +0, and
+// t - (+0) is t for every t: no count is checked.  What bounds a level is that
+// chain of subtractions and the instructions a wave issues.
+// Against the form that shuffled every product to the row's lanes and
+// selected by the row's count, several rows' worth of steps per level
+// whatever their length: 96^3 FP64 solve 45.7 -> 24.3 ms, 48^3 27-point FP32
+// solve 70.4 -> 37.8 ms.
+template <typename T>
+struct FpWords;
+template <>
+struct FpWords<float> {
+  static constexpr int k16 = 4;  // values in 16 bytes
+  static __device__ __forceinline__ float load(__amdgpu_buffer_rsrc_t b, int v, int s) {
+    return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(b, v, s, 0));
+  }
+  static __device__ __forceinline__ void store(float x, __amdgpu_buffer_rsrc_t b, int v, int s) {
+    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(x), b, v, s, 0);
+  }
+};
+using RpWord2 = __attribute__((ext_vector_type(2))) unsigned;
+template <>
+struct FpWords<double> {
+  static constexpr int k16 = 2;
+  static __device__ __forceinline__ double load(__amdgpu_buffer_rsrc_t b, int v, int s) {
+    return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(b, v, s, 0));
+  }
+  static __device__ __forceinline__ void store(double x, __amdgpu_buffer_rsrc_t b, int v, int s) {
+    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(RpWord2, x), b, v, s, 0);
+  }
+};
+template <typename T>
+using FpVec16 = __attribute__((ext_vector_type(16 / sizeof(T)))) T;
+template <typename T>
+using LdsOf = __attribute__((address_space(3))) T;
+template <typename T>
+__device__ __forceinline__ LdsOf<T>* fp_lds(unsigned off) {  // as rp_lds
+  return reinterpret_cast<LdsOf<T>*>(off);
+}
+
+template <typename T, int kE, int kFq>
 struct RpfPre {
-  int lo, hi;
-  int dep[kR][kE];
-  T val[kR][kE];
-  T xfar[kR][kE];
-  T dinv[kR], in[kR];
-  int cnt[kR];
+  int lo, cnt, steps;     // first position, rows, subtractions per row (scalars)
+  RpWord4 code[kE / 4];
+  FpVec16<T> val[kE * sizeof(T) / 16];
+  T xfar[kFq > 0 ? kFq : 1];
+  T dinv, in;
 };
 
-// kR rows per lane: lane t serves rows t, t + kThreads, ... of the level.
-template <int kThreads, typename T, int kE, int kR>
-__device__ __forceinline__ void rpf_load(RpfPre<T, kE, kR>& r, int lo, int hi,
-                                         const int* __restrict__ rdep, const T* __restrict__ rval,
-                                         const int* __restrict__ rcnt,
-                                         const T* __restrict__ dinv,
-                                         const T* __restrict__ in) {
+struct RpfArgs {
+  __amdgpu_buffer_rsrc_t code, val, dinv, in, out;
+  unsigned ring_mask;     // ring size in bytes - 1
+  int lg;                 // log2 of the lanes per row
+  int fence_mask;
+};
+
+struct RpfLane {
+  int code_off, val_off;  // its entries' byte offsets from the piece's first row's
+  int row_off;            // its row's byte offset in a vector
+  int owner;              // its row for the row's first lane, else INT32_MAX
+  unsigned put, get;      // LDS offsets: its products, the row's products
+};
+
+template <typename T, int kE, int kFq>
+__device__ __forceinline__ T rpf_val(const RpfPre<T, kE, kFq>& r, int q) {
+  constexpr int k = FpWords<T>::k16;
+  return r.val[q / k][q % k];
+}
+
+template <typename T, int kE, int kFq>
+__device__ __forceinline__ void rpf_load(RpfPre<T, kE, kFq>& r, int lo, int hi, int steps,
+                                         const RpfArgs& a, const RpfLane& ln) {
+  constexpr int kT = sizeof(T);
   r.lo = lo;
-  r.hi = hi;
+  r.cnt = hi - lo;
+  r.steps = steps;
+  const unsigned e = static_cast<unsigned>(lo) << a.lg;
+  const int ce = static_cast<int>(e * (kE * 4)), ve = static_cast<int>(e * (kE * kT));
 #pragma unroll
-  for (int u = 0; u < kR; ++u) {
-    const int idx = lo + static_cast<int>(threadIdx.x) + u * kThreads;
-    const int id = idx < hi ? idx : 0;  // lanes past the level's end load position 0
+  for (int h = 0; h < kE / 4; ++h)
+    r.code[h] = __builtin_amdgcn_raw_buffer_load_b128(a.code, ln.code_off + 16 * h, ce, 0);
 #pragma unroll
-    for (int q = 0; q < kE; ++q) {
-      r.dep[u][q] = rdep[static_cast<size_t>(id) * kE + q];
-      r.val[u][q] = rval[static_cast<size_t>(id) * kE + q];
-    }
-    r.cnt[u] = rcnt[id];
-    r.dinv[u] = dinv[id];
-    r.in[u] = in[id];
-  }
-}
-
-template <int kThreads, typename T, int kE, int kR>
-__device__ __forceinline__ void rpf_far(RpfPre<T, kE, kR>& r, const T* out) {
-#pragma unroll
-  for (int u = 0; u < kR; ++u) {
-    const bool ok = r.lo + static_cast<int>(threadIdx.x) + u * kThreads < r.hi;
-#pragma unroll
-    for (int q = 0; q < kE; ++q) {
-      const int d = r.dep[u][q];
-      r.xfar[u][q] = out[(ok && d < 0) ? -d - 1 : 0];
-    }
-  }
-}
-
-template <typename T, TriKind K, int kWaves, bool kFar, int kE, int kR, int kD, int kA>
-__device__ __forceinline__ void rpf_level(RpfPre<T, kE, kR>& cur, RpfPre<T, kE, kR>& ahead,
-                                          int L, int nl, const int* lvo, T* ring, int rmask,
-                                          const int* __restrict__ rdep,
-                                          const T* __restrict__ rval,
-                                          const int* __restrict__ rcnt,
-                                          const T* __restrict__ dinv,
-                                          const T* __restrict__ in, T* out) {
-  constexpr int kThreads = 64 * kWaves;
-  const int Lp = min(L + kD, nl);
-  const int plo = lvo[Lp], phi = lvo[min(Lp + 1, nl)];
-  if (kFar) rpf_far<kThreads>(ahead, out);
-  T xv[kR][kE];
-#pragma unroll
-  for (int u = 0; u < kR; ++u)
-#pragma unroll
-    for (int q = 0; q < kE; ++q) xv[u][q] = ring[cur.dep[u][q] & rmask];
-  if (kFar) {
-#pragma unroll
-    for (int u = 0; u < kR; ++u)
-#pragma unroll
-      for (int q = 0; q < kE; ++q)
-        if (__any(cur.dep[u][q] < 0)) xv[u][q] = cur.dep[u][q] < 0 ? cur.xfar[u][q] : xv[u][q];
-  }
-#pragma unroll
-  for (int u = 0; u < kR; ++u) {
-    T t = cur.in[u];
-#pragma unroll
-    for (int q = 0; q < kE; ++q) t = q < cur.cnt[u] ? acc_sub<T>(t, cur.val[u][q], xv[u][q]) : t;
-    const int k = cur.lo + static_cast<int>(threadIdx.x) + u * kThreads;
-    if (k < cur.hi) {
-      const T v = acc_final<T, K>(t, cur.dinv[u], 0, 0);
-      ring[k & rmask] = v;
-      out[k] = v;
-    }
-  }
-  if (kFar && (L % kEpFence) == kEpFence - 1)
-    __syncthreads();
-  else
-    ep_sync<kWaves>();
-  rpf_load<kThreads>(cur, plo, phi, rdep, rval, rcnt, dinv, in);
-}
-
-template <typename T, TriKind K, int kWaves, bool kFar, int kE, int kR, int kD, int kA>
-__global__ __launch_bounds__(64 * kWaves) void k_tri_chain_rpf(
-    const int* __restrict__ rdep, const T* __restrict__ rval, const int* __restrict__ rcnt,
-    const T* __restrict__ dinv, const int* __restrict__ lev_ptr,
-    const int* __restrict__ chain_lev, int rmask, const T* __restrict__ in, T* out) {
-  constexpr int kThreads = 64 * kWaves;
-  static_assert(kA >= 1 && kA < kD, "far values need their entries loaded first");
-  static_assert(kEpFarLevels >= kA + kEpFence,
-                "far dependencies must be fenced before their values are loaded");
-  extern __shared__ __align__(16) unsigned char smem_f[];
-  T* ring = reinterpret_cast<T*>(smem_f);
-  int* lvo = reinterpret_cast<int*>(ring + rmask + 1);
-  const int t = threadIdx.x;
-  const int lb = chain_lev[2 * blockIdx.x], le = chain_lev[2 * blockIdx.x + 1];
-  const int nl = le - lb;
-  // The ring starts zeroed: a skipped entry's value is then never a
-  // leftover bit pattern.
-  for (int k = t; k <= rmask; k += kThreads) ring[k] = T(0);
-  for (int k = t; k <= nl; k += kThreads) lvo[k] = lev_ptr[lb + k];
-  __syncthreads();
-  RpfPre<T, kE, kR> buf[kD];
-#pragma unroll
-  for (int d = 0; d < kD; ++d) {
-    const int Lc = min(d, nl);
-    rpf_load<kThreads>(buf[d], lvo[Lc], lvo[min(Lc + 1, nl)], rdep, rval, rcnt, dinv, in);
-  }
-  int L0 = 0;
-  for (; L0 + kD <= nl; L0 += kD) {
-#pragma unroll
-    for (int d = 0; d < kD; ++d)
-      rpf_level<T, K, kWaves, kFar, kE, kR, kD, kA>(buf[d], buf[(d + kA) % kD], L0 + d, nl, lvo,
-                                                    ring, rmask, rdep, rval, rcnt, dinv, in,
-                                                    out);
-  }
-#pragma unroll
-  for (int d = 0; d < kD; ++d)
-    if (L0 + d < nl)
-      rpf_level<T, K, kWaves, kFar, kE, kR, kD, kA>(buf[d], buf[(d + kA) % kD], L0 + d, nl, lvo,
-                                                    ring, rmask, rdep, rval, rcnt, dinv, in,
-                                                    out);
-}
-
-template <typename T, int kWaves, bool kFar, int kE, int kR>
-hipError_t tri_rpf_go(const TriLayout& L, const TriSegment& seg, const T* in, T* out,
-                      hipStream_t s) {
-  constexpr TriKind K = TriKind::kLD;
-  const size_t lds = sizeof(T) * static_cast<size_t>(L.ring) +
-                     sizeof(int) * (static_cast<size_t>(L.ep_maxlev) + 1);
-  if (lds > static_cast<size_t>(kTriBlockedMaxLds)) return hipErrorInvalidValue;
-  // prefetch 4 levels ahead; 3 with two rows per lane, 2 for two FP64 rows
-  // of 8 entries (whose registers spill otherwise); far values 2 ahead (1)
-  constexpr int kD = kR == 1 ? 4 : (sizeof(T) == 8 && kE == 8) ? 2 : 3;
-  constexpr int kA = kD > 2 ? 2 : 1;
-  auto kern = &k_tri_chain_rpf<T, K, kWaves, kFar, kE, kR, kD, kA>;
-  static bool attr = false;
-  if (!attr) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
-                                       hipFuncAttributeMaxDynamicSharedMemorySize,
-                                       static_cast<int>(kTriBlockedMaxLds));
-    if (e != hipSuccess) return e;
-    attr = true;
-  }
-  hipLaunchKernelGGL(kern, dim3(seg.nchain), dim3(64 * kWaves), static_cast<uint32_t>(lds), s,
-                     L.rpf_dep, static_cast<const T*>(L.rpf_val), L.rpf_cnt,
-                     static_cast<const T*>(L.ldiag), L.lev_ptr, seg.chain_lev, L.ring - 1, in,
-                     out);
-  return hipGetLastError();
-}
-
-template <typename T, int kWaves, int kR>
-hipError_t tri_rpf_layout(const TriLayout& L, const TriSegment& seg, const T* in, T* out,
-                          hipStream_t s) {
-  if (L.ep_far) {
-    if (L.rp_e == 4) return tri_rpf_go<T, kWaves, true, 4, kR>(L, seg, in, out, s);
-    return tri_rpf_go<T, kWaves, true, 8, kR>(L, seg, in, out, s);
-  }
-  if (L.rp_e == 4) return tri_rpf_go<T, kWaves, false, 4, kR>(L, seg, in, out, s);
-  return tri_rpf_go<T, kWaves, false, 8, kR>(L, seg, in, out, s);
-}
-
-template <typename T, int kR>
-hipError_t tri_rpf_rows(const TriLayout& L, const TriSegment& seg, const T* in, T* out,
-                        hipStream_t s) {
-  const int w = L.rp_waves;
-  if (w <= 1) return tri_rpf_layout<T, 1, kR>(L, seg, in, out, s);
-  if (w <= 2) return tri_rpf_layout<T, 2, kR>(L, seg, in, out, s);
-  if (w <= 4) return tri_rpf_layout<T, 4, kR>(L, seg, in, out, s);
-  return tri_rpf_layout<T, 8, kR>(L, seg, in, out, s);
+  for (int h = 0; h < kE * kT / 16; ++h)
+    r.val[h] = __builtin_bit_cast(
+        FpVec16<T>, __builtin_amdgcn_raw_buffer_load_b128(a.val, ln.val_off + 16 * h, ve, 0));
+  r.dinv = FpWords<T>::load(a.dinv, ln.row_off, lo * kT);
+  r.in = FpWords<T>::load(a.in, ln.row_off, lo * kT);
 }
 
 template <typename T>
-hipError_t tri_rpf_waves(const TriLayout& L, const TriSegment& seg, const T* in, T* out,
-                         hipStream_t s) {
-  // one or two rows per lane (levels of more than 512 rows)
-  if (L.rp_rows == 2) return tri_rpf_rows<T, 2>(L, seg, in, out, s);
-  return tri_rpf_rows<T, 1>(L, seg, in, out, s);
+struct FpBlock8 {
+  FpVec16<T> v[8 * sizeof(T) / 16];
+};
+template <typename T>
+__device__ __forceinline__ FpBlock8<T> rpf_get8(unsigned off) {
+  FpBlock8<T> b;
+#pragma unroll
+  for (int h = 0; h < static_cast<int>(8 * sizeof(T) / 16); ++h)
+    b.v[h] = *fp_lds<FpVec16<T>>(off + 16 * h);
+  return b;
+}
+template <typename T>
+__device__ __forceinline__ T rpf_sub8(T t, const FpBlock8<T>& b) {
+  constexpr int k = FpWords<T>::k16;
+#pragma unroll
+  for (int q = 0; q < 8; ++q) t = t - b.v[q / k][q % k];
+  return t;
 }
 
-// FP row-parallel LD solve with several lanes per row (solvers 0 and 1;
-// factors of up to kG * kE dependencies per row, no far entries): a row's
-// entries are split into kG contiguous chunks of kE, lane g holding entries
-// g kE .. g kE + kE - 1.  Every lane forms its products val * x in parallel;
-// the row's first lane then takes them in stored order (lane by lane, slot
-// by slot, through cross-lane moves) and subtracts them one at a time, as
-// the sequential solve does, so the result is the reference's bit for bit.
-// Chains, levels, LDS ring and prefetch as in k_tri_chain_rpf; waves per
-// workgroup are a launch parameter.
-template <typename T, int kG, int kE>
-struct RpgPre {
-  int lo, hi;
-  int dep[kE];
-  T val[kE];
-  T xfar[kE];  // far values (far layouts only)
-  T dinv, in;
-  int cnt;
-};
-
-// How a row's lanes combine their products: shuffled to every lane of the
-// row; staged in LDS and read back by the row's first lane; shuffled, with
-// far dependencies (dep < 0: position -dep-1, at least kEpFarLevels levels
-// back) read from `out` as in k_tri_chain_rpf.
-constexpr int kRpgShuffle = 0, kRpgStage = 1, kRpgFar = 2;
-
-template <typename T, int kG, int kE>
-__device__ __forceinline__ void rpg_load(RpgPre<T, kG, kE>& r, int lo, int hi, int threads,
-                                         const int* __restrict__ rdep, const T* __restrict__ rval,
-                                         const int* __restrict__ rcnt,
-                                         const T* __restrict__ dinv, const T* __restrict__ in) {
-  const int t = threadIdx.x;
-  const int idx = lo + t / kG;
-  const int id = idx < hi ? idx : 0;  // lanes past the level's end load position 0
-  r.lo = lo;
-  r.hi = hi;
-  const size_t base = (static_cast<size_t>(id) * kG + t % kG) * kE;
+template <typename T, bool kTail, int kMaxWaves, bool kLanes, int kE, int kD, int kA, int kFq>
+__device__ __forceinline__ void rpf_level(RpfPre<T, kE, kFq>& cur, RpfPre<T, kE, kFq>& nxt,
+                                          RpfPre<T, kE, kFq>& ahead, int L, int (&pend)[3],
+                                          const int2* lvo, const RpfArgs& a, const RpfLane& ln) {
+  constexpr int kT = sizeof(T);
+  T xv[kE];
 #pragma unroll
   for (int q = 0; q < kE; ++q) {
-    r.dep[q] = rdep[base + q];
-    r.val[q] = rval[base + q];
+    int c = static_cast<int>(cur.code[q / 4][q % 4]);
+    if (q < kFq) c = max(c, 0);
+    xv[q] = *fp_lds<T>(static_cast<unsigned>(c));
   }
-  r.cnt = rcnt[id];
-  r.dinv = dinv[id];
-  r.in = in[id];
-  (void)threads;
-}
-
-template <typename T, TriKind K, int kG, int kE, int kD, int kMode>
-__device__ __forceinline__ void rpg_level(RpgPre<T, kG, kE>& cur, RpgPre<T, kG, kE>& ahead, int L,
-                                          int nl, int threads, const int* lvo, T* ring, T* stage,
-                                          int rmask, const int* __restrict__ rdep,
-                                          const T* __restrict__ rval,
-                                          const int* __restrict__ rcnt,
-                                          const T* __restrict__ dinv,
-                                          const T* __restrict__ in, T* out) {
-  constexpr bool kFar = kMode == kRpgFar;
-  const int Lp = min(L + kD, nl);
-  const int plo = lvo[Lp], phi = lvo[min(Lp + 1, nl)];
-  const int t = threadIdx.x;
-  const int g = t % kG;
-  if constexpr (kFar) {
-    // far values of level L + kA (its entries are loaded already)
-    const bool ok = ahead.lo + t / kG < ahead.hi;
+  int plo = 0, phi = 0, pst = 0;
+  if (!kTail) {
+    plo = __builtin_amdgcn_readfirstlane(pend[0]);
+    phi = __builtin_amdgcn_readfirstlane(pend[1]);
+    pst = __builtin_amdgcn_readfirstlane(pend[2]);
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  if (!kTail) rpf_load<T, kE, kFq>(nxt, plo, phi, pst, a, ln);
+  if (kFq > 0) {
 #pragma unroll
-    for (int q = 0; q < kE; ++q) {
-      const int d = ahead.dep[q];
-      ahead.xfar[q] = out[(ok && d < 0) ? -d - 1 : 0];
+    for (int q = 0; q < kFq; ++q) {
+      // ~code is the byte offset of a far entry's value, else past the end
+      const unsigned c = ahead.code[q / 4][q % 4];
+      ahead.xfar[q] = FpWords<T>::load(a.out, static_cast<int>(~c), 0);
     }
   }
-  if constexpr (kMode == kRpgStage) {
-    // each lane forms the products of its chunk and stages them in the
-    // row's LDS slots (entry m of the row at stage[row * kG * kE + m]); the
-    // row's lanes are in one wave, whose LDS accesses stay in order, so its
-    // first lane then reads them back and subtracts them in stored order
-    T* st = stage + static_cast<size_t>(t / kG) * (kG * kE);
+  if (!kTail) {
+    const int2 p = lvo[L + kD];
+    pend[0] = p.x;
+    pend[2] = p.y;
+    pend[1] = lvo[L + kD + 1].x;
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  if (kFq > 0) {
 #pragma unroll
-    for (int q = 0; q < kE; ++q) st[g * kE + q] = cur.val[q] * ring[cur.dep[q] & rmask];
+    for (int q = 0; q < kFq; ++q) {
+      const int c = static_cast<int>(cur.code[q / 4][q % 4]);
+      if (__any(c < 0)) xv[q] = c < 0 ? cur.xfar[q] : xv[q];
+    }
+  }
+  T t = cur.in;
+  if constexpr (!kLanes) {
+#pragma unroll
+    for (int q = 0; q < kE; ++q) t = t - rpf_val<T, kE, kFq>(cur, q) * xv[q];
+  } else {
+    constexpr int k = FpWords<T>::k16;
+#pragma unroll
+    for (int h = 0; h < kE * kT / 16; ++h) {
+      FpVec16<T> p;
+#pragma unroll
+      for (int q = 0; q < k; ++q) p[q] = cur.val[h][q] * xv[h * k + q];
+      *fp_lds<FpVec16<T>>(ln.put + 16 * h) = p;
+    }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
-    const int k = cur.lo + t / kG;
-    if (k < cur.hi && g == 0) {
-      T tt = cur.in;
-#pragma unroll 16
-      for (int m = 0; m < kG * kE; ++m)
-        if (m < cur.cnt) tt = tt - st[m];
-      const T v = acc_final<T, K>(tt, cur.dinv, 0, 0);
-      ring[k & rmask] = v;
-      out[k] = v;
-    }
-  } else {
-    // no room for the staging area: the products reach every lane of the
-    // row by shuffles and each subtracts them in stored order
-    const int lane0 = (t & 63) - g;  // the row's first lane inside the wave
-    T prod[kE];
-#pragma unroll
-    for (int q = 0; q < kE; ++q) {
-      T x = ring[cur.dep[q] & rmask];
-      if constexpr (kFar) x = cur.dep[q] < 0 ? cur.xfar[q] : x;
-      prod[q] = cur.val[q] * x;
-    }
-    T tt = cur.in;
-#pragma unroll
-    for (int h = 0; h < kG; ++h)
-#pragma unroll
-      for (int q = 0; q < kE; ++q) {
-        const T v = __shfl(prod[q], lane0 + h, 64);
-        tt = h * kE + q < cur.cnt ? tt - v : tt;
-      }
-    const int k = cur.lo + t / kG;
-    if (k < cur.hi && g == 0) {
-      const T v = acc_final<T, K>(tt, cur.dinv, 0, 0);
-      ring[k & rmask] = v;
-      out[k] = v;
+    // steps is a multiple of 8; blocks read past it are not subtracted (the
+    // offsets stay inside the array: kRpfReadAhead bytes follow the last row)
+    FpBlock8<T> b0 = rpf_get8<T>(ln.get), b1 = rpf_get8<T>(ln.get + 8 * kT), b2;
+    unsigned g = ln.get + 16 * kT;
+    for (int left = cur.steps;;) {
+      b2 = rpf_get8<T>(g);
+      t = rpf_sub8(t, b0);
+      if (left <= 8) break;
+      b0 = rpf_get8<T>(g + 8 * kT);
+      t = rpf_sub8(t, b1);
+      if (left <= 16) break;
+      b1 = rpf_get8<T>(g + 16 * kT);
+      t = rpf_sub8(t, b2);
+      if (left <= 24) break;
+      left -= 24;
+      g += 24 * kT;
     }
   }
-  // far layouts: a full workgroup fence every kEpFence levels makes the
-  // values in `out` visible before any far load of them is issued
-  if (kFar && (L % kEpFence) == kEpFence - 1)
+  const T v = t * cur.dinv;
+  if (ln.owner < cur.cnt) {
+    const int lob = cur.lo * kT;
+    *fp_lds<T>(static_cast<unsigned>(lob + ln.row_off) & a.ring_mask) = v;
+    FpWords<T>::store(v, a.out, ln.row_off, lob);
+  }
+  // as in rp_level
+  if (kFq > 0 && (L & a.fence_mask) == a.fence_mask)
     __syncthreads();
   else
-    lds_barrier();
-  rpg_load<T, kG, kE>(cur, plo, phi, threads, rdep, rval, rcnt, dinv, in);
+    ep_sync<kMaxWaves>();
 }
 
-template <typename T, TriKind K, int kG, int kE, int kD, int kMode>
-__global__ __launch_bounds__(512) void k_tri_chain_rpg(
-    const int* __restrict__ rdep, const T* __restrict__ rval, const int* __restrict__ rcnt,
-    const T* __restrict__ dinv, const int* __restrict__ lev_ptr,
-    const int* __restrict__ chain_lev, int rmask, const T* __restrict__ in, T* out) {
-  constexpr bool kStage = kMode == kRpgStage;
-  constexpr int kA = kD > 2 ? 2 : 1;  // far values are loaded kA levels ahead
-  static_assert(kMode != kRpgFar || (kA < kD && kEpFarLevels >= kA + kEpFence),
-                "far values need their entries loaded and their writes fenced first");
-  extern __shared__ __align__(16) unsigned char smem_g[];
-  T* ring = reinterpret_cast<T*>(smem_g);
-  T* stage = ring + rmask + 1;  // kE products per thread (staged variant)
-  const int threads = static_cast<int>(blockDim.x);
-  int* lvo = reinterpret_cast<int*>(stage + (kStage ? static_cast<size_t>(threads) * kE : 0));
+template <typename T, int kFirst, int kMaxWaves, bool kLanes, int kE, int kD, int kA, int kFq>
+__device__ __forceinline__ void rpf_tail(RpfPre<T, kE, kFq> (&buf)[kD], int L0, int nl,
+                                         int (&pend)[3], const int2* lvo, const RpfArgs& a,
+                                         const RpfLane& ln) {
+  if constexpr (kFirst < kD - 1) {
+    if (L0 + kFirst < nl) {
+      rpf_level<T, true, kMaxWaves, kLanes, kE, kD, kA, kFq>(
+          buf[kFirst], buf[(kFirst + kD - 1) % kD], buf[(kFirst + kA) % kD], L0 + kFirst, pend,
+          lvo, a, ln);
+      rpf_tail<T, kFirst + 1, kMaxWaves, kLanes, kE, kD, kA, kFq>(buf, L0, nl, pend, lvo, a, ln);
+    }
+  }
+}
+
+// LDS: the ring, 16 bytes of zeros, the rows' products (kLanes), then the
+// chain's {first position, steps} per piece (as in k_tri_chain_rp).
+template <typename T, int kMaxWaves, bool kLanes, int kE, int kD, int kA, int kFq>
+__global__ __launch_bounds__(64 * kMaxWaves) void k_tri_chain_rpf(
+    const int* __restrict__ code, const T* __restrict__ val, const T* __restrict__ dinv,
+    const int* __restrict__ lev_ptr, const int* __restrict__ lev_steps,
+    const int* __restrict__ chain_lev, int n, int ring_bytes, int lg, int fence,
+    const T* __restrict__ in, T* out) {
+  constexpr int kT = sizeof(T);
+  static_assert(kFq == 0 || (kA >= 1 && kA < kD - 1), "far values need their entries first");
+  static_assert(kA <= kRpMaxAhead, "the plan's fence period allows for kRpMaxAhead");
+  static_assert(kD + 1 <= kRpPadLevels, "level offsets are read kD + 1 past the end");
+  extern __shared__ __align__(16) unsigned char smem_f[];
   const int t = threadIdx.x;
+  const int threads = kMaxWaves == 1 ? 64 : static_cast<int>(blockDim.x);
+  const int lanes = 1 << lg;
+  const int row_bytes = lanes * kE * kT + 16;  // rows on different banks
+  const int stage = ring_bytes + 16;
+  const int stage_bytes = kLanes ? (threads >> lg) * row_bytes + kRpfReadAhead : 0;
+  int2* lvo = reinterpret_cast<int2*>(smem_f + stage + stage_bytes);
   const int lb = chain_lev[2 * blockIdx.x], le = chain_lev[2 * blockIdx.x + 1];
   const int nl = le - lb;
-  // the ring starts zeroed: a skipped entry's slot never holds a leftover
-  // bit pattern (its product is formed but not subtracted)
-  for (int k = t; k <= rmask; k += threads) ring[k] = T(0);
-  for (int k = t; k <= nl; k += threads) lvo[k] = lev_ptr[lb + k];
+  // a slot that nothing has been written to yet holds no leftover bits
+  for (int k = 4 * t; k < stage; k += 4 * threads) *fp_lds<int>(k) = 0;
+  for (int k = t; k <= nl + kD + 1; k += threads)
+    lvo[k] = make_int2(lev_ptr[lb + min(k, nl)], k < nl ? lev_steps[lb + k] : 8);
   __syncthreads();
-  RpgPre<T, kG, kE> buf[kD];
+  const unsigned nb = static_cast<unsigned>(n) * kT;
+  const unsigned slots = (static_cast<unsigned>(n) << lg) * kE;
+  const RpfArgs a{rp_buffer(code, slots * 4), rp_buffer(val, slots * kT), rp_buffer(dinv, nb),
+                  rp_buffer(in, nb), rp_buffer(out, nb), static_cast<unsigned>(ring_bytes) - 1u,
+                  lg, fence - 1};
+  const int row = t >> lg, lane = t & (lanes - 1);
+  RpfLane ln;
+  ln.code_off = t * (kE * 4);
+  ln.val_off = t * (kE * kT);
+  ln.row_off = row * kT;
+  ln.owner = lane == 0 ? row : INT32_MAX;
+  ln.get = static_cast<unsigned>(stage + row * row_bytes);
+  ln.put = ln.get + static_cast<unsigned>(lane * kE * kT);
+  RpfPre<T, kE, kFq> buf[kD];
 #pragma unroll
-  for (int d = 0; d < kD; ++d) {
-    const int Lc = min(d, nl);
-    rpg_load<T, kG, kE>(buf[d], lvo[Lc], lvo[min(Lc + 1, nl)], threads, rdep, rval, rcnt, dinv,
-                        in);
-  }
+  for (int d = 0; d < kD - 1; ++d)
+    rpf_load<T, kE, kFq>(buf[d], __builtin_amdgcn_readfirstlane(lvo[d].x),
+                         __builtin_amdgcn_readfirstlane(lvo[d + 1].x),
+                         __builtin_amdgcn_readfirstlane(lvo[d].y), a, ln);
+  int pend[3] = {lvo[kD - 1].x, lvo[kD].x, lvo[kD - 1].y};
   int L0 = 0;
   for (; L0 + kD <= nl; L0 += kD) {
 #pragma unroll
     for (int d = 0; d < kD; ++d)
-      rpg_level<T, K, kG, kE, kD, kMode>(buf[d], buf[(d + kA) % kD], L0 + d, nl, threads, lvo,
-                                         ring, stage, rmask, rdep, rval, rcnt, dinv, in, out);
+      rpf_level<T, false, kMaxWaves, kLanes, kE, kD, kA, kFq>(
+          buf[d], buf[(d + kD - 1) % kD], buf[(d + kA) % kD], L0 + d, pend, lvo, a, ln);
   }
-#pragma unroll
-  for (int d = 0; d < kD; ++d)
-    if (L0 + d < nl)
-      rpg_level<T, K, kG, kE, kD, kMode>(buf[d], buf[(d + kA) % kD], L0 + d, nl, threads, lvo,
-                                         ring, stage, rmask, rdep, rval, rcnt, dinv, in, out);
+  rpf_tail<T, 0, kMaxWaves, kLanes, kE, kD, kA, kFq>(buf, L0, nl, pend, lvo, a, ln);
 }
 
-template <typename T, int kG, int kE, int kMode>
-hipError_t tri_rpg_go(const TriLayout& L, const TriSegment& seg, const T* in, T* out,
-                      hipStream_t s) {
-  constexpr TriKind K = TriKind::kLD;
-  constexpr bool kStage = kMode == kRpgStage;
-  const size_t lds = rpg_lds_bytes(sizeof(T), L.ring, L.rp_waves, kE, L.ep_maxlev, kStage);
-  if (lds > static_cast<size_t>(kTriBlockedMaxLds) || L.rp_waves < 1 || L.rp_waves > 8)
+template <typename T, int kMaxWaves, bool kLanes, int kE, int kD, int kA, int kFq>
+hipError_t tri_rpf_go(const TriLayout& L, const T* in, T* out, hipStream_t s) {
+  const size_t lds = rpf_lds_bytes(sizeof(T), L.rp_ring, L.rp_waves, L.rp_lanes, kE, L.rp_maxlev);
+  int lg = 0;
+  while ((1 << lg) < L.rp_lanes) ++lg;
+  if (lds > static_cast<size_t>(kTriBlockedMaxLds) || L.n <= 0 || L.rp_fence < 1 ||
+      (1 << lg) != L.rp_lanes || (L.rp_lanes > 1) != kLanes ||
+      static_cast<uint64_t>(L.n) * L.rp_lanes * kE * sizeof(T) > UINT32_MAX)
     return hipErrorInvalidValue;
-  // prefetch 4 levels ahead; fewer where the registers spill otherwise:
-  // 3 for staged FP64 rows of 8-entry chunks, 2 for 16-entry chunks
-  constexpr int kD = kE == 16 ? 2 : (kStage && sizeof(T) == 8 && kE == 8) ? 3 : 4;
-  auto kern = &k_tri_chain_rpg<T, K, kG, kE, kD, kMode>;
+  auto kern = &k_tri_chain_rpf<T, kMaxWaves, kLanes, kE, kD, kA, kFq>;
   static bool attr = false;
   if (!attr) {
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
@@ -2135,54 +2050,41 @@ hipError_t tri_rpg_go(const TriLayout& L, const TriSegment& seg, const T* in, T*
     if (e != hipSuccess) return e;
     attr = true;
   }
-  hipLaunchKernelGGL(kern, dim3(seg.nchain), dim3(64 * L.rp_waves), static_cast<uint32_t>(lds),
-                     s, L.rpf_dep, static_cast<const T*>(L.rpf_val), L.rpf_cnt,
-                     static_cast<const T*>(L.ldiag), L.lev_ptr, seg.chain_lev, L.ring - 1, in,
-                     out);
+  hipLaunchKernelGGL(kern, dim3(L.rp_nchain), dim3(64 * L.rp_waves), static_cast<uint32_t>(lds),
+                     s, L.rpf_dep, static_cast<const T*>(L.rpf_val),
+                     static_cast<const T*>(L.ldiag), L.rp_lev, L.rp_steps, L.rp_chain, L.n,
+                     L.rp_ring * static_cast<int>(sizeof(T)), lg, L.rp_fence, in, out);
   return hipGetLastError();
 }
 
-template <typename T>
-hipError_t tri_rpg(const TriLayout& L, const TriSegment& seg, const T* in, T* out,
-                   hipStream_t s) {
-  auto lanes = [&](auto e_tag) -> hipError_t {
-    constexpr int E = decltype(e_tag)::value;
-    // the layout builder makes: staged products for FP64 rows over 16
-    // lanes only, far dependencies for rows over 2 or 4 lanes only, no
-    // shuffled FP64 rows of 16 chunks of 8 (whose registers spill), and
-    // chunks of 16 for FP32 rows over at most 8 lanes only
-    if constexpr (sizeof(T) == 8 && E == 16) return hipErrorInvalidValue;
-    else {
-      if (L.rp_stage && L.ep_far) return hipErrorInvalidValue;
-      if constexpr (sizeof(T) == 8) {
-        if (L.rp_stage)
-          return L.rp_lanes == 16 ? tri_rpg_go<T, 16, E, kRpgStage>(L, seg, in, out, s)
-                                  : hipErrorInvalidValue;
-      } else {
-        if (L.rp_stage) return hipErrorInvalidValue;
-      }
-      if (L.ep_far) {
-        switch (L.rp_lanes) {
-          case 2: return tri_rpg_go<T, 2, E, kRpgFar>(L, seg, in, out, s);
-          case 4: return tri_rpg_go<T, 4, E, kRpgFar>(L, seg, in, out, s);
-          default: return hipErrorInvalidValue;
-        }
-      }
-      switch (L.rp_lanes) {
-        case 2: return tri_rpg_go<T, 2, E, kRpgShuffle>(L, seg, in, out, s);
-        case 4: return tri_rpg_go<T, 4, E, kRpgShuffle>(L, seg, in, out, s);
-        case 8: return tri_rpg_go<T, 8, E, kRpgShuffle>(L, seg, in, out, s);
-        case 16:
-          if constexpr ((sizeof(T) == 8 && E == 8) || E == 16) return hipErrorInvalidValue;
-          else return tri_rpg_go<T, 16, E, kRpgShuffle>(L, seg, in, out, s);
-        default: return hipErrorInvalidValue;
-      }
+// Prefetch distances as far as 256 registers allow.  Far values: the leading
+// slots that can hold one with one lane per row (the 7-point factor's only
+// far entry is its first), else every slot.
+template <typename T, int kMaxWaves, bool kLanes>
+hipError_t tri_rpf_layout(const TriLayout& L, const T* in, T* out, hipStream_t s) {
+  constexpr bool kD64 = sizeof(T) == 8;
+  if (L.rp_e == 4) {
+    if (L.rp_farq == 0) return tri_rpf_go<T, kMaxWaves, kLanes, 4, kD64 ? 8 : 10, 1, 0>(L, in, out, s);
+    if constexpr (!kLanes) {
+      if (L.rp_farq == 1) return tri_rpf_go<T, kMaxWaves, kLanes, 4, 8, 3, 1>(L, in, out, s);
     }
-  };
-  if (L.rp_e == 4) return lanes(std::integral_constant<int, 4>{});
-  if (L.rp_e == 8) return lanes(std::integral_constant<int, 8>{});
-  if (L.rp_e == 16) return lanes(std::integral_constant<int, 16>{});
+    return tri_rpf_go<T, kMaxWaves, kLanes, 4, kD64 ? 6 : 8, 2, 4>(L, in, out, s);
+  }
+  if (L.rp_e == 8) {
+    if (L.rp_farq == 0) return tri_rpf_go<T, kMaxWaves, kLanes, 8, kD64 ? 5 : 8, 1, 0>(L, in, out, s);
+    return tri_rpf_go<T, kMaxWaves, kLanes, 8, kD64 ? 4 : 6, 2, 8>(L, in, out, s);
+  }
   return hipErrorInvalidValue;
+}
+
+template <typename T>
+hipError_t tri_rpf(const TriLayout& L, const T* in, T* out, hipStream_t s) {
+  if (L.rp_waves < 1 || L.rp_waves > 8) return hipErrorInvalidValue;
+  if (L.rp_lanes > 1)
+    return L.rp_waves == 1 ? tri_rpf_layout<T, 1, true>(L, in, out, s)
+                           : tri_rpf_layout<T, 8, true>(L, in, out, s);
+  return L.rp_waves == 1 ? tri_rpf_layout<T, 1, false>(L, in, out, s)
+                         : tri_rpf_layout<T, 8, false>(L, in, out, s);
 }
 
 // One level, many workgroups, level-ordered layout.
@@ -2493,22 +2395,12 @@ hipError_t launch_trsv_rp_blk(const TriLayout& L, int groups, int bit, int dbit,
                           static_cast<int32_t*>(out), s);
 }
 
-hipError_t launch_trsv_rpf(Elem e, const TriLayout& L, const TriSegment& seg, const void* in,
-                           void* out, hipStream_t s) {
-  if (L.rp_lanes > 1) {
-    if (e == Elem::kF64)
-      return tri_rpg<double>(L, seg, static_cast<const double*>(in), static_cast<double*>(out),
-                             s);
-    if (e == Elem::kF32)
-      return tri_rpg<float>(L, seg, static_cast<const float*>(in), static_cast<float*>(out), s);
-    return hipErrorInvalidValue;
-  }
+hipError_t launch_trsv_rpf(Elem e, const TriLayout& L, const void* in, void* out,
+                           hipStream_t s) {
   if (e == Elem::kF64)
-    return tri_rpf_waves<double>(L, seg, static_cast<const double*>(in),
-                                 static_cast<double*>(out), s);
+    return tri_rpf<double>(L, static_cast<const double*>(in), static_cast<double*>(out), s);
   if (e == Elem::kF32)
-    return tri_rpf_waves<float>(L, seg, static_cast<const float*>(in), static_cast<float*>(out),
-                                s);
+    return tri_rpf<float>(L, static_cast<const float*>(in), static_cast<float*>(out), s);
   return hipErrorInvalidValue;
 }
 

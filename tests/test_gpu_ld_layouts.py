@@ -1,5 +1,5 @@
-"""The row-parallel integer LD solve (k_tri_chain_rp) in the layouts that the
-plan picks at the ends of its range: one wave and 9-16 waves, 1-64 lanes per
+"""The row-parallel LD solves (k_tri_chain_rp, k_tri_chain_rpf) in the layouts
+that the plan picks at the ends of its range: one wave and 9-16 waves, 1-64 lanes per
 row, levels cut into pieces, a single chain with levels of more than 1,024
 rows, odd sizes.  Every LD solve equals the oracle's bit for bit (whole
 numbers: no tolerance)."""
@@ -22,11 +22,11 @@ LAYOUT = re.compile(r"\[sc23ad plan\] kind 0 n (\d+) .*rp waves (\d+) entries (\
 
 
 
-def _check(a, smoother, monkeypatch, capfd):
+def _check(a, smoother, monkeypatch, capfd, prec=S.INT):
     """LD solves of every level against the oracle; the layouts picked."""
     monkeypatch.setenv("SC23AD_VERBOSE", "1")
     a.lmax1_scaling(np.zeros(a.n))
-    h = S.Hierarchy(a, S.INT, S.amg_param(smoother))
+    h = S.Hierarchy(a, prec, S.amg_param(smoother))
     capfd.readouterr()
     amg = S.Amg(h)
     plans = [tuple(map(int, m.groups())) for m in LAYOUT.finditer(capfd.readouterr().err)]
@@ -39,9 +39,14 @@ def _check(a, smoother, monkeypatch, capfd):
     rng = np.random.default_rng(7)
     for lv in range(amg.depth):
         n = oh.level_n(lv)
-        x = rng.integers(-2**29, 2**29, n).astype(np.int32)
-        assert np.array_equal(amg.level_op(lv, S.OP_TRSV_LD, x, n),
-                              oh.level_op(lv, S.OP_TRSV_LD, x, n)), lv
+        if prec == S.INT:
+            x = rng.integers(-2**29, 2**29, n).astype(np.int32)
+        else:  # signed zeros and subnormals among them: compared bit for bit
+            x = rng.standard_normal(n).astype(np.float64 if prec == S.FP64 else np.float32)
+            x[::7] = -0.0
+            x[3::11] = 1e-310 if prec == S.FP64 else 1e-40
+        y, yo = amg.level_op(lv, S.OP_TRSV_LD, x, n), oh.level_op(lv, S.OP_TRSV_LD, x, n)
+        assert y.tobytes() == yo.tobytes(), lv
     return plans
 
 
@@ -69,3 +74,25 @@ def test_sixteen_waves(monkeypatch, capfd):
     monkeypatch.setenv("SC23AD_RP_WAVES", "16")
     plans = _check(S.CsrMat.generate(S.GEN_POISSON2D, 67), S.SOR, monkeypatch, capfd)
     assert any(p[1] == 16 for p in plans)
+
+
+@pytest.mark.parametrize("prec", [S.FP64, S.FP32], ids=["fp64", "fp32"])
+@pytest.mark.parametrize("lanes", [1, 2, 4, 8, 16, 32, 64])
+@pytest.mark.parametrize("waves", [1, 3, 8])
+def test_forced_fp_layouts(lanes, waves, prec, monkeypatch, capfd):
+    """One lane per row on the 2D factor (2-4 entries per row), several on the
+    27-point one (up to 13 and more), whose pieces subtract 8 to 64 products."""
+    monkeypatch.setenv("SC23AD_RP_LANES", str(lanes))
+    monkeypatch.setenv("SC23AD_RP_WAVES", str(waves))
+    a = (S.CsrMat.generate(S.GEN_POISSON2D, 67) if lanes == 1 else
+         S.CsrMat.generate(S.GEN_DIFFUSION27, 17, 5, 1.0, 1.0, 1e-3, 3))
+    plans = _check(a, S.SOR, monkeypatch, capfd, prec)
+    assert any(p[1] == waves and p[3] == lanes for p in plans)
+
+
+@pytest.mark.parametrize("prec", [S.FP64, S.FP32], ids=["fp64", "fp32"])
+@pytest.mark.parametrize("smoother", [S.SOR, S.BLOCK_SOR], ids=["sor", "block"])
+def test_fp_far_dependencies_small_ring(smoother, prec, monkeypatch, capfd):
+    monkeypatch.setenv("SC23AD_FP_RING_FAR", "1")
+    _check(S.CsrMat.generate(S.GEN_DIFFUSION27, 29, 5, 1.0, 1.0, 1e-3, 3), smoother, monkeypatch,
+           capfd, prec)
