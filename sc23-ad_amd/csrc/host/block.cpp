@@ -148,11 +148,13 @@ void DevAmg::vcycle_lo_blk(const void* in, void* out, BlockWork& w) const {
 }
 
 void DevAmg::check_errors(BlockWork& w) const {
-  hip_check(hipMemcpyAsync(w.host_err.get(), w.err.get(), sizeof(int), hipMemcpyDeviceToHost,
+  int word = 0;
+  const int* e = w.host_err.get() ? w.host_err.get() : &word;
+  hip_check(hipMemcpyAsync(const_cast<int*>(e), w.err.get(), sizeof(int), hipMemcpyDeviceToHost,
                            lib_stream()),
             "error flag");
   hip_check(hipStreamSynchronize(lib_stream()), "sync");
-  if (*w.host_err.get() != 0) {
+  if (*e != 0) {
     hip_check(dev::launch_fill_zero(sizeof(int), w.err.get(), lib_stream()), "error reset");
     hip_check(hipStreamSynchronize(lib_stream()), "sync");
     throw DevError{5, "coarse solve: a block waited too long for its dependencies"};
@@ -164,7 +166,9 @@ std::unique_ptr<DevAmg::BlockWork> DevAmg::take_block_work(int groups) {
     std::lock_guard<std::mutex> lock(idle_mutex_);
     if (idle_ && idle_->groups == groups) return std::move(idle_);
   }
-  return make_block_work(groups);
+  auto w = make_block_work(groups);
+  w->host_err.alloc();
+  return w;
 }
 
 void DevAmg::give_block_work(std::unique_ptr<BlockWork> w) {

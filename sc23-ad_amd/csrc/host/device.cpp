@@ -68,7 +68,8 @@ void DevBuf::download(void* dst, size_t bytes, size_t off) const {
   hip_check(hipStreamSynchronize(lib_stream()), "download sync");
 }
 
-PinnedInt::PinnedInt() {
+void PinnedInt::alloc() {
+  if (p_) return;
   lib_stream();
   hip_check(hipHostMalloc(reinterpret_cast<void**>(&p_), sizeof(int), hipHostMallocDefault),
             "hipHostMalloc");
@@ -1178,8 +1179,8 @@ void tune_spmv(DevMat& m, Elem e, SpmvMode mode) {
   dev::DCsr csr = m.d;
   csr.soff = nullptr;
   csr.srow = nullptr;
+  const double avg = static_cast<double>(m.d.nnz) / m.d.n;
   if (e == Elem::kI32) {
-    const double avg = static_cast<double>(m.d.nnz) / m.d.n;
     for (int g = 1; g <= 64; g *= 2) {
       if (g > 2 * avg + 2) break;
       csr.group = g;
@@ -1194,6 +1195,12 @@ void tune_spmv(DevMat& m, Elem e, SpmvMode mode) {
       }
   } else {
     cands.push_back(csr);
+    for (int r = 8; r <= 128; r *= 2)
+      if (r * avg >= 512 && r * avg <= 8192) {
+        dev::DCsr st = csr;
+        st.stream = r;
+        cands.push_back(st);
+      }
   }
   if (m.d.soff) cands.push_back(m.d);
   if (m.d.soff && m.scol16.get()) {
@@ -1345,6 +1352,7 @@ std::unique_ptr<DevAmg> DevAmg::upload(const IntHierarchy& h, const LaunchCfg& c
     build_tiles(a->uc_plan, TriKind::kDU, h.uc.n, h.uc.rptr, h.uc.cind, h.uc.val);
   }
   a->work_ = a->make_work();
+  a->work_->host_err.alloc();
   a->tune();
   return a;
 }
@@ -1379,6 +1387,7 @@ std::unique_ptr<DevAmg> DevAmg::upload_fp(const FpHierarchy<T>& h, const LaunchC
     build_tiles_fp(a->uc_plan, TriKind::kDU, h.uc.n, h.uc.rptr, h.uc.cind, h.uc.val);
   }
   a->work_ = a->make_work();
+  a->work_->host_err.alloc();
   a->tune();
   return a;
 }
@@ -1478,12 +1487,14 @@ void DevAmg::smooth(int l, const void* in, void* out, bool inited, Work& w) cons
 
 void DevAmg::check_errors(Work& w) const {
   const bool waits = lc_plan.dense || uc_plan.dense || lc_plan.dense_fp || uc_plan.dense_fp;
+  int word = 0;
+  const int* e = w.host_err.get() ? w.host_err.get() : &word;
   if (waits)
-    hip_check(hipMemcpyAsync(w.host_err.get(), w.err.get(), sizeof(int), hipMemcpyDeviceToHost,
+    hip_check(hipMemcpyAsync(const_cast<int*>(e), w.err.get(), sizeof(int), hipMemcpyDeviceToHost,
                              lib_stream()),
               "error flag");
   hip_check(hipStreamSynchronize(lib_stream()), "sync");
-  if (waits && *w.host_err.get() != 0) {
+  if (waits && *e != 0) {
     // clear the word so that later calls on this work context start clean
     hip_check(dev::launch_fill_zero(sizeof(int), w.err.get(), lib_stream()), "error flag reset");
     hip_check(hipStreamSynchronize(lib_stream()), "sync");

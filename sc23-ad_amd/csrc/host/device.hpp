@@ -74,10 +74,13 @@ class DevBuf {
   size_t bytes_ = 0;
 };
 
-// One int of pinned host memory (device-to-host copies of an error word).
+// One int of pinned host memory (device-to-host copies of an error word),
+// none until alloc(): allocating it takes longer than a pageable copy, so only
+// work contexts that serve many short calls have one.
 class PinnedInt {
  public:
-  PinnedInt();
+  PinnedInt() = default;
+  void alloc();
   ~PinnedInt();
   PinnedInt(const PinnedInt&) = delete;
   PinnedInt& operator=(const PinnedInt&) = delete;
@@ -192,7 +195,7 @@ class DevAmg {
     DevBuf r0, tmpc, vin0, vout0;         // fine residual, coarse temp, level-0 order in/out
     DevBuf lflags, uflags, err;           // tiled coarse solves: {epoch, value} words, errors
     DevBuf tickets;                       // tiled coarse solves: L counters [0,1], U [2,3]
-    PinnedInt host_err;                   // where check_errors reads the error word
+    PinnedInt host_err;                   // where check_errors reads the error word, if pinned
     int lepoch = 0, uepoch = 0;           // last flag values raised
     EventTimer* trsv_timer = nullptr;     // times the level-0 LD solves (owner's hook)
   };

@@ -25,8 +25,8 @@ struct DCsr {
   const int* cind = nullptr;
   const void* val = nullptr;
   int group = 8;  // lanes per row for the integer SpMV (power of two <= 64)
-  // integer CSR: rows per workgroup of the LDS-streamed kernel (16, 32, 64,
-  // 128 or 256), 0: `group` lanes per row
+  // CSR: rows per workgroup of the LDS-streamed kernel (integers 16 to 256, FP
+  // 8 to 128, powers of two), 0: `group` lanes per row
   int stream = 0;
   // SELL-64 copy (rows with near-uniform lengths): slices of 64 rows, entry k
   // of row r of slice s at soff[s] + 64 k + r, padded with column -1 / value 0.

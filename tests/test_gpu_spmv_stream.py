@@ -1,7 +1,7 @@
-"""The integer CSR product streamed through LDS (k_spmv_stream_int): every row
+"""The CSR products streamed through LDS (k_spmv_stream_int, _fp): every row
 count per workgroup, rows shorter and longer than a tile of 2,048 entries,
 empty rows and workgroups without entries, sizes off the workgroup's.  Whole
-numbers: no tolerance."""
+numbers, or FP sums in stored order: no tolerance."""
 from __future__ import annotations
 
 import os
@@ -39,20 +39,34 @@ def test_rows_per_workgroup(n):
                               _reference(rptr, cind, val, bit, x)), bit
 
 
-def test_fused_modes_on_a_hierarchy(monkeypatch):
+@pytest.mark.parametrize("prec", [S.INT, S.FP64, S.FP32], ids=["int", "fp64", "fp32"])
+def test_fused_modes_on_a_hierarchy(prec, monkeypatch):
     """Forced on every matrix that has a streamed candidate: each level's
-    products and one V-cycle, whose residuals and corrections are fused."""
+    products and one V-cycle, whose residuals and corrections are fused.  FP
+    rows are added in stored order: the same bits, signed zeros included."""
     monkeypatch.setenv("SC23AD_SPMV_FORMAT", "stream")
     sy = S.make_system(S.GEN_INCLUSIONS3D, (24, 8, 2.0, 4.0, 1e4, 3), 5)
-    h = S.Hierarchy(sy.a, S.INT, S.amg_param(S.BLOCK_SOR))
+    h = S.Hierarchy(sy.a, prec, S.amg_param(S.BLOCK_SOR))
     path = export(h)
     amg, oh = S.Amg(h), O.OracleHier(path)
     os.unlink(path)
     rng = np.random.default_rng(31)
+
+    def vector(n):
+        if prec == S.INT:
+            return rng.integers(-2**20, 2**20, n).astype(np.int32)
+        v = rng.standard_normal(n).astype(np.float64 if prec == S.FP64 else np.float32)
+        v[::3] = -0.0
+        return v
+
     for lv in range(amg.depth):
-        n = oh.level_n(lv)
-        x = rng.integers(-2**29, 2**29, n).astype(np.int32)
+        n, nxt = oh.level_n(lv), oh.level_n(lv + 1)
+        x, xc = vector(n), vector(nxt)
         for op in (S.OP_SPMV_A, S.OP_SPMV_U):
-            assert np.array_equal(amg.level_op(lv, op, x, n), oh.level_op(lv, op, x, n)), lv
-    v = rng.integers(-2**20, 2**20, sy.a.n).astype(np.int32)
-    assert np.array_equal(amg.precondition(v), oh.vcycle(v))
+            assert amg.level_op(lv, op, x, n).tobytes() == oh.level_op(lv, op, x, n).tobytes(), lv
+        assert (amg.level_op(lv, S.OP_SPMV_R, x, nxt).tobytes()
+                == oh.level_op(lv, S.OP_SPMV_R, x, nxt).tobytes()), lv
+        assert (amg.level_op(lv, S.OP_SPMV_P, xc, n).tobytes()
+                == oh.level_op(lv, S.OP_SPMV_P, xc, n).tobytes()), lv
+    v = vector(sy.a.n)
+    assert amg.precondition(v).tobytes() == oh.vcycle(v).tobytes()
