@@ -955,8 +955,7 @@ bool build_blocked(TriPlan& plan, TriKind kind, int n, const std::vector<int>& r
   return true;
 }
 
-// Dense 64-wide column-block slices of an integer triangular factor.
-// Tiles of an integer coarse factor for the one-workgroup-per-block solve:
+// Tiles of an integer coarse factor for the tiled solve (values negated):
 // for block b, the 64 x 64 tiles of the blocks it depends on in processing
 // order, then its diagonal tile; column-major inside a tile.
 void build_tiles(TriPlan& plan, TriKind kind, int n, const std::vector<int>& rptr,
@@ -970,6 +969,8 @@ void build_tiles(TriPlan& plan, TriKind kind, int n, const std::vector<int>& rpt
   for (int i = 0; i < n; ++i)
     for (int p = rptr[i] + 1; p < rptr[i + 1]; ++p)
       if (cind[p] <= cind[p - 1]) return;
+  for (int32_t v : val)  // the tiles hold negated values
+    if (v == INT32_MIN) return;
   const bool fwd = kind != TriKind::kDU;
   std::vector<long long> toff(nb + 1, 0);
   for (int b = 0; b < nb; ++b) toff[b + 1] = toff[b] + static_cast<long long>(fwd ? b + 1 : nb - b) * W * W;
@@ -993,7 +994,7 @@ void build_tiles(TriPlan& plan, TriKind kind, int n, const std::vector<int>& rpt
         throw DevError{1, "coarse factor entry on the wrong side of the diagonal"};
       const int slot = fwd ? bc : nb - 1 - bc;  // tile position in processing order
       tl[static_cast<size_t>(toff[b]) + static_cast<size_t>(slot) * W * W +
-         static_cast<size_t>(c - bc * W) * W + (i - b * W)] = val[p];
+         static_cast<size_t>(c - bc * W) * W + (i - b * W)] = -val[p];
     }
   }
   plan.slice.alloc(sizeof(int32_t) * tl.size());
@@ -1314,7 +1315,9 @@ std::unique_ptr<DevAmg::Work> DevAmg::make_work() const {
   w->tmp[0].alloc(es * n0s);
   w->tmpc.alloc(es * std::max(n_coarse, 1));
   // published-value words of the tiled coarse solves: epoch 0 = never written
-  std::vector<unsigned long long> zero(static_cast<size_t>(std::max(n_coarse, 1)), 0);
+  // (FP64 values take two words)
+  std::vector<unsigned long long> zero(
+      static_cast<size_t>(std::max(n_coarse, 1)) * (elem == Elem::kF64 ? 2 : 1), 0);
   for (DevBuf* f : {&w->lflags, &w->uflags}) {
     f->alloc(sizeof(unsigned long long) * zero.size());
     f->upload(zero.data(), sizeof(unsigned long long) * zero.size());
@@ -1411,22 +1414,13 @@ bool DevAmg::trsv_timing_aware(const TriPlan& plan) const {
 
 void DevAmg::trsv(const TriPlan& plan, const DevMat& m, const void* in, void* out,
                   unsigned long long* flags, int* epoch, int* err, unsigned* tickets) const {
-  if (plan.dense && elem == Elem::kI32 && flags) {
+  if ((elem == Elem::kI32 ? plan.dense : plan.dense_fp) && flags) {
     *epoch = *epoch == INT32_MAX ? 1 : *epoch + 1;
-    hip_check(dev::launch_trsv_tiles(plan.kind, m.d.n, plan.nb, plan.slice.as<int32_t>(),
-                                     plan.boff.as<long long>(), plan.ddinv.as<int32_t>(),
-                                     m.d.bit, m.d.dbit, in, out, flags, *epoch, err, tickets,
-                                     lib_stream()),
+    hip_check(dev::launch_trsv_tiles(elem, plan.kind, m.d.n, plan.nb, plan.slice.get(),
+                                     plan.boff.as<long long>(), plan.tmask.as<uint64_t>(),
+                                     plan.ddinv.get(), m.d.bit, m.d.dbit, in, out, flags, *epoch,
+                                     err, tickets, lib_stream()),
               "trsv tiles");
-    return;
-  }
-  if (plan.dense_fp && elem != Elem::kI32 && flags) {
-    *epoch = *epoch == INT32_MAX ? 1 : *epoch + 1;
-    hip_check(dev::launch_trsv_tiles_fp(elem, plan.kind, m.d.n, plan.nb, plan.slice.get(),
-                                        plan.boff.as<long long>(), plan.tmask.as<uint64_t>(),
-                                        plan.ddinv.get(), in, out, flags, *epoch, err, tickets,
-                                        lib_stream()),
-              "trsv tiles fp");
     return;
   }
   if (plan.blocked) {

@@ -169,125 +169,6 @@ __global__ __launch_bounds__(kBk) void k_spmv_blk_sell(int n, int m,
   }
 }
 
-// ---- tiled coarse solve, four right-hand sides per workgroup --------------
-// k_tri_tiles_int (the single-vector kernel) for a group of four right-hand
-// sides: workgroup (block b, group g) owns rows 64b .. 64b+63 of group g;
-// the four waves share the dependency products, then wave q sweeps the
-// diagonal tile for right-hand side q.  A
-// solved row publishes one {epoch, value} word per right-hand side
-// (xp[((g * n) + row) * 4 + c]); a consumer polls the 4 x 64 words of a
-// dependency block until all carry the current epoch.  Workgroups take
-// their (block, group) from a ticket counter, in processing order, so a
-// workgroup only waits for tickets handed out before its own, whatever
-// order the hardware starts workgroups in; the last workgroup to finish
-// resets the counters for the next launch.  A launch out of its wait budget
-// (tile_wait_over) records an error and gives up instead of hanging.
-template <TriKind K>
-__global__ __launch_bounds__(kTileThreads) void k_tri_tiles_blk(
-    int n, int nb, int groups, const int32_t* __restrict__ tiles,
-    const long long* __restrict__ toff, const int32_t* __restrict__ dinv_g, int bit, int dbit,
-    const int4* __restrict__ in_all, int4* out_all, unsigned long long* xp_all, int epoch,
-    int* err, unsigned* tickets) {
-  static_assert(kTileThreads == 256, "one wave per right-hand side of a group of four");
-  constexpr bool fwd = (K != TriKind::kDU);
-  __shared__ uint64_t part[kTileThreads / 64][4][64];
-  __shared__ int32_t xsh[4][64];
-  __shared__ int ticket_sh;
-  const long long t0 = wall_clock64();
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const int ticket = tile_ticket(tickets, &ticket_sh);
-  // tickets in processing order (forward: blocks 0, 1, ...; backward: nb-1,
-  // nb-2, ...), block-major, so every block's dependency blocks (all
-  // groups) hold smaller tickets
-  const int pb = ticket / groups, g = ticket % groups;
-  const int b = fwd ? pb : nb - 1 - pb;
-  const size_t goff = static_cast<size_t>(g) * n;
-  const int4* in = in_all + goff;
-  int4* out = out_all + goff;
-  unsigned long long* xp = xp_all + goff * 4;
-  const int r0 = b * kTB;
-  const int rows = min(kTB, n - r0);
-  const int32_t* T = tiles + toff[b];
-  const int ndep = fwd ? b : nb - 1 - b;
-  // wave w owns right-hand side w of the group: its accumulators, its
-  // reduction of the dependency products and its diagonal sweep, so the
-  // four sweeps run side by side on the CU's four SIMDs
-  const int32_t* in32 = reinterpret_cast<const int32_t*>(in);
-  uint64_t t = 0;
-  if (lane < rows)
-    t = static_cast<uint64_t>(static_cast<int64_t>(in32[static_cast<size_t>(r0 + lane) * 4 + w]))
-        << bit;
-  // the diagonal tile and the row scales depend on no other block: loaded
-  // before the first wait, so their latency stays off the chain
-  int32_t reg[kTB];
-  const int32_t* Td = T + static_cast<size_t>(ndep) * (kTB * kTB);
-#pragma unroll
-  for (int c = 0; c < kTB; ++c) reg[c] = Td[c * kTB + lane];
-  const int32_t dv = (K != TriKind::kL && lane < rows) ? dinv_g[r0 + lane] : 0;
-  for (int k = 0; k < ndep; ++k) {
-    const int bp = fwd ? k : nb - 1 - k;
-    const int32_t* Tk = T + static_cast<size_t>(k) * (kTB * kTB);
-    int32_t tv[16];
-#pragma unroll
-    for (int j = 0; j < 16; ++j) tv[j] = Tk[(16 * w + j) * kTB + lane];
-    if (w == 0) {
-      const int c = bp * kTB + lane;
-      unsigned long long v[4] = {0, 0, 0, 0};
-      int spins = 0;
-      while (true) {
-        bool ready = true;
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          v[q] = c < n ? __hip_atomic_load(&xp[static_cast<size_t>(c) * 4 + q], __ATOMIC_RELAXED,
-                                           __HIP_MEMORY_SCOPE_AGENT)
-                       : static_cast<unsigned long long>(static_cast<unsigned>(epoch)) << 32;
-          ready = ready && static_cast<int>(v[q] >> 32) == epoch;
-        }
-        if (__all(ready)) break;
-        __builtin_amdgcn_s_sleep(1);
-        if ((++spins & 31) == 0 && tile_wait_over(t0, err)) {
-          if (lane == 0) atomicAdd(err, 1);
-          break;
-        }
-      }
-#pragma unroll
-      for (int q = 0; q < 4; ++q)
-        xsh[q][lane] = c < n ? static_cast<int32_t>(static_cast<uint32_t>(v[q])) : 0;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      uint64_t ps = 0;
-#pragma unroll
-      for (int j = 0; j < 16; ++j) ps += prod64(tv[j], xsh[q][16 * w + j]);
-      part[w][q][lane] = ps;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int ww = 0; ww < kTileThreads / 64; ++ww) t -= part[ww][w][lane];
-  }
-  int32_t xv = 0;
-#pragma unroll
-  for (int st = 0; st < kTB; ++st) {
-    const int c = fwd ? st : kTB - 1 - st;
-    if (c < rows) {
-      const int32_t mine = acc_final<int32_t, K>(t, dv, bit, dbit);
-      if (lane == c) xv = mine;
-      const int32_t xc = __builtin_amdgcn_readlane(mine, c);
-      t -= prod64(reg[c], xc);
-    }
-  }
-  if (lane < rows) {
-    reinterpret_cast<int32_t*>(out)[static_cast<size_t>(r0 + lane) * 4 + w] = xv;
-    const unsigned long long word =
-        (static_cast<unsigned long long>(static_cast<unsigned>(epoch)) << 32) |
-        static_cast<uint32_t>(xv);
-    __hip_atomic_store(&xp[static_cast<size_t>(r0 + lane) * 4 + w], word, __ATOMIC_RELAXED,
-                       __HIP_MEMORY_SCOPE_AGENT);
-  }
-  tile_done(tickets, nb * groups);
-}
-
 }  // namespace
 
 hipError_t launch_permute_blk(int n, int groups, const int* perm, const void* src, void* dst,
@@ -387,20 +268,5 @@ hipError_t launch_spmv_blk(const DCsr& a, int groups, SpmvMode mode, const void*
   return spmv_blk_mode<2>(a, groups, x, z, y, s);
 }
 
-hipError_t launch_trsv_tiles_blk(TriKind kind, int n, int nb, int groups, const int32_t* tiles,
-                                 const long long* toff, const int32_t* dinv, int bit, int dbit,
-                                 const void* in, void* out, unsigned long long* xp, int epoch,
-                                 int* err, unsigned* tickets, hipStream_t s) {
-  if (n <= 0) return hipSuccess;
-  auto go = [&](auto kern) -> hipError_t {
-    hipLaunchKernelGGL(kern, dim3(nb * groups), dim3(kTileThreads), 0, s, n, nb, groups, tiles,
-                       toff, dinv, bit, dbit, static_cast<const int4*>(in),
-                       static_cast<int4*>(out), xp, epoch, err, tickets);
-    return hipGetLastError();
-  };
-  if (kind == TriKind::kL) return go(&k_tri_tiles_blk<TriKind::kL>);
-  if (kind == TriKind::kDU) return go(&k_tri_tiles_blk<TriKind::kDU>);
-  return go(&k_tri_tiles_blk<TriKind::kLD>);
-}
 
 }  // namespace sc23ad::dev

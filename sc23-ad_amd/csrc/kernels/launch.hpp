@@ -206,25 +206,17 @@ hipError_t launch_trsv_layout(Elem e, TriKind kind, const TriLayout& L,
 constexpr int kTriBlockWidth = 64;
 constexpr size_t kTriBlockedMaxLds = 160 * 1024;
 size_t tri_blocked_lds(int n, size_t elem, size_t acc);
-// Integer factor stored as dense 64-wide slices per column block (see
-// k_tri_dense_int); dinv[i] is row i's stored inverse diagonal (LD / DU).
-// Tiled integer solve of a coarse factor, one workgroup per 64-row block
-// (see k_tri_tiles_int); xp: n words {epoch, value} publishing the solved
-// rows, epoch: a value no word holds yet, err: incremented when a wait gives
-// up.
+// Tiled solve of a coarse factor (see k_tri_tiles); dinv[i]: row i's stored
+// inverse diagonal (DU); tmask (FP): one 64-bit mask of present entries per
+// tile row; xp: n words (FP64: 2 n) publishing the solved rows, epoch: a value
+// no word holds yet, err: incremented when a wait gives up, tickets: two
+// counters, zero between launches.
 constexpr int kTileMaxBlocks = 64;
-hipError_t launch_trsv_tiles(TriKind kind, int n, int nb, const int32_t* tiles,
-                             const long long* toff, const int32_t* dinv, int bit, int dbit,
-                             const void* in, void* out, unsigned long long* xp, int epoch,
-                             int* err, unsigned* tickets, hipStream_t s);
-// Tiled FP coarse solve (one wave per 64-row block, each row's terms in the
-// sequential order): tiles as for launch_trsv_tiles with FP values, tmask
-// one 64-bit mask of present entries per tile row, flags nb words raised to
-// epoch when a block is done (see k_tri_tiles_fp).
-hipError_t launch_trsv_tiles_fp(Elem e, TriKind kind, int n, int nb, const void* tiles,
-                                const long long* toff, const uint64_t* tmask, const void* dinv,
-                                const void* in, void* out, unsigned long long* flags, int epoch,
-                                int* err, unsigned* tickets, hipStream_t s);
+hipError_t launch_trsv_tiles(Elem e, TriKind kind, int n, int nb, const void* tiles,
+                             const long long* toff, const uint64_t* tmask, const void* dinv,
+                             int bit, int dbit, const void* in, void* out,
+                             unsigned long long* xp, int epoch, int* err, unsigned* tickets,
+                             hipStream_t s);
 hipError_t launch_trsv_blocked(Elem e, TriKind kind, const DCsr& a, const int* bptr,
                                int nb, const void* in, void* out, hipStream_t s);
 

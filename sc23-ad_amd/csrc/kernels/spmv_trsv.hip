@@ -791,159 +791,60 @@ __global__ __launch_bounds__(kBlkThreads) void k_tri_blocked_int(
   }
 }
 
-// Tiled integer coarse solve, one workgroup per 64-row block.  Workgroup b
-// owns rows 64b .. 64b+63.  Its factor entries are stored as dense 64 x 64
-// tiles (zeros where the factor has no entry), column-major (entry (row r,
-// column c) of a tile at c * 64 + r), in processing order: the off-diagonal
-// tiles of the blocks it depends on (forward: 0 .. b-1; backward: nb-1 ..
-// b+1), then its diagonal tile.  A solved row is published as one 64-bit
-// word {epoch, value} (xp[row], an agent-scope atomic store), so a consumer
-// learns that a value is ready and reads it in the same load.  For each
-// dependency block, wave 0 polls the block's 64 words until all carry the
-// current epoch, the workgroup subtracts the tile's product (four waves, 16
-// columns each; integer sums are order-free), then wave 0 sweeps the
-// diagonal tile: at step c lane c finishes its row and the value is broadcast
-// to the other lanes.  Dependencies point to blocks earlier in processing
-// order (forward: lower blocks; backward: higher ones), and workgroups take
-// their block from a ticket counter in that order, so a workgroup only ever
-// waits for workgroups that started before it, whatever order the hardware
-// starts them in and whatever else shares the GPU.  A launch that runs out
-// of its wait budget (tile_wait_over) records an error and gives up instead
-// of hanging.
-
-template <TriKind K>
-__global__ __launch_bounds__(kTileThreads) void k_tri_tiles_int(
-    int n, int nb, const int32_t* __restrict__ tiles, const long long* __restrict__ toff,
-    const int32_t* __restrict__ dinv_g, int bit, int dbit, const int32_t* __restrict__ in,
-    int32_t* out, unsigned long long* xp, int epoch, int* err, unsigned* tickets) {
-  constexpr bool fwd = (K != TriKind::kDU);
-  __shared__ uint64_t part[kTileThreads / 64][64];
-  __shared__ int32_t xsh[64];
-  __shared__ int ticket_sh;
-  const long long t0 = wall_clock64();
-  const int pb = tile_ticket(tickets, &ticket_sh);
-  const int b = fwd ? pb : nb - 1 - pb;
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const int r0 = b * kTB;
-  const int rows = min(kTB, n - r0);
-  const int32_t* T = tiles + toff[b];
-  const int ndep = fwd ? b : nb - 1 - b;
-  uint64_t t = 0;
-  if (w == 0 && lane < rows) t = static_cast<uint64_t>(static_cast<int64_t>(in[r0 + lane])) << bit;
-  // the diagonal tile and the row scales depend on no other block: wave 0
-  // loads them before its first wait, so their latency stays off the chain
-  int32_t reg[kTB];
-  int32_t dv = 0;
-  if (w == 0) {
-    const int32_t* Td = T + static_cast<size_t>(ndep) * (kTB * kTB);
-#pragma unroll
-    for (int c = 0; c < kTB; ++c) reg[c] = Td[c * kTB + lane];
-    dv = (K != TriKind::kL && lane < rows) ? dinv_g[r0 + lane] : 0;
-  }
-  for (int k = 0; k < ndep; ++k) {
-    const int bp = fwd ? k : nb - 1 - k;
-    const int32_t* Tk = T + static_cast<size_t>(k) * (kTB * kTB);
-    int32_t tv[16];
-#pragma unroll
-    for (int j = 0; j < 16; ++j) tv[j] = Tk[(16 * w + j) * kTB + lane];
-    if (w == 0) {
-      // two polls in flight: the next load is issued before the previous
-      // one is checked, so a block's words are seen about half a round trip
-      // sooner than with one poll at a time
-      const int c = bp * kTB + lane;
-      const unsigned long long none =
-          static_cast<unsigned long long>(static_cast<unsigned>(epoch)) << 32;
-      // every lane loads (rows past the end read row 0's word and ignore
-      // it): a load under a divergent branch would make the compiler wait
-      // for both polls where the paths join
-      const int cl = c < n ? c : 0;
-      auto poll = [&]() {
-        const unsigned long long u =
-            __hip_atomic_load(&xp[cl], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        return c < n ? u : none;
-      };
-      auto ready = [&](unsigned long long u) {
-        return __all(static_cast<int>(u >> 32) == epoch);
-      };
-      unsigned long long v = 0, va = poll();
-      int spins = 0;
-      while (true) {
-        __builtin_amdgcn_s_sleep(1);
-        const unsigned long long vb = poll();
-        if (ready(va)) {
-          v = va;
-          break;
-        }
-        __builtin_amdgcn_s_sleep(1);
-        va = poll();
-        if (ready(vb)) {
-          v = vb;
-          break;
-        }
-        if ((++spins & 15) == 0 && tile_wait_over(t0, err)) {
-          if (lane == 0) atomicAdd(err, 1);
-          v = vb;
-          break;
-        }
-      }
-      xsh[lane] = c < n ? static_cast<int32_t>(static_cast<uint32_t>(v)) : 0;
-    }
-    __syncthreads();
-    uint64_t ps = 0;
-#pragma unroll
-    for (int j = 0; j < 16; ++j) ps += prod64(tv[j], xsh[16 * w + j]);
-    part[w][lane] = ps;
-    __syncthreads();
-    if (w == 0) {
-#pragma unroll
-      for (int q = 0; q < kTileThreads / 64; ++q) t -= part[q][lane];
-    }
-  }
-  if (w == 0) {
-    // Diagonal sweep: at step c every lane finishes its row, lane c's value
-    // is broadcast and subtracted from the later rows.  (Chaining the row
-    // finish on the scalar unit instead, the next row's accumulator read
-    // from its lane, measured 45-55 % slower: the dependent scalar
-    // multiplies and the lane reads cost more than the vector finish.)
-    int32_t xv = 0;
-#pragma unroll
-    for (int st = 0; st < kTB; ++st) {
-      const int c = fwd ? st : kTB - 1 - st;
-      if (c < rows) {
-        const int32_t mine = acc_final<int32_t, K>(t, dv, bit, dbit);
-        if (lane == c) xv = mine;
-        const int32_t xc = __builtin_amdgcn_readlane(mine, c);
-        t -= prod64(reg[c], xc);
-      }
-    }
-    if (lane < rows) {
-      out[r0 + lane] = xv;
-      const unsigned long long word =
-          (static_cast<unsigned long long>(static_cast<unsigned>(epoch)) << 32) |
-          static_cast<uint32_t>(xv);
-      __hip_atomic_store(&xp[r0 + lane], word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-  }
-  tile_done(tickets, nb);
+// low32(mul_wrap(t >> bit, dinv) >> dbit) for shifts 0..31.  With q = t >> bit
+// as words qhi:qlo and dinv read as unsigned u = dinv + 2^32 [dinv < 0], the
+// low 64 bits of q dinv are qlo u plus, in the high word, qhi u - qlo
+// [dinv < 0]; the two products and the correction do not wait for each other.
+__device__ __forceinline__ int32_t rp_finish(uint64_t t, int32_t dinv, int bit, int dbit) {
+  const unsigned lo = static_cast<unsigned>(t), hi = static_cast<unsigned>(t >> 32);
+  const unsigned neg = static_cast<unsigned>(dinv >> 31);
+  const unsigned qlo = __builtin_amdgcn_alignbit(hi, lo, static_cast<unsigned>(bit));
+  const unsigned qhi = static_cast<unsigned>(static_cast<int>(hi) >> bit);
+  unsigned m;  // opaque: folded into the other product it would wait for it
+  asm("v_mul_lo_u32 %0, %1, %2" : "=v"(m) : "v"(qhi), "v"(dinv));
+  const uint64_t p = static_cast<uint64_t>(qlo) * static_cast<unsigned>(dinv);
+  const unsigned ph = static_cast<unsigned>(p >> 32) + m + ((0u - qlo) & neg);
+  return static_cast<int32_t>(
+      __builtin_amdgcn_alignbit(ph, static_cast<unsigned>(p), static_cast<unsigned>(dbit)));
 }
 
-// Tiled FP coarse solve (solvers 0 and 1), one wave per 64-row block, with
-// each row's terms subtracted in the sequential solve's order: the
-// dependency blocks in processing order (forward 0, 1, ...; backward nb-1,
-// nb-2, ...) and inside a tile the columns in the same direction, so a row
-// receives its terms in ascending column order (L) or descending (DU),
-// entries absent from the factor (clear bits of the row's 64-bit mask per
-// tile) skipped, exactly as the sequential CSR solve does.  Lane r owns row
-// 64 b + r.  A finished block publishes its values in `out`, then raises its
-// flag to the call's epoch (agent-scope release); a consumer waits for the
-// flag (acquire) and reads the block's values.  Blocks are taken from a
-// ticket counter in processing order, so every wait is on a workgroup that
-// started earlier; a launch out of its wait budget (tile_wait_over) records
-// an error and gives up instead of hanging.
+// Tiled coarse solve (integer and FP), one wave per 64-row block, kB
+// consecutive blocks per workgroup.  A block's factor entries are stored as
+// dense 64 x 64 tiles, column-major (entry (row r, column c) of a tile at c *
+// 64 + r), in processing order: the off-diagonal tiles of the blocks it
+// depends on (forward: 0 .. b-1; backward: nb-1 .. b+1), then its diagonal
+// tile.  Lane r owns row r and subtracts its terms column by column in that
+// order, the sequential solve's (ascending columns for L, descending for DU),
+// so FP sums round as the CPU's; integer sums are order-free.  FP: the product
+// of an entry absent from the factor (a clear bit of the row's 64-bit mask per
+// tile) is masked to +0, which leaves the sum unchanged, so only the
+// subtractions form a chain.
+//
+// A solved row is published as one 64-bit word {epoch, value} (FP64: two, for
+// the value's halves) in xp, an agent-scope atomic store, so a consumer learns
+// that a value is ready and reads it in the same load; two polls are in flight,
+// so the words are seen about half a round trip sooner.  Inside a workgroup
+// the values go through LDS: wave q sweeps its diagonal tile (at step c lane c
+// finishes its row and the value is broadcast), then the later waves subtract
+// its block's terms; the tiles among a workgroup's blocks wait in LDS.  The
+// tile of the next outside dependency is loaded into the registers of the
+// columns just used, so its latency is covered by the wait.
+//
+// What bounds it is the chain: per block the sweep's 64 dependent steps and a
+// tile product, plus per workgroup one hand-off through memory.  With a
+// workgroup per block, its four waves sharing the products, every block paid
+// the hand-off (integer, 128^3: 83 + 105 us per solve, now 60 + 82; FP64, 96^3: 30
+// blocks, 187 + 190 us, now 92 + 93; FP32, 48^3: 89 + 89, now 43 + 43).
+//
+// Workgroups take their blocks (and right-hand side) from a ticket counter in
+// processing order, so a workgroup only ever waits for workgroups that started
+// before it, whatever order the hardware starts them in and whatever else
+// shares the GPU.  A launch that runs out of its wait budget (tile_wait_over)
+// records an error and gives up instead of hanging.
 template <typename T>
-__device__ __forceinline__ T readlane_fp(T v, int src);
+__device__ __forceinline__ T readlane_of(T v, int src);
 template <>
-__device__ __forceinline__ double readlane_fp<double>(double v, int src) {
+__device__ __forceinline__ double readlane_of<double>(double v, int src) {
   const long long b = __double_as_longlong(v);
   const int lo = __builtin_amdgcn_readlane(static_cast<int>(static_cast<unsigned long long>(b)), src);
   const int hi = __builtin_amdgcn_readlane(static_cast<int>(static_cast<unsigned long long>(b) >> 32), src);
@@ -951,77 +852,205 @@ __device__ __forceinline__ double readlane_fp<double>(double v, int src) {
       (static_cast<unsigned long long>(static_cast<unsigned>(hi)) << 32) | static_cast<unsigned>(lo)));
 }
 template <>
-__device__ __forceinline__ float readlane_fp<float>(float v, int src) {
+__device__ __forceinline__ float readlane_of<float>(float v, int src) {
   return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), src));
 }
+template <>
+__device__ __forceinline__ int32_t readlane_of<int32_t>(int32_t v, int src) {
+  return __builtin_amdgcn_readlane(v, src);
+}
 
-template <typename T, TriKind K>
-__global__ __launch_bounds__(64) void k_tri_tiles_fp(
-    int n, int nb, const T* __restrict__ tiles, const long long* __restrict__ toff,
-    const uint64_t* __restrict__ tmask, const T* __restrict__ dinv_g,
-    const T* __restrict__ in, T* out, unsigned long long* flags, int epoch, int* err,
+// t - v x where bit `c` of the row's mask is set (FP); integer tiles hold
+// negated values, zero where the factor has no entry: t + v x
+__device__ __forceinline__ uint64_t tile_sub(uint64_t t, int32_t v, int32_t x, uint64_t, int) {
+  return t + prod64(v, x);
+}
+__device__ __forceinline__ float tile_sub(float t, float v, float x, uint64_t mask, int c) {
+  const unsigned w = static_cast<unsigned>(c < 32 ? mask : mask >> 32);
+  const int m = __builtin_amdgcn_sbfe(static_cast<int>(w), c % 32, 1);
+  return t - __int_as_float(__float_as_int(v * x) & m);
+}
+__device__ __forceinline__ double tile_sub(double t, double v, double x, uint64_t mask, int c) {
+  const unsigned w = static_cast<unsigned>(c < 32 ? mask : mask >> 32);
+  const int m = __builtin_amdgcn_sbfe(static_cast<int>(w), c % 32, 1);
+  const unsigned long long b = static_cast<unsigned long long>(__double_as_longlong(v * x));
+  const unsigned lo = static_cast<unsigned>(b) & m, hi = static_cast<unsigned>(b >> 32) & m;
+  return t - __longlong_as_double(
+                 static_cast<long long>((static_cast<unsigned long long>(hi) << 32) | lo));
+}
+
+// The row's value; kShort: integer shifts of 0..31 (a shorter chain).
+template <typename T, TriKind K, bool kShort>
+__device__ __forceinline__ T tile_finish(typename AccOf<T>::type t, T dinv, int bit, int dbit) {
+  if constexpr (std::is_same_v<T, int32_t> && kShort) {
+    if constexpr (K == TriKind::kL)
+      return static_cast<int32_t>(__builtin_amdgcn_alignbit(
+          static_cast<unsigned>(t >> 32), static_cast<unsigned>(t), static_cast<unsigned>(bit)));
+    else
+      return rp_finish(t, dinv, bit, dbit);
+  } else {
+    return acc_final<T, K>(t, dinv, bit, dbit);
+  }
+}
+
+// kS: 1 for plain vectors; 4 for a block of nrhs right-hand sides (element
+// (row i, right-hand side r) at ((r / 4) n + i) 4 + r % 4).
+template <typename T, TriKind K, bool kShort, int kS, int kB>
+__global__ __launch_bounds__(64 * kB) void k_tri_tiles(
+    int n, int nb, int nrhs, const T* __restrict__ tiles, const long long* __restrict__ toff,
+    const uint64_t* __restrict__ tmask, const T* __restrict__ dinv_g, int bit, int dbit,
+    const T* __restrict__ in_all, T* out_all, unsigned long long* xp_all, int epoch, int* err,
     unsigned* tickets) {
-  constexpr bool fwd = (K != TriKind::kDU);
-  __shared__ T dl[kTB][kTB];  // the diagonal tile, [column][row]: lane r reads only its row
+  constexpr bool fwd = (K != TriKind::kDU), kFp = !std::is_same_v<T, int32_t>;
+  constexpr int kW = sizeof(T) / 4;  // published words per row
+  // wave w's tiles against the workgroup's blocks 0 .. w (its diagonal tile
+  // last), column-major: lane r reads only row r's values
+  extern __shared__ __align__(16) unsigned char smem_t[];
+  __shared__ T xs[kB][kTB];
   __shared__ int ticket_sh;
   const long long t0 = wall_clock64();
-  const int pb = tile_ticket(tickets, &ticket_sh);
-  const int b = fwd ? pb : nb - 1 - pb;
-  const int lane = threadIdx.x;
+  const int ticket = tile_ticket(tickets, &ticket_sh);
+  const int group = ticket / nrhs, r = ticket % nrhs;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int first = group * kB;  // dependencies of earlier workgroups
+  const int pb = first + w;      // place in processing order = dependencies
+  const bool valid = pb < nb;
+  const int b = !valid ? 0 : fwd ? pb : nb - 1 - pb;
+  const size_t off = kS == 1 ? 0 : static_cast<size_t>(r >> 2) * n * 4 + (r & 3);
+  const T* in = in_all + off;
+  T* out = out_all + off;
+  unsigned long long* xp = xp_all + static_cast<size_t>(r) * n * kW;
   const int r0 = b * kTB;
-  const int rows = min(kTB, n - r0);
+  const int rows = valid ? min(kTB, n - r0) : 0;
   const T* Tb = tiles + toff[b];
-  const uint64_t* Mb = tmask + toff[b] / kTB;  // one mask per tile row
-  const int ndep = fwd ? b : nb - 1 - b;
-  // the diagonal tile, its masks and the row scales depend on no other
-  // block: loaded before the first wait, so their latency stays off the chain
-  const T* Td = Tb + static_cast<size_t>(ndep) * (kTB * kTB);
+  const uint64_t* Mb = kFp ? tmask + toff[b] / kTB : nullptr;  // one mask per tile row
+  T* mine_lds = reinterpret_cast<T*>(smem_t) + static_cast<size_t>(w * (w + 1) / 2) * (kTB * kTB);
+  uint64_t mi[kB];  // masks of the tiles in LDS
 #pragma unroll
-  for (int c = 0; c < kTB; ++c) dl[c][lane] = Td[c * kTB + lane];
-  const uint64_t md = Mb[static_cast<size_t>(ndep) * kTB + lane];
+  for (int q = 0; q < kB; ++q) mi[q] = 0;
+  if (valid) {
+#pragma unroll
+    for (int q = 0; q < kB; ++q)
+      if (q <= w) {
+        const T* Tq = Tb + static_cast<size_t>(first + q) * (kTB * kTB);
+#pragma unroll 16
+        for (int c = 0; c < kTB; ++c)
+          mine_lds[(q * kTB + c) * kTB + lane] = Tq[c * kTB + lane];
+        if (kFp) mi[q] = Mb[static_cast<size_t>(first + q) * kTB + lane];
+      }
+  }
   const T dv = (K != TriKind::kL && lane < rows) ? dinv_g[r0 + lane] : T(0);
-  T t = lane < rows ? in[r0 + lane] : T(0);
-  const unsigned long long want = static_cast<unsigned long long>(static_cast<unsigned>(epoch));
-  for (int k = 0; k < ndep; ++k) {
-    const int bp = fwd ? k : nb - 1 - k;
-    // the dependency tile is loaded before the wait for its block
-    const T* Tk = Tb + static_cast<size_t>(k) * (kTB * kTB);
-    T vk[kTB];
+  typename AccOf<T>::type t =
+      acc_init<T>(lane < rows ? in[static_cast<size_t>(r0 + lane) * kS] : T(0), bit);
+  // vk: the current outside dependency's tile (without one: any, unused)
+  T vk[kTB];
 #pragma unroll
-    for (int c = 0; c < kTB; ++c) vk[c] = Tk[c * kTB + lane];
-    const uint64_t mk = Mb[static_cast<size_t>(k) * kTB + lane];
+  for (int c = 0; c < kTB; ++c) vk[c] = Tb[c * kTB + lane];
+  uint64_t mk = kFp ? Mb[lane] : 0;
+  const unsigned long long tag = static_cast<unsigned long long>(static_cast<unsigned>(epoch))
+                                 << 32;
+  for (int k = 0; k < (valid ? first : 0); ++k) {
+    // every lane loads (rows past the end the last row's words, which no entry
+    // names): a load under a divergent branch would make the compiler wait
+    // for both polls where the paths join
+    const int row = min((fwd ? k : nb - 1 - k) * kTB + lane, n - 1);
+    struct Words {
+      unsigned long long w[kW];
+    };
+    auto poll = [&]() {
+      Words u;
+#pragma unroll
+      for (int q = 0; q < kW; ++q)
+        u.w[q] = __hip_atomic_load(&xp[kW * row + q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      return u;
+    };
+    auto ready = [&](const Words& u) {
+      bool ok = true;
+#pragma unroll
+      for (int q = 0; q < kW; ++q) ok = ok && (u.w[q] >> 32) == (tag >> 32);
+      return __all(ok);
+    };
+    Words v, va = poll();
     int spins = 0;
-    while (__hip_atomic_load(&flags[bp], __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT) != want) {
+    while (true) {
       __builtin_amdgcn_s_sleep(1);
-      if ((++spins & 31) == 0 && tile_wait_over(t0, err)) {
+      const Words vb = poll();
+      if (ready(va)) {
+        v = va;
+        break;
+      }
+      __builtin_amdgcn_s_sleep(1);
+      va = poll();
+      if (ready(vb)) {
+        v = vb;
+        break;
+      }
+      if ((++spins & 15) == 0 && tile_wait_over(t0, err)) {
         if (lane == 0) atomicAdd(err, 1);
+        v = vb;
         break;
       }
     }
-    const int cmax = min(kTB, n - bp * kTB);
-    const T xmine = lane < cmax ? out[bp * kTB + lane] : T(0);
+    T x;
+    if constexpr (kW == 2)
+      x = __longlong_as_double(
+          static_cast<long long>((v.w[1] << 32) | static_cast<unsigned>(v.w[0])));
+    else if constexpr (kFp)
+      x = __uint_as_float(static_cast<unsigned>(v.w[0]));
+    else
+      x = static_cast<int32_t>(static_cast<unsigned>(v.w[0]));
+    // the terms of dependency k; the next one's tile replaces this one's
+    const size_t nx = static_cast<size_t>(min(k + 1, first - 1));
+    const T* Tn = Tb + nx * (kTB * kTB);
+    const uint64_t mn = kFp ? Mb[nx * kTB + lane] : 0;
 #pragma unroll
     for (int st = 0; st < kTB; ++st) {
       const int c = fwd ? st : kTB - 1 - st;
-      const T xc = readlane_fp<T>(xmine, c);
-      if ((mk >> c) & 1) t = t - vk[c] * xc;
+      t = tile_sub(t, vk[c], readlane_of<T>(x, c), mk, c);
+      vk[c] = Tn[c * kTB + lane];
     }
+    mk = mn;
   }
-  T xv = T(0);
 #pragma unroll
-  for (int st = 0; st < kTB; ++st) {
-    const int c = fwd ? st : kTB - 1 - st;
-    if (c < rows) {
-      const T mine = acc_final<T, K>(t, dv, 0, 0);
-      if (lane == c) xv = mine;
-      const T xc = readlane_fp<T>(mine, c);
-      if ((md >> c) & 1) t = t - dl[c][lane] * xc;
+  for (int q = 0; q < kB; ++q) {
+    if (w == q && valid) {
+#pragma unroll
+      for (int st = 0; st < kTB; ++st) {
+        // no test for rows past the end, whose values are zero and which no
+        // entry names: a branch per step would keep the tile's LDS reads from
+        // being issued ahead
+        const int c = fwd ? st : kTB - 1 - st;
+        const T mine = tile_finish<T, K, kShort>(t, dv, bit, dbit);
+        t = tile_sub(t, mine_lds[(q * kTB + c) * kTB + lane], readlane_of<T>(mine, c), mi[q], c);
+      }
+      // a row has no entries at its own step or later: its sum still stands
+      const T xv = tile_finish<T, K, kShort>(t, dv, bit, dbit);
+      xs[q][lane] = xv;
+      if (lane < rows) {
+        unsigned long long bits;
+        if constexpr (kW == 2) bits = static_cast<unsigned long long>(__double_as_longlong(xv));
+        else if constexpr (kFp) bits = __float_as_uint(xv);
+        else bits = static_cast<uint32_t>(xv);
+#pragma unroll
+        for (int h = 0; h < kW; ++h)
+          __hip_atomic_store(&xp[kW * (r0 + lane) + h],
+                             tag | static_cast<uint32_t>(bits >> (32 * h)), __ATOMIC_RELAXED,
+                             __HIP_MEMORY_SCOPE_AGENT);
+        out[static_cast<size_t>(r0 + lane) * kS] = xv;
+      }
+    }
+    if (q + 1 == kB) break;
+    lds_barrier();
+    if (w > q && valid) {
+      const T x = xs[q][lane];
+#pragma unroll
+      for (int st = 0; st < kTB; ++st) {
+        const int c = fwd ? st : kTB - 1 - st;
+        t = tile_sub(t, mine_lds[(q * kTB + c) * kTB + lane], readlane_of<T>(x, c), mi[q], c);
+      }
     }
   }
-  if (lane < rows) out[r0 + lane] = xv;
-  __threadfence();
-  if (lane == 0) __hip_atomic_store(&flags[b], want, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
-  tile_done(tickets, nb);
+  tile_done(tickets, (nb + kB - 1) / kB * nrhs);
 }
 
 template <typename T, TriKind K>
@@ -1586,23 +1615,6 @@ __device__ __forceinline__ uint64_t group_sum_dpp(uint64_t v) {
   if (kG >= 32) v = permlane_add(v, false);
   if (kG >= 64) v = permlane_add(v, true);
   return v;
-}
-
-// low32(mul_wrap(t >> bit, dinv) >> dbit) for shifts 0..31.  With q = t >> bit
-// as words qhi:qlo and dinv read as unsigned u = dinv + 2^32 [dinv < 0], the
-// low 64 bits of q dinv are qlo u plus, in the high word, qhi u - qlo
-// [dinv < 0]; the two products and the correction do not wait for each other.
-__device__ __forceinline__ int32_t rp_finish(uint64_t t, int32_t dinv, int bit, int dbit) {
-  const unsigned lo = static_cast<unsigned>(t), hi = static_cast<unsigned>(t >> 32);
-  const unsigned neg = static_cast<unsigned>(dinv >> 31);
-  const unsigned qlo = __builtin_amdgcn_alignbit(hi, lo, static_cast<unsigned>(bit));
-  const unsigned qhi = static_cast<unsigned>(static_cast<int>(hi) >> bit);
-  unsigned m;  // opaque: folded into the other product it would wait for it
-  asm("v_mul_lo_u32 %0, %1, %2" : "=v"(m) : "v"(qhi), "v"(dinv));
-  const uint64_t p = static_cast<uint64_t>(qlo) * static_cast<unsigned>(dinv);
-  const unsigned ph = static_cast<unsigned>(p >> 32) + m + ((0u - qlo) & neg);
-  return static_cast<int32_t>(
-      __builtin_amdgcn_alignbit(ph, static_cast<unsigned>(p), static_cast<unsigned>(dbit)));
 }
 
 // Level L (buffer cur).  nxt: the buffer level L - 1 has freed, filled for
@@ -2362,46 +2374,65 @@ size_t tri_blocked_lds(int n, size_t elem, size_t acc) {
   return b + 8 * kTB + elem * kTB * kTB;
 }
 
-hipError_t launch_trsv_tiles(TriKind kind, int n, int nb, const int32_t* tiles,
-                             const long long* toff, const int32_t* dinv, int bit, int dbit,
-                             const void* in, void* out, unsigned long long* xp, int epoch,
-                             int* err, unsigned* tickets, hipStream_t s) {
-  if (n <= 0) return hipSuccess;
+// Blocks per workgroup: the most whose tiles fit in LDS with one workgroup per
+// CU (kB (kB + 1) / 2 of them); one for a block of right-hand sides, whose many
+// workgroups share the CUs with other systems' kernels.
+template <typename T, bool kShort, int kS>
+static hipError_t tri_tiles_go(TriKind kind, int n, int nb, int nrhs, const void* tiles,
+                               const long long* toff, const uint64_t* tmask, const void* dinv,
+                               int bit, int dbit, const void* in, void* out,
+                               unsigned long long* xp, int epoch, int* err, unsigned* tickets,
+                               hipStream_t s) {
+  if (n <= 0 || nrhs <= 0) return hipSuccess;
+  if (nb > kTileMaxBlocks) return hipErrorInvalidValue;
+  constexpr int kB = kS > 1 ? 1 : sizeof(T) == 8 ? 2 : 3;
+  constexpr size_t lds = sizeof(T) * kTB * kTB * kB * (kB + 1) / 2;
   auto go = [&](auto kern) -> hipError_t {
-    hipLaunchKernelGGL(kern, dim3(nb), dim3(kTileThreads), 0, s, n, nb, tiles, toff, dinv, bit,
-                       dbit, static_cast<const int32_t*>(in), static_cast<int32_t*>(out), xp,
-                       epoch, err, tickets);
+    if constexpr (lds > 65536) {
+      const hipError_t e =
+          hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
+                              hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
+      if (e != hipSuccess) return e;
+    }
+    hipLaunchKernelGGL(kern, dim3((nb + kB - 1) / kB * nrhs), dim3(64 * kB), lds, s, n, nb, nrhs, static_cast<const T*>(tiles),
+                       toff, tmask, static_cast<const T*>(dinv), bit, dbit,
+                       static_cast<const T*>(in), static_cast<T*>(out), xp, epoch, err, tickets);
     return hipGetLastError();
   };
-  if (kind == TriKind::kL) return go(&k_tri_tiles_int<TriKind::kL>);
-  if (kind == TriKind::kDU) return go(&k_tri_tiles_int<TriKind::kDU>);
-  return go(&k_tri_tiles_int<TriKind::kLD>);
+  if (kind == TriKind::kL) return go(&k_tri_tiles<T, TriKind::kL, kShort, kS, kB>);
+  if (kind == TriKind::kDU) return go(&k_tri_tiles<T, TriKind::kDU, kShort, kS, kB>);
+  return hipErrorInvalidValue;  // only the coarse factors are tiled
 }
 
-hipError_t launch_trsv_tiles_fp(Elem e, TriKind kind, int n, int nb, const void* tiles,
-                                const long long* toff, const uint64_t* tmask, const void* dinv,
-                                const void* in, void* out, unsigned long long* flags, int epoch,
-                                int* err, unsigned* tickets, hipStream_t s) {
-  if (n <= 0) return hipSuccess;
-  if (nb > kTileMaxBlocks) return hipErrorInvalidValue;
-  auto go = [&](auto tag, auto kern) -> hipError_t {
-    using T = decltype(tag);
-    hipLaunchKernelGGL(kern, dim3(nb), dim3(64), 0, s, n, nb, static_cast<const T*>(tiles), toff,
-                       tmask, static_cast<const T*>(dinv), static_cast<const T*>(in),
-                       static_cast<T*>(out), flags, epoch, err, tickets);
-    return hipGetLastError();
-  };
-  if (e == Elem::kF64) {
-    if (kind == TriKind::kL) return go(double{}, &k_tri_tiles_fp<double, TriKind::kL>);
-    if (kind == TriKind::kDU) return go(double{}, &k_tri_tiles_fp<double, TriKind::kDU>);
-    return go(double{}, &k_tri_tiles_fp<double, TriKind::kLD>);
-  }
-  if (e == Elem::kF32) {
-    if (kind == TriKind::kL) return go(float{}, &k_tri_tiles_fp<float, TriKind::kL>);
-    if (kind == TriKind::kDU) return go(float{}, &k_tri_tiles_fp<float, TriKind::kDU>);
-    return go(float{}, &k_tri_tiles_fp<float, TriKind::kLD>);
-  }
-  return hipErrorInvalidValue;
+hipError_t launch_trsv_tiles(Elem e, TriKind kind, int n, int nb, const void* tiles,
+                             const long long* toff, const uint64_t* tmask, const void* dinv,
+                             int bit, int dbit, const void* in, void* out,
+                             unsigned long long* xp, int epoch, int* err, unsigned* tickets,
+                             hipStream_t s) {
+  if (e == Elem::kF64)
+    return tri_tiles_go<double, false, 1>(kind, n, nb, 1, tiles, toff, tmask, dinv, 0, 0, in, out,
+                                          xp, epoch, err, tickets, s);
+  if (e == Elem::kF32)
+    return tri_tiles_go<float, false, 1>(kind, n, nb, 1, tiles, toff, tmask, dinv, 0, 0, in, out,
+                                         xp, epoch, err, tickets, s);
+  const bool in_word = bit >= 0 && bit < 32 && (kind == TriKind::kL || (dbit >= 0 && dbit < 32));
+  return in_word ? tri_tiles_go<int32_t, true, 1>(kind, n, nb, 1, tiles, toff, nullptr, dinv, bit,
+                                                  dbit, in, out, xp, epoch, err, tickets, s)
+                 : tri_tiles_go<int32_t, false, 1>(kind, n, nb, 1, tiles, toff, nullptr, dinv,
+                                                   bit, dbit, in, out, xp, epoch, err, tickets, s);
+}
+
+hipError_t launch_trsv_tiles_blk(TriKind kind, int n, int nb, int groups, const int32_t* tiles,
+                                 const long long* toff, const int32_t* dinv, int bit, int dbit,
+                                 const void* in, void* out, unsigned long long* xp, int epoch,
+                                 int* err, unsigned* tickets, hipStream_t s) {
+  const bool in_word = bit >= 0 && bit < 32 && (kind == TriKind::kL || (dbit >= 0 && dbit < 32));
+  return in_word
+             ? tri_tiles_go<int32_t, true, 4>(kind, n, nb, 4 * groups, tiles, toff, nullptr, dinv,
+                                              bit, dbit, in, out, xp, epoch, err, tickets, s)
+             : tri_tiles_go<int32_t, false, 4>(kind, n, nb, 4 * groups, tiles, toff, nullptr,
+                                               dinv, bit, dbit, in, out, xp, epoch, err, tickets,
+                                               s);
 }
 
 hipError_t launch_trsv_blocked(Elem e, TriKind kind, const DCsr& a, const int* bptr,

@@ -61,7 +61,6 @@ __device__ __forceinline__ int32_t acc_final<int32_t, TriKind::kDU>(uint64_t t, 
   return low32(mul_wrap(as_i64(t) >> bit, dinv) >> dbit);
 }
 
-constexpr int kTileThreads = 256;
 
 // Wait budget of the tiled coarse solves: one launch gives up its waits once
 // 2^27 ticks of the constant 100 MHz clock (1.3 s) have passed since the
