@@ -1217,7 +1217,7 @@ void tune_spmv(DevMat& m, Elem e, SpmvMode mode) {
       c.remap = 1;
       cands.push_back(c);
     }
-  // SC23AD_SPMV_FORMAT=csr|sell|sell16 keeps only that format's candidates
+  // SC23AD_SPMV_FORMAT=csr|stream|sell|sell16|sellcol keeps only that format's candidates
   // where the matrix has it (tests run every kernel this way).
   if (const char* f = std::getenv("SC23AD_SPMV_FORMAT")) {
     const std::string want(f);

@@ -2387,20 +2387,22 @@ static hipError_t tri_tiles_go(TriKind kind, int n, int nb, int nrhs, const void
   if (nb > kTileMaxBlocks) return hipErrorInvalidValue;
   constexpr int kB = kS > 1 ? 1 : sizeof(T) == 8 ? 2 : 3;
   constexpr size_t lds = sizeof(T) * kTB * kTB * kB * (kB + 1) / 2;
-  auto go = [&](auto kern) -> hipError_t {
-    if constexpr (lds > 65536) {
+  auto go = [&](auto kern, bool& attr) -> hipError_t {
+    if (!attr) {
       const hipError_t e =
           hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                               hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
       if (e != hipSuccess) return e;
+      attr = true;
     }
     hipLaunchKernelGGL(kern, dim3((nb + kB - 1) / kB * nrhs), dim3(64 * kB), lds, s, n, nb, nrhs, static_cast<const T*>(tiles),
                        toff, tmask, static_cast<const T*>(dinv), bit, dbit,
                        static_cast<const T*>(in), static_cast<T*>(out), xp, epoch, err, tickets);
     return hipGetLastError();
   };
-  if (kind == TriKind::kL) return go(&k_tri_tiles<T, TriKind::kL, kShort, kS, kB>);
-  if (kind == TriKind::kDU) return go(&k_tri_tiles<T, TriKind::kDU, kShort, kS, kB>);
+  static bool attr_l = false, attr_du = false;
+  if (kind == TriKind::kL) return go(&k_tri_tiles<T, TriKind::kL, kShort, kS, kB>, attr_l);
+  if (kind == TriKind::kDU) return go(&k_tri_tiles<T, TriKind::kDU, kShort, kS, kB>, attr_du);
   return hipErrorInvalidValue;  // only the coarse factors are tiled
 }
 
