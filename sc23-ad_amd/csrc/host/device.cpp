@@ -438,7 +438,7 @@ void plan_rp(TriPlan& plan, int n, const std::vector<int>& lbeg, const std::vect
     for (int e : {4, 6, 8, 10, 12}) {
       const int g = 1 << lg;
       if (g * e < md || (g == 1 && e == 6) ||
-          static_cast<uint64_t>(n) * (g * e * 8) > UINT32_MAX)
+          static_cast<uint64_t>(n) * (g * e * 8) > dev::kRpMaxBytes)
         continue;
       // far entries over several lanes: 8 entries or more, kRpFarSlots far ones
       if (farq > 0 && g > 1 && (e < 8 || farq > dev::kRpFarSlots * g)) continue;
@@ -559,7 +559,7 @@ void plan_rpf(TriPlan& plan, int n, const std::vector<int>& lbeg, const std::vec
   for (int g = 1; g <= 64; g *= 2)
     for (int e : {4, 8}) {
       if (g * e < md || (only_lanes > 0 && g != only_lanes) ||
-          static_cast<uint64_t>(n) * g * e * kT > UINT32_MAX)
+          static_cast<uint64_t>(n) * g * e * kT > dev::kRpMaxBytes)
         continue;
       for (int w = 1; w <= 8; ++w) {
         if (only_waves > 0 && w != only_waves) continue;

@@ -147,6 +147,9 @@ constexpr int kRpMaxWaves = 16;   // more than 8: one lane of 4 entries per row
 constexpr int kRpFarSlots = 4;    // far entries per lane of layouts over several lanes
 constexpr int kRpMaxAhead = 4;    // far values are loaded at most this many levels ahead
 constexpr int kRpPadLevels = 12;  // level offsets past a chain's last one
+// Most bytes of padded entries: 32-bit offsets, with room for the lanes past
+// the last row (at most 16 waves of 128 bytes per lane).
+constexpr uint64_t kRpMaxBytes = (uint64_t{1} << 32) - 16 * 64 * 128;
 hipError_t launch_trsv_rp(const TriLayout& L, int bit, int dbit, const void* in, void* out,
                           hipStream_t s);
 hipError_t launch_trsv_rpf(Elem e, const TriLayout& L, const void* in, void* out,

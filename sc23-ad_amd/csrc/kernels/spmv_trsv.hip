@@ -1503,10 +1503,14 @@ hipError_t tri_ep_launch(const TriLayout& L, const TriSegment& seg, int bit, int
 //    no address arithmetic) and the negated value, so a row's sum starts from
 //    in * 2^bit and only adds products; a far entry (the first kFq slots of a
 //    row at most) holds ~(4 * position) instead;
-//  * entries, inverse diagonals, right-hand sides and results are buffers
-//    addressed by a scalar offset per level plus a lane offset that never
-//    changes; lanes past a level's end load what follows (past the buffer's
-//    end: 0) and never store;
+//  * entries, inverse diagonals, right-hand sides and results are buffers of
+//    exactly their bytes, addressed by a lane's place in the level plus the
+//    level's start; lanes past a level's end load what follows (past the
+//    buffer's end: 0) and never store.  The sum is the instruction's vector
+//    offset, the one that the hardware compares with the buffer's size: with
+//    the level's start as its scalar offset, which that comparison does not
+//    count (or subtracts from the size, where it may pass it), the rows past
+//    the last one would be read from beyond the buffer;
 //  * the loads of level L + kD - 1 are issued into the buffer that level L - 1
 //    has freed, between this level's ring reads and their first use;
 //  * shifts by bit and dbit (0..30) are single 32-bit funnel shifts, and the
@@ -1538,14 +1542,13 @@ struct RpArgs {
 
 // Constants of a lane.
 struct RpLane {
-  int ent_off;            // its entries' byte offset from the level's first row's
-  int row4;               // 4 * its row in the level
-  int vec_off;            // its row's byte offset in the vectors (stride 4 or 16)
+  unsigned ent_off;       // its entries' byte offset from the level's first row's
+  unsigned row4;          // 4 * its row in the level
   int owner;              // its row for the row's first lane, else INT32_MAX
   int32_t scale;          // 2^bit for the row's first lane, else 0
 };
 
-// A buffer of `bytes` bytes; loads past its end return 0.
+// A buffer of `bytes` bytes; loads whose vector offset is past its end return 0.
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t rp_buffer(const void* p, unsigned bytes) {
   constexpr int kRaw32 = 0x00020000;  // untyped, 32-bit elements
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, static_cast<int>(bytes),
@@ -1564,12 +1567,15 @@ __device__ __forceinline__ void rp_load(RpPre<kE, kFq>& r, int lo, int hi, const
                                         const RpLane& ln) {
   r.lo = lo;
   r.cnt = hi - lo;
-  const int lo4 = 4 * lo, loe = static_cast<int>(static_cast<unsigned>(lo) * (kG * kE * 8));
+  const unsigned pos4 = 4u * static_cast<unsigned>(lo) + ln.row4;
+  const unsigned ent = static_cast<unsigned>(lo) * (kG * kE * 8) + ln.ent_off;
 #pragma unroll
   for (int h = 0; h < kE / 2; ++h)
-    r.ent[h] = __builtin_amdgcn_raw_buffer_load_b128(a.rent, ln.ent_off + 16 * h, loe, 0);
-  r.dinv = static_cast<int>(__builtin_amdgcn_raw_buffer_load_b32(a.dinv, ln.row4, lo4, 0));
-  r.in = static_cast<int>(__builtin_amdgcn_raw_buffer_load_b32(a.in, ln.vec_off, kS * lo4, 0));
+    r.ent[h] = __builtin_amdgcn_raw_buffer_load_b128(a.rent, static_cast<int>(ent) + 16 * h, 0, 0);
+  r.dinv = static_cast<int>(
+      __builtin_amdgcn_raw_buffer_load_b32(a.dinv, static_cast<int>(pos4), 0, 0));
+  r.in = static_cast<int>(
+      __builtin_amdgcn_raw_buffer_load_b32(a.in, static_cast<int>(kS * pos4), 0, 0));
 }
 
 // acc + dpp(acc) on 64-bit values, one stage of a group sum: the low words'
@@ -1675,10 +1681,10 @@ __device__ __forceinline__ void rp_level(RpPre<kE, kFq>& cur, RpPre<kE, kFq>& nx
   acc = group_sum_dpp<kG>(acc + acc2);
   const int32_t v = rp_finish(acc, cur.dinv, a.bit, a.dbit);
   if (ln.owner < cur.cnt) {
-    const int lo4 = 4 * cur.lo;
-    *rp_lds(static_cast<unsigned>(lo4 + ln.row4) & a.ring_mask) = v;
-    __builtin_amdgcn_raw_buffer_store_b32(static_cast<unsigned>(v), a.out, ln.vec_off, kS * lo4,
-                                          0);
+    const unsigned pos4 = 4u * static_cast<unsigned>(cur.lo) + ln.row4;
+    *rp_lds(pos4 & a.ring_mask) = v;
+    __builtin_amdgcn_raw_buffer_store_b32(static_cast<unsigned>(v), a.out,
+                                          static_cast<int>(kS * pos4), 0, 0);
   }
   // a full fence every fence_mask + 1 levels makes far values visible before
   // any load of them; it also drains the loads in flight, so the plan makes
@@ -1731,9 +1737,8 @@ __global__ __launch_bounds__(64 * kMaxWaves) void k_tri_chain_rp(
   const RpArgs a{rp_buffer(rent, n4 * (kG * kE * 2)), rp_buffer(dinv, n4),
                  rp_buffer(in + off, vec_bytes), rp_buffer(out + off, vec_bytes), static_cast<unsigned>(ring4) - 1u, bit, dbit, fence - 1};
   RpLane ln;
-  ln.ent_off = t * (kE * 8);
-  ln.row4 = 4 * (t / kG);
-  ln.vec_off = kS * ln.row4;
+  ln.ent_off = static_cast<unsigned>(t) * (kE * 8);
+  ln.row4 = 4u * static_cast<unsigned>(t / kG);
   ln.owner = t % kG == 0 ? t / kG : INT32_MAX;
   ln.scale = t % kG == 0 ? 1 << bit : 0;
   RpPre<kE, kFq> buf[kD];
@@ -1762,7 +1767,8 @@ hipError_t tri_rp_go(const TriLayout& L, int nrhs, int bit, int dbit, const int3
                      int32_t* out, hipStream_t s) {
   const size_t lds = rp_lds_bytes(L.rp_ring, L.rp_maxlev);
   if (lds > static_cast<size_t>(kTriBlockedMaxLds) || L.n <= 0 || bit < 0 || bit > 30 ||
-      dbit < 0 || dbit > 30 || L.rp_fence < 1 || static_cast<uint64_t>(L.n) * (kG * kE * 8) > UINT32_MAX)
+      dbit < 0 || dbit > 30 || L.rp_fence < 1 ||
+      static_cast<uint64_t>(L.n) * (kG * kE * 8) > kRpMaxBytes)
     return hipErrorInvalidValue;
   static bool attr = false;
   if (!attr) {
@@ -1880,22 +1886,22 @@ struct FpWords;
 template <>
 struct FpWords<float> {
   static constexpr int k16 = 4;  // values in 16 bytes
-  static __device__ __forceinline__ float load(__amdgpu_buffer_rsrc_t b, int v, int s) {
-    return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(b, v, s, 0));
+  static __device__ __forceinline__ float load(__amdgpu_buffer_rsrc_t b, int v) {
+    return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(b, v, 0, 0));
   }
-  static __device__ __forceinline__ void store(float x, __amdgpu_buffer_rsrc_t b, int v, int s) {
-    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(x), b, v, s, 0);
+  static __device__ __forceinline__ void store(float x, __amdgpu_buffer_rsrc_t b, int v) {
+    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(x), b, v, 0, 0);
   }
 };
 using RpWord2 = __attribute__((ext_vector_type(2))) unsigned;
 template <>
 struct FpWords<double> {
   static constexpr int k16 = 2;
-  static __device__ __forceinline__ double load(__amdgpu_buffer_rsrc_t b, int v, int s) {
-    return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(b, v, s, 0));
+  static __device__ __forceinline__ double load(__amdgpu_buffer_rsrc_t b, int v) {
+    return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(b, v, 0, 0));
   }
-  static __device__ __forceinline__ void store(double x, __amdgpu_buffer_rsrc_t b, int v, int s) {
-    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(RpWord2, x), b, v, s, 0);
+  static __device__ __forceinline__ void store(double x, __amdgpu_buffer_rsrc_t b, int v) {
+    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(RpWord2, x), b, v, 0, 0);
   }
 };
 template <typename T>
@@ -1924,8 +1930,8 @@ struct RpfArgs {
 };
 
 struct RpfLane {
-  int code_off, val_off;  // its entries' byte offsets from the piece's first row's
-  int row_off;            // its row's byte offset in a vector
+  unsigned slot;          // its first entry's place from the piece's first row's
+  unsigned row_off;       // its row's byte offset from the piece's first row's
   int owner;              // its row for the row's first lane, else INT32_MAX
   unsigned put, get;      // LDS offsets: its products, the row's products
 };
@@ -1943,17 +1949,19 @@ __device__ __forceinline__ void rpf_load(RpfPre<T, kE, kFq>& r, int lo, int hi, 
   r.lo = lo;
   r.cnt = hi - lo;
   r.steps = steps;
-  const unsigned e = static_cast<unsigned>(lo) << a.lg;
-  const int ce = static_cast<int>(e * (kE * 4)), ve = static_cast<int>(e * (kE * kT));
+  // vector offsets, as in rp_load
+  const unsigned e = (static_cast<unsigned>(lo) << a.lg) * kE + ln.slot;
+  const int ce = static_cast<int>(e * 4), ve = static_cast<int>(e * kT);
+  const int row = static_cast<int>(static_cast<unsigned>(lo) * kT + ln.row_off);
 #pragma unroll
   for (int h = 0; h < kE / 4; ++h)
-    r.code[h] = __builtin_amdgcn_raw_buffer_load_b128(a.code, ln.code_off + 16 * h, ce, 0);
+    r.code[h] = __builtin_amdgcn_raw_buffer_load_b128(a.code, ce + 16 * h, 0, 0);
 #pragma unroll
   for (int h = 0; h < kE * kT / 16; ++h)
     r.val[h] = __builtin_bit_cast(
-        FpVec16<T>, __builtin_amdgcn_raw_buffer_load_b128(a.val, ln.val_off + 16 * h, ve, 0));
-  r.dinv = FpWords<T>::load(a.dinv, ln.row_off, lo * kT);
-  r.in = FpWords<T>::load(a.in, ln.row_off, lo * kT);
+        FpVec16<T>, __builtin_amdgcn_raw_buffer_load_b128(a.val, ve + 16 * h, 0, 0));
+  r.dinv = FpWords<T>::load(a.dinv, row);
+  r.in = FpWords<T>::load(a.in, row);
 }
 
 template <typename T>
@@ -2001,7 +2009,7 @@ __device__ __forceinline__ void rpf_level(RpfPre<T, kE, kFq>& cur, RpfPre<T, kE,
     for (int q = 0; q < kFq; ++q) {
       // ~code is the byte offset of a far entry's value, else past the end
       const unsigned c = ahead.code[q / 4][q % 4];
-      ahead.xfar[q] = FpWords<T>::load(a.out, static_cast<int>(~c), 0);
+      ahead.xfar[q] = FpWords<T>::load(a.out, static_cast<int>(~c));
     }
   }
   if (!kTail) {
@@ -2054,9 +2062,9 @@ __device__ __forceinline__ void rpf_level(RpfPre<T, kE, kFq>& cur, RpfPre<T, kE,
   }
   const T v = t * cur.dinv;
   if (ln.owner < cur.cnt) {
-    const int lob = cur.lo * kT;
-    *fp_lds<T>(static_cast<unsigned>(lob + ln.row_off) & a.ring_mask) = v;
-    FpWords<T>::store(v, a.out, ln.row_off, lob);
+    const unsigned row = static_cast<unsigned>(cur.lo) * kT + ln.row_off;
+    *fp_lds<T>(row & a.ring_mask) = v;
+    FpWords<T>::store(v, a.out, static_cast<int>(row));
   }
   // as in rp_level
   if (kFq > 0 && (L & a.fence_mask) == a.fence_mask)
@@ -2113,9 +2121,8 @@ __global__ __launch_bounds__(64 * kMaxWaves) void k_tri_chain_rpf(
                   lg, fence - 1};
   const int row = t >> lg, lane = t & (lanes - 1);
   RpfLane ln;
-  ln.code_off = t * (kE * 4);
-  ln.val_off = t * (kE * kT);
-  ln.row_off = row * kT;
+  ln.slot = static_cast<unsigned>(t) * kE;
+  ln.row_off = static_cast<unsigned>(row) * kT;
   ln.owner = lane == 0 ? row : INT32_MAX;
   ln.get = static_cast<unsigned>(stage + row * row_bytes);
   ln.put = ln.get + static_cast<unsigned>(lane * kE * kT);
@@ -2143,7 +2150,7 @@ hipError_t tri_rpf_go(const TriLayout& L, const T* in, T* out, hipStream_t s) {
   while ((1 << lg) < L.rp_lanes) ++lg;
   if (lds > static_cast<size_t>(kTriBlockedMaxLds) || L.n <= 0 || L.rp_fence < 1 ||
       (1 << lg) != L.rp_lanes || (L.rp_lanes > 1) != kLanes ||
-      static_cast<uint64_t>(L.n) * L.rp_lanes * kE * sizeof(T) > UINT32_MAX)
+      static_cast<uint64_t>(L.n) * L.rp_lanes * kE * sizeof(T) > kRpMaxBytes)
     return hipErrorInvalidValue;
   auto kern = &k_tri_chain_rpf<T, kMaxWaves, kLanes, kE, kD, kA, kFq>;
   static bool attr = false;
