@@ -371,6 +371,22 @@ bool segmented_wins(const std::vector<int>& lev_ptr, int single_wg_max, double c
   return wide && segmented <= cost;
 }
 
+// What the entry-parallel kernel takes for a chain's levels, in ns, from its
+// mean entries and rows per level: fitted to its solves of 27-point 48^3, 64^3
+// and 80^3, 7-point 63^3 and 48^3-inclusions SOR hierarchies and the 27-point
+// 64^3 BlockSOR one.  92 entries in 8 rows took 354 ns, 166 in 13: 558, 728 in
+// 21: 729, 1,226 in 36: 844, 3,265 in 104: 1,312, 3,898 in 448: 2,340.
+double ep_cost(int levels, double entries, double rows) {
+  return levels * (entries <= 100 ? 360 : 480 + 0.17 * entries + 2.7 * rows);
+}
+
+// The row-parallel kernel's cost for that comparison: plan_rp's, but at least
+// what a workgroup needs to read a piece's entries, 512 bytes per wave and slot
+// at 72 GB/s (8 waves of 8 / 12: 546 / 697 ns, 6 of 8 / 12: 358 / 500).
+double rp_cost_of(long long pieces, int waves, int e, double piece_cost) {
+  return static_cast<double>(pieces) * std::max(piece_cost, 7.1 * waves * e);
+}
+
 // Row-parallel layout of an integer smoother factor (k_tri_chain_rp).
 //
 // A level is cut into pieces of at most 64 waves / lanes rows (rows of a level
@@ -381,12 +397,13 @@ bool segmented_wins(const std::vector<int>& lev_ptr, int single_wg_max, double c
 // are the launch's, each further wave 20 / 47 ns for its barrier and its share
 // of the CU's load bandwidth).  The layout with the least total over the
 // longest chain wins; so narrow levels get one wave, which needs no barrier,
-// and wide ones several.
-void plan_rp(TriPlan& plan, int n, const std::vector<int>& lbeg, const std::vector<int>& lpos,
-             const std::vector<int32_t>& lval, const std::vector<int>& lev_ptr,
-             const std::vector<int>& chain_lev, long long span, int single_wg_max) {
+// and wide ones several.  Returns the layout's cost in ns (0: one that was
+// asked for by name, or none).
+double plan_rp(TriPlan& plan, int n, const std::vector<int>& lbeg, const std::vector<int>& lpos,
+               const std::vector<int32_t>& lval, const std::vector<int>& lev_ptr,
+               const std::vector<int>& chain_lev, long long span, int single_wg_max) {
   const char* env_rp = std::getenv("SC23AD_TRI_RP");
-  if ((env_rp && env_rp[0] == '0') || n <= 0 || n >= (1 << 29)) return;
+  if ((env_rp && env_rp[0] == '0') || n <= 0 || n >= (1 << 29)) return 0;
   const bool one_lane = env_rp && env_rp[0] == '1';
   const bool force_groups = env_rp && env_rp[0] == '2';  // lanes per row even for short rows
   const bool pow2 = std::getenv("SC23AD_RP_POW2") != nullptr;
@@ -400,7 +417,7 @@ void plan_rp(TriPlan& plan, int n, const std::vector<int>& lbeg, const std::vect
   const int nlev = static_cast<int>(lev_ptr.size()) - 1;
   // the kernel keeps negated values
   for (int32_t v : lval)
-    if (v == INT32_MIN) return;
+    if (v == INT32_MIN) return 0;
   // LDS ring: a dependency is read from it when no later position of its
   // level's end has overwritten it, else (at least kEpFarLevels levels back)
   // from global memory
@@ -423,7 +440,7 @@ void plan_rp(TriPlan& plan, int n, const std::vector<int>& lbeg, const std::vect
       }
     farq = std::max(farq, c);
   }
-  if (farq > 0 && far_dist < dev::kEpFarLevels) return;
+  if (farq > 0 && far_dist < dev::kEpFarLevels) return 0;
   auto pieces_of = [&](size_t chain, int cap) {
     long long k = 0;
     for (int Lv = chain_lev[2 * chain]; Lv < chain_lev[2 * chain + 1]; ++Lv)
@@ -464,9 +481,9 @@ void plan_rp(TriPlan& plan, int n, const std::vector<int>& lbeg, const std::vect
         }
       }
     }
-  if (best_w == 0) return;
-  if (nchain == 1 && segmented_wins(lev_ptr, single_wg_max, best)) return;
-  const std::vector<int> piece_ptr = put_pieces(plan, lev_ptr, chain_lev, 64 * best_w / best_g);
+  if (best_w == 0) return 0;
+  if (nchain == 1 && segmented_wins(lev_ptr, single_wg_max, best)) return 0;
+  put_pieces(plan, lev_ptr, chain_lev, 64 * best_w / best_g);
   std::vector<int> rent(static_cast<size_t>(n) * best_g * best_e * 2, 0);
   std::vector<int> ord;
   for (int idx = 0; idx < n; ++idx) {
@@ -499,6 +516,8 @@ void plan_rp(TriPlan& plan, int n, const std::vector<int>& lbeg, const std::vect
   L.rp_waves = best_w;
   L.rp_farq = farq;
   plan.nlaunch = 1;
+  if (env_rp || only_lanes > 0 || only_waves > 0) return 0;
+  return rp_cost_of(best_pieces, best_w, best_e, best / static_cast<double>(best_pieces));
 }
 
 // Row-parallel layout of an FP smoother factor (k_tri_chain_rpf): as plan_rp,
@@ -810,11 +829,10 @@ void build_plan(TriPlan& plan, TriKind kind, int n, const std::vector<int>& rptr
   L.n = n;
   // Row-parallel mode (integer smoother factors): lanes per row, entries per
   // lane and waves chosen by plan_rp; SC23AD_TRI_RP=0 keeps the other kernels.
+  double rp_cost = 0;
   if constexpr (std::is_same_v<V, int32_t>) {
-    if (kind == TriKind::kLD && plan.identity) {
-      std::vector<int> chains = chain_lev;
-      plan_rp(plan, n, lbeg, lpos, lval, lev_ptr, chains, span, single_wg_max);
-    }
+    if (kind == TriKind::kLD && plan.identity)
+      rp_cost = plan_rp(plan, n, lbeg, lpos, lval, lev_ptr, chain_lev, span, single_wg_max);
   }
   // Entry-parallel mode (integer factors): a dependency is read from the LDS
   // ring when the ring holds it, else from global memory, which needs it at
@@ -846,7 +864,20 @@ void build_plan(TriPlan& plan, TriKind kind, int n, const std::vector<int>& rptr
                     dev::kTriBlockedMaxLds)
     copies = false;
   const int ep_acc = copies ? acc_rows * dev::kEpCopies : dev::kEpMaxRows;
-  if (std::is_same_v<V, int32_t> && L.rp_waves == 0 && plan.identity && one_launch_chains &&
+  // Beside a row-parallel layout, for single vectors, where a few long rows
+  // make every piece of that one expensive (the entry-parallel kernel's work is
+  // the entries', not the longest row's): 27-point 64^3 SOR, levels 3 to 7,
+  // longest row 163-238 for a mean of 9-34, took 1,308 / 952 / 468 / 250 / 121
+  // us row-parallel, 1,135 / 762 / 412 / 221 / 86 entry-parallel.  Blocks of
+  // right-hand sides keep the row-parallel one, a workgroup for each, where the
+  // other would take them one by one.
+  const double per_level = static_cast<double>(std::max<size_t>(all_chain_lev.size() / 2, 1)) *
+                           std::max(maxlev_chain, 1);
+  const bool ep_first =
+      rp_cost > 0 && ep_cost(maxlev_chain, static_cast<double>(offdiag) / per_level,
+                             n / per_level) < rp_cost;
+  if (std::is_same_v<V, int32_t> && (L.rp_waves == 0 || ep_first) && plan.identity &&
+      one_launch_chains &&
       maxlev_rows <= static_cast<size_t>(dev::kEpMaxRows) &&
       dev::ep_lds_bytes(ep_ring, maxlev_chain, ep_acc) <= dev::kTriBlockedMaxLds) {
     std::vector<int> lev_of(static_cast<size_t>(std::max(n, 1)), 0);
@@ -905,6 +936,7 @@ void build_plan(TriPlan& plan, TriKind kind, int n, const std::vector<int>& rptr
       // every row of a level and about as many entries.
       L.ep_narrow = (maxlev_rows <= static_cast<size_t>(w) * 64 && overflowing(w, 4) * 16 <= nlev)
                         ? 1 : 0;
+      L.ep_first = ep_first;
     }
   }
   // FP smoother factors (solvers 0 and 1): plan_rpf; SC23AD_TRI_RP=0 keeps
@@ -920,11 +952,12 @@ void build_plan(TriPlan& plan, TriKind kind, int n, const std::vector<int>& rptr
                  "[sc23ad plan] kind %d n %d nnz %zu chains %d levels(max chain) %d "
                  "max level rows %zu launches %d ring %d span %lld max deps %d ep waves %d far %d "
                  "narrow %d copies %d rp waves %d entries %d rows 1 lanes %d identity %d "
-                 "| rp: pieces %d far %d fence %d\n",
+                 "| rp: pieces %d far %d fence %d%s\n",
                  static_cast<int>(kind), n, cind.size(), nchain, plan.nlevels, maxlev_rows,
                  plan.nlaunch, L.ring, span, maxdeps, L.ep_waves, L.ep_far, L.ep_narrow,
                  L.ep_copies, L.rp_waves, L.rp_e, L.rp_lanes, plan.identity ? 1 : 0,
-                 L.rp_maxlev, L.rp_farq, L.rp_fence);
+                 L.rp_maxlev, L.rp_farq, L.rp_fence,
+                 L.ep_first ? " | single vectors: entry-parallel" : "");
   }
 }
 
@@ -1429,7 +1462,7 @@ void DevAmg::trsv(const TriPlan& plan, const DevMat& m, const void* in, void* ou
               "trsv blocked");
     return;
   }
-  if (plan.layout.rp_waves > 0 && elem == Elem::kI32) {
+  if (plan.layout.rp_waves > 0 && !plan.layout.ep_first && elem == Elem::kI32) {
     hip_check(dev::launch_trsv_rp(plan.layout, m.d.bit, m.d.dbit, in, out, lib_stream()),
               "trsv rp");
     return;

@@ -111,8 +111,8 @@ struct TriLayout {
   int ep_acc = 0;    // accumulator slots in LDS
   // row-parallel mode (LD factors with short rows): rp_lanes lanes per row,
   // each holding rp_e entries (int2 {code, -val}, padded, see k_tri_chain_rp)
-  // of its row, rp_waves waves per chain; its own levels (pieces of the level schedule's), chains
-  // and ring, and the far rule of the entry-parallel mode
+  // of its row, rp_waves waves per chain; its own levels (pieces of the level
+  // schedule's), chains and ring, and the far rule of the entry-parallel mode
   const void* rent = nullptr;
   const int* rp_lev = nullptr;
   const int* rp_chain = nullptr;
@@ -121,6 +121,7 @@ struct TriLayout {
   int rp_ring = 0;
   int rp_fence = 1;   // levels between full fences (power of two; far entries only)
   int rp_waves = 0;  // > 0: use the row-parallel kernel
+  bool ep_first = false;  // ... except for single vectors: the entry-parallel one
   int rp_e = 0;
   int rp_lanes = 1;
   int rp_farq = 0;   // leading slots per row that can hold a far entry

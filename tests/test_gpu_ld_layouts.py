@@ -18,19 +18,19 @@ from helpers import export
 pytestmark = pytest.mark.gpu
 
 LAYOUT = re.compile(r"\[sc23ad plan\] kind 0 n (\d+) .*rp waves (\d+) entries (\d+) rows \d+ "
-                    r"lanes (\d+) .*rp: pieces (\d+)")
-
-
+                    r"lanes (\d+) .*rp: pieces (\d+) far (\d+) fence \d+(.*)")
 
 def _check(a, smoother, monkeypatch, capfd, prec=S.INT):
-    """LD solves of every level against the oracle; the layouts picked."""
+    """LD solves of every level against the oracle; the layouts picked: (rows,
+    waves, entries, lanes, pieces, far entries, single vectors entry-parallel)."""
     monkeypatch.setenv("SC23AD_VERBOSE", "1")
     a.lmax1_scaling(np.zeros(a.n))
     h = S.Hierarchy(a, prec, S.amg_param(smoother))
     capfd.readouterr()
     amg = S.Amg(h)
-    plans = [tuple(map(int, m.groups())) for m in LAYOUT.finditer(capfd.readouterr().err)]
-    print("[ld layouts] (n, waves, entries, lanes, pieces):", plans, flush=True)
+    plans = [(*map(int, m.groups()[:-1]), "entry-parallel" in m.group(7))
+             for m in LAYOUT.finditer(capfd.readouterr().err)]
+    print("[ld layouts] (n, waves, entries, lanes, pieces, far, ep):", plans, flush=True)
     path = export(h)
     try:
         oh = O.OracleHier(path)
@@ -58,6 +58,25 @@ def _check(a, smoother, monkeypatch, capfd, prec=S.INT):
 def test_layouts_of_the_plan(kind, params, smoother, waves, lanes, monkeypatch, capfd):
     plans = _check(S.CsrMat.generate(kind, *params), smoother, monkeypatch, capfd)
     assert max(p[1] for p in plans) >= waves and max(p[3] for p in plans) >= lanes
+
+
+def test_entry_parallel_where_few_rows_are_long(monkeypatch, capfd):
+    """27-point SOR levels whose longest row is many times their mean: single
+    vectors take the entry-parallel kernel, blocks the row-parallel one."""
+    a = S.CsrMat.generate(S.GEN_DIFFUSION27, 64, 8, 1.0, 1.0, 1e-3, 2)
+    plans = _check(a, S.SOR, monkeypatch, capfd)
+    assert not plans[0][6] and any(p[6] for p in plans)
+    assert all(p[1] > 0 for p in plans)
+    h = S.Hierarchy(a, S.INT, S.amg_param(S.SOR))
+    path = export(h)
+    amg, oh = S.Amg(h), O.OracleHier(path)
+    os.unlink(path)
+    assert S.block_native(amg)
+    v = np.random.default_rng(3).integers(-2**29, 2**29, (2, a.n)).astype(np.int32)
+    out = S.precondition_block(amg, v)
+    for k in range(2):
+        assert np.array_equal(out[k], oh.vcycle(v[k]))
+        assert np.array_equal(out[k], amg.precondition(v[k]))
 
 
 @pytest.mark.parametrize("lanes", [1, 2, 4, 8, 16, 32, 64])
