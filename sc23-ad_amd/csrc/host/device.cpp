@@ -371,6 +371,18 @@ bool segmented_wins(const std::vector<int>& lev_ptr, int single_wg_max, double c
   return wide && segmented <= cost;
 }
 
+// Whether a row-parallel layout of `slots` padded entries per row takes too
+// much memory: more than 192 slots, 64 MB and 32 times the factor's own
+// entries.  A single row decides the slots of every row, so one of 600 entries
+// among 300,000 of 15 would take 1.5 GB (43 times) on the host and the GPU and
+// be streamed by every solve.  27-point SOR hierarchies, whose coarse levels
+// have the longest rows for their mean, reach 28 times at 5 MB.
+bool padded_too_far(int n, int slots, size_t entries, size_t entry_bytes) {
+  const double padded = static_cast<double>(n) * slots;
+  return slots > 192 && padded * static_cast<double>(entry_bytes) > 64.0 * (1 << 20) &&
+         padded > 32.0 * static_cast<double>(entries);
+}
+
 // What the entry-parallel kernel takes for a chain's levels, in ns, from its
 // mean entries and rows per level: fitted to its solves of 27-point 48^3, 64^3
 // and 80^3, 7-point 63^3 and 48^3-inclusions SOR hierarchies and the 27-point
@@ -455,7 +467,8 @@ double plan_rp(TriPlan& plan, int n, const std::vector<int>& lbeg, const std::ve
     for (int e : {4, 6, 8, 10, 12}) {
       const int g = 1 << lg;
       if (g * e < md || (g == 1 && e == 6) ||
-          static_cast<uint64_t>(n) * (g * e * 8) > dev::kRpMaxBytes)
+          static_cast<uint64_t>(n) * (g * e * 8) > dev::kRpMaxBytes ||
+          padded_too_far(n, g * e, lpos.size(), 8))
         continue;
       // far entries over several lanes: 8 entries or more, kRpFarSlots far ones
       if (farq > 0 && g > 1 && (e < 8 || farq > dev::kRpFarSlots * g)) continue;
@@ -578,7 +591,8 @@ void plan_rpf(TriPlan& plan, int n, const std::vector<int>& lbeg, const std::vec
   for (int g = 1; g <= 64; g *= 2)
     for (int e : {4, 8}) {
       if (g * e < md || (only_lanes > 0 && g != only_lanes) ||
-          static_cast<uint64_t>(n) * g * e * kT > dev::kRpMaxBytes)
+          static_cast<uint64_t>(n) * g * e * kT > dev::kRpMaxBytes ||
+          padded_too_far(n, g * e, lpos.size(), 4 + kT))
         continue;
       for (int w = 1; w <= 8; ++w) {
         if (only_waves > 0 && w != only_waves) continue;

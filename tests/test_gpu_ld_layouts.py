@@ -79,6 +79,27 @@ def test_entry_parallel_where_few_rows_are_long(monkeypatch, capfd):
         assert np.array_equal(out[k], amg.precondition(v[k]))
 
 
+@pytest.mark.parametrize("prec", [S.INT, S.FP64, S.FP32], ids=["int", "fp64", "fp32"])
+def test_one_long_row_is_not_padded_to(prec, monkeypatch, capfd):
+    """A 5-point system of 48,400 rows whose last row has 400 entries more (in
+    its BlockSOR block): a layout padded to it would take 200-300 MB for 1-2 MB of
+    entries."""
+    n = 220 * 220
+    rptr, cind, val = S.CsrMat.generate(S.GEN_POISSON2D, 220).arrays()
+    rng = np.random.default_rng(17)
+    old = cind[rptr[n - 1]:]
+    extra = np.setdiff1d(n - 1200 + rng.choice(1199, 400, replace=False), old).astype(np.int32)
+    cols = np.concatenate([old, extra])
+    vals = np.concatenate([val[rptr[n - 1]:], np.full(len(extra), -2.0**-9)])
+    order = np.argsort(cols)
+    rptr = rptr.copy()
+    rptr[n] += len(extra)
+    a = S.CsrMat.from_arrays(n, rptr, np.concatenate([cind[:len(cind) - len(old)], cols[order]]),
+                             np.concatenate([val[:len(val) - len(old)], vals[order]]))
+    plans = _check(a, S.BLOCK_SOR, monkeypatch, capfd, prec)
+    assert plans[0][0] == n and plans[0][1] == 0
+
+
 @pytest.mark.parametrize("lanes", [1, 2, 4, 8, 16, 32, 64])
 @pytest.mark.parametrize("waves", [1, 3])
 def test_forced_layouts(lanes, waves, monkeypatch, capfd):
