@@ -249,7 +249,9 @@ int sc23ad_solve_batch(int count, sc23ad_solver* const* solvers, const double* c
 typedef struct sc23ad_block_solver_s sc23ad_block_solver;
 /* One V-cycle on nrhs vectors in the block layout: element (row i, vector r)
    at ((r / 4) * n + i) * 4 + r % 4 (int32; ceil(nrhs / 4) * 4 * n words).
-   Integer hierarchies only. */
+   Integer hierarchies only.  The hierarchy keeps the work vectors of its
+   widest call (about 8 block vectors) until sc23ad_amg_destroy; a call that
+   overlaps another one allocates its own for its duration. */
 int sc23ad_amg_precondition_block(sc23ad_amg* m, int nrhs, const int32_t* in, int32_t* out,
                                   int on_device);
 /* Mean duration of `reps` back-to-back block V-cycles on nrhs device

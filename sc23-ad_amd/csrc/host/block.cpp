@@ -16,7 +16,7 @@ using dev::SpmvMode;
 std::unique_ptr<DevAmg::BlockWork> DevAmg::make_block_work(int groups) const {
   if (elem != Elem::kI32) throw DevError{1, "block V-cycle: integer hierarchies only"};
   auto w = std::make_unique<BlockWork>();
-  w->groups = groups;
+  w->groups = w->capacity = groups;
   const size_t row = 16 * static_cast<size_t>(groups);  // bytes of one block row
   w->ee.resize(depth + 1);
   w->xx.resize(depth + 1);
@@ -162,20 +162,25 @@ void DevAmg::check_errors(BlockWork& w) const {
 }
 
 std::unique_ptr<DevAmg::BlockWork> DevAmg::take_block_work(int groups) {
+  std::unique_ptr<BlockWork> w;
   {
     std::lock_guard<std::mutex> lock(idle_mutex_);
-    if (idle_ && idle_->groups == groups) return std::move(idle_);
+    w = std::move(idle_);
   }
-  auto w = make_block_work(groups);
+  if (w && w->capacity >= groups) {
+    w->groups = groups;
+    return w;
+  }
+  w.reset();  // too small: freed before the larger one is allocated
+  w = make_block_work(groups);
   w->host_err.alloc();
   return w;
 }
 
 void DevAmg::give_block_work(std::unique_ptr<BlockWork> w) {
-  std::unique_ptr<BlockWork> old;  // freed after the lock is dropped
   std::lock_guard<std::mutex> lock(idle_mutex_);
-  old = std::move(idle_);
-  idle_ = std::move(w);
+  if (!idle_ || idle_->capacity < w->capacity) std::swap(idle_, w);
+  // the other one, if any, is freed with w, after the lock is dropped
 }
 
 // ---------------------------------------------------------------------------

@@ -226,7 +226,8 @@ class DevAmg {
   // Vectors hold element (row i, right-hand side r) at ((r / 4) * n + i) * 4
   // + r % 4 (see block.hip).  One BlockWork per concurrent block user.
   struct BlockWork {
-    int groups = 0;
+    int groups = 0;    // of the call
+    int capacity = 0;  // groups that the buffers hold; any fewer fit in them too
     std::vector<DevBuf> ee, xx, rr, tmp;   // per level (1..depth); tmp[0] fine
     DevBuf r0, vin0, vout0, tmpc;
     DevBuf lflags, uflags, tickets, err;   // tiled coarse solves
@@ -236,9 +237,10 @@ class DevAmg {
   };
   std::unique_ptr<BlockWork> make_block_work(int groups) const;
   // A work context for a preconditioner call, which hands it back once its
-  // stream is idle.  One idle context is kept per hierarchy (allocating one
-  // took 3.9 of the 6.8 ms of a 16-vector call at 96^3); callers that overlap
-  // each get their own.
+  // stream is idle.  One idle context is kept per hierarchy, the widest so far
+  // (allocating one took 3.9 of the 6.8 ms of a 16-vector call at 96^3), and
+  // serves calls of any width up to its own; callers that overlap each get
+  // their own.
   std::unique_ptr<BlockWork> take_block_work(int groups);
   void give_block_work(std::unique_ptr<BlockWork> w);
   void vcycle_blk(const void* in, void* out, BlockWork& w) const;

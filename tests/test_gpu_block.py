@@ -18,6 +18,7 @@ import os
 
 import numpy as np
 import pytest
+import torch
 
 import oracle as O
 import sc23ad as S
@@ -74,6 +75,27 @@ def test_block_vcycle_matches_oracle(golden, case, smoother, k):
     # twice: no state left behind between calls
     outs2 = S.precondition_block(amg, vins[::-1].copy())
     assert np.array_equal(outs2, outs[::-1])
+
+
+def test_block_workspace_serves_narrower_calls():
+    """The work vectors of the widest call stay with the hierarchy and serve
+    narrower ones: no memory moves when full and ragged blocks alternate (the
+    vectors of 16 right-hand sides take about 50 MB here, of 3 a quarter), and
+    neither width finds anything of the other's."""
+    a = _scaled(S.GEN_LAPLACE3D, (48,))
+    h = S.Hierarchy(a, S.INT, S.amg_param(S.BLOCK_SOR))
+    amg, oh = S.Amg(h), _oracle(h)
+    v = np.random.default_rng(9).integers(-(2**29), 2**29, (16, a.n)).astype(np.int32)
+    want = [oh.vcycle(x) for x in v]
+    free = []
+    for k in (3, 16, 3, 16, 5):
+        out = S.precondition_block(amg, v[16 - k:])
+        for r in range(k):
+            assert np.array_equal(out[r], want[16 - k + r]), (k, r)
+        free.append(torch.cuda.mem_get_info()[0] >> 20)
+    print(f"[block workspace] MiB free after each call {free}", flush=True)
+    assert free[0] - free[1] > 24  # grown once
+    assert max(free[1:]) - min(free[1:]) <= 4
 
 
 def _compare_block_with_singles(a, hi, hd, bs, nrms, m, eps, bits=None, seq_check=True):
