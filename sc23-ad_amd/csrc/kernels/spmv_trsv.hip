@@ -2523,8 +2523,16 @@ bool trsv_rp_blk_supported(const TriLayout& L) {
 hipError_t launch_trsv_rp_blk(const TriLayout& L, int groups, int bit, int dbit, const void* in,
                               void* out, hipStream_t s) {
   if (!trsv_rp_blk_supported(L)) return hipErrorInvalidValue;
-  return trsv_rp_waves<4>(L, 4 * groups, bit, dbit, static_cast<const int32_t*>(in),
-                          static_cast<int32_t*>(out), s);
+  // a right-hand side per workgroup in y, whose grids have at most 65,535
+  constexpr int kSlice = 65535 / 4;
+  for (int g0 = 0; g0 < groups; g0 += kSlice) {
+    const size_t off = static_cast<size_t>(g0) * L.n * 4;
+    const hipError_t e =
+        trsv_rp_waves<4>(L, 4 * std::min(kSlice, groups - g0), bit, dbit,
+                         static_cast<const int32_t*>(in) + off, static_cast<int32_t*>(out) + off, s);
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
 }
 
 hipError_t launch_trsv_rpf(Elem e, const TriLayout& L, const void* in, void* out,

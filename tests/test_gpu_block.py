@@ -98,6 +98,20 @@ def test_block_workspace_serves_narrower_calls():
     assert max(free[1:]) - min(free[1:]) <= 4
 
 
+def test_block_vcycle_of_more_vectors_than_a_grid_is_wide():
+    """65,541 right-hand sides: more than the 65,535 workgroups that one launch
+    has in y."""
+    k = 65541
+    a = _scaled(S.GEN_POISSON2D, (24,))
+    h = S.Hierarchy(a, S.INT, S.amg_param(S.SOR))
+    amg, oh = S.Amg(h), _oracle(h)
+    assert S.block_native(amg) and amg.depth >= 1
+    v = np.random.default_rng(10).integers(-(2**29), 2**29, (k, a.n)).astype(np.int32)
+    out = S.precondition_block(amg, v)
+    for r in (0, 1, 2, 3, 40000, 65530, 65531, 65532, 65535, 65536, 65539, 65540):
+        assert np.array_equal(out[r], oh.vcycle(v[r])), r
+
+
 def _compare_block_with_singles(a, hi, hd, bs, nrms, m, eps, bits=None, seq_check=True):
     amg_i = S.Amg(hi)
     if bits is None:
