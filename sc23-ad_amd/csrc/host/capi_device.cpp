@@ -141,12 +141,7 @@ int sc23ad_spmv_int(int n, const int* rptr, const int* cind, const int32_t* val,
     a.cind = cind;
     a.val = val;
     a.bit = bit;
-    // streamed, with fewer rows per workgroup where 128 leave CUs idle (the
-    // row lengths are not known here)
-    a.stream = n >= 128 * 512 ? 128 : n >= 32 * 512 ? 32 : 16;
-    hip_check(dev::launch_spmv(dev::Elem::kI32, a, dev::SpmvMode::kPlain, x, nullptr, y,
-                               lib_stream()),
-              "spmv_int");
+    hip_check(dev::launch_spmv_rows_unknown(a, x, y, lib_stream()), "spmv_int");
     hip_check(hipStreamSynchronize(lib_stream()), "sync");
     return SC23AD_OK;
   });

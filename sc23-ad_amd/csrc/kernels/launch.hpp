@@ -63,6 +63,12 @@ enum class SpmvMode : int { kPlain = 0, kSub = 1, kAdd = 2 };
 //   kDU  inverse diagonal first, then the upper entries; solved backward (dutri)
 enum class TriKind : int { kLD = 0, kL = 1, kDU = 2 };
 
+// y = spmv(x) on integer CSR arrays whose row lengths nobody has looked at:
+// streamed, with fewer rows per workgroup where more leave CUs idle (65,536
+// rows of 3 / 200,000 of 7 entries: 128 rows 15 / 17 us a call, 32 rows 16 / 22;
+// 16,000 of 5: 16 rows 15, 4 rows 19; 100 of 50,000: 4 rows 175, 8 lanes per row
+// 748, but 100 of 5: 14.2 and 13.4).
+hipError_t launch_spmv_rows_unknown(const DCsr& a, const void* x, void* y, hipStream_t s);
 // y = spmv(x)  |  y = z - spmv(x)  |  y = z + spmv(x)   (y may alias z)
 hipError_t launch_spmv(Elem e, const DCsr& a, SpmvMode mode, const void* x,
                        const void* z, void* y, hipStream_t s);

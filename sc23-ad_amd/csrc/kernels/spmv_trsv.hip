@@ -107,7 +107,14 @@ __global__ __launch_bounds__(kBlock) void k_spmv_int(
 // clamped loads where a row is shorter than 8 G: with 8 lanes per row 79 us on
 // the 95^3 27-point operator and 134 us on the 128^3 7-point one, against 43
 // and 35 us here with 128 rows (4.5 and 4.1 TB/s).
-template <int kRows, int MODE>
+//
+// kLong (rows of unknown lengths): a row of more than 32 entries per lane would
+// hold up its workgroup, one LDS read after another by few lanes (65,536 rows
+// of 300: 140 us at two lanes per row; 100 rows of 50,000: 1,974).  A workgroup
+// that has one shares every tile's products among the rows that the tile
+// holds, up to all its lanes for one row, and adds the parts to the rows' sums
+// in LDS (60 and 175 us).
+template <int kRows, int MODE, bool kLong>
 __global__ __launch_bounds__(kBlock) void k_spmv_stream_int(
     int n, const int* __restrict__ rptr, const int* __restrict__ cind,
     const int32_t* __restrict__ val, int bit, const int32_t* __restrict__ x,
@@ -115,9 +122,25 @@ __global__ __launch_bounds__(kBlock) void k_spmv_stream_int(
   constexpr int kPer = 8, kTile = kBlock * kPer, kLanes = kBlock / kRows;
   __shared__ uint64_t prod[kTile];
   __shared__ int rp[kRows + 1];
+  __shared__ unsigned long long sums[kLong ? kRows : 1];
+  __shared__ int long_in[kBlock / 64];
   const int t = threadIdx.x;
   const int r0 = blockIdx.x * kRows, nr = min(kRows, n - r0);
-  for (int k = t; k <= nr; k += kBlock) rp[k] = rptr[r0 + k];
+  if constexpr (kLong) {
+    static_assert(kRows <= kBlock, "a row per thread");
+    bool mine = false;
+    if (t < nr) {
+      const int rb = rptr[r0 + t], re = rptr[r0 + t + 1];
+      rp[t] = rb;
+      if (t == nr - 1) rp[nr] = re;
+      sums[t] = 0;
+      mine = re - rb > 32 * kLanes;
+    }
+    const bool any = __any(mine);
+    if ((t & 63) == 0) long_in[t >> 6] = any;
+  } else {
+    for (int k = t; k <= nr; k += kBlock) rp[k] = rptr[r0 + k];
+  }
   const int row = t / kLanes, lane = t % kLanes;
   const int32_t zv = MODE != 0 && row < nr && lane == 0 ? z[r0 + row] : 0;
   __syncthreads();
@@ -136,6 +159,13 @@ __global__ __launch_bounds__(kBlock) void k_spmv_stream_int(
     }
   };
   if (e0 < e1) load(e0);
+  bool any_long = false;
+  if constexpr (kLong) {
+    int any = 0;
+#pragma unroll
+    for (int k = 0; k < kBlock / 64; ++k) any |= long_in[k];
+    any_long = __builtin_amdgcn_readfirstlane(any) != 0;
+  }
   bool more = e0 < e1;
   for (int p0 = e0; more; p0 += kTile) {
     more = e1 - p0 > kTile;
@@ -146,11 +176,36 @@ __global__ __launch_bounds__(kBlock) void k_spmv_stream_int(
     for (int j = 0; j < kPer; ++j) prod[t + kBlock * j] = prod64(vv[j], xx[j]);
     if (more) load(p0 + kTile);
     lds_barrier();
-    const int lo = max(b - p0, 0), hi = min(e - p0, kTile);
-    for (int q = lo + lane; q < hi; q += kLanes) acc += prod[q];
+    if (!kLong || !any_long) {
+      const int lo = max(b - p0, 0), hi = min(e - p0, kTile);
+      for (int q = lo + lane; q < hi; q += kLanes) acc += prod[q];
+    } else {
+      // rows that end after p0 from the first on, and those that begin in the tile
+      int first = 0, last = 0;
+#pragma unroll
+      for (int k = 0; k < kRows; k += 64) {
+        const int r = min(k + (t & 63), nr - 1);
+        const bool mine = k + (t & 63) < nr;
+        first += __popcll(__ballot(mine && rp[r + 1] <= p0));
+        last += __popcll(__ballot(mine && rp[r] - p0 < kTile));
+      }
+      // 2^lg lanes for each of them (at least kLanes: there are kRows at most)
+      const int lg = 31 - __clz(kBlock / (last - first));
+      const int g = t >> lg, part = t & ((1 << lg) - 1);
+      const int mine = min(first + g, nr - 1);
+      const int lo = max(rp[mine] - p0, 0);
+      const int hi = first + g < last ? min(rp[mine + 1] - p0, kTile) : 0;
+      uint64_t s = 0;
+      for (int q = lo + part; q < hi; q += 1 << lg) s += prod[q];
+      for (int o = 1; o < min(1 << lg, 64); o *= 2) s += __shfl_xor(s, o, 64);
+      if ((part & 63) == 0 && lo < hi) atomicAdd(&sums[mine], s);
+    }
     lds_barrier();
   }
-  acc = group_sum<kLanes>(acc);
+  if (kLong && any_long) acc = lane == 0 && row < nr ? sums[row] : 0;
+  acc = group_sum<(kLanes < 16 ? kLanes : 16)>(acc);
+#pragma unroll
+  for (int o = 16; o < kLanes; o *= 2) acc += __shfl_xor(acc, o, 64);
   if (row < nr && lane == 0) {
     const int32_t s = low32(as_i64(acc) >> bit);
     if (MODE == 0) y[r0 + row] = s;
@@ -385,10 +440,10 @@ hipError_t spmv_int_g(const DCsr& a, const void* x, const void* z, void* y,
   return hipGetLastError();
 }
 
-template <int R, int MODE>
+template <int R, int MODE, bool kLong = false>
 hipError_t spmv_stream_go(const DCsr& a, const void* x, const void* z, void* y, hipStream_t s) {
   if (a.n <= 0) return hipSuccess;
-  launch_timed(&k_spmv_stream_int<R, MODE>, dim3((a.n + R - 1) / R), dim3(kBlock), 0, s, a.n,
+  launch_timed(&k_spmv_stream_int<R, MODE, kLong>, dim3((a.n + R - 1) / R), dim3(kBlock), 0, s, a.n,
                a.rptr, a.cind, static_cast<const int32_t*>(a.val), a.bit,
                static_cast<const int32_t*>(x), static_cast<const int32_t*>(z),
                static_cast<int32_t*>(y));
@@ -2350,6 +2405,13 @@ hipError_t spmv_sell_mode(const DCsr& a, int md, const void* x, const void* z, v
   if (md == 0) return spmv_sell<T, 0>(a, x, z, y, s);
   if (md == 1) return spmv_sell<T, 1>(a, x, z, y, s);
   return spmv_sell<T, 2>(a, x, z, y, s);
+}
+
+hipError_t launch_spmv_rows_unknown(const DCsr& a, const void* x, void* y, hipStream_t s) {
+  if (a.n >= 128 * 512) return spmv_stream_go<128, 0, true>(a, x, nullptr, y, s);
+  if (a.n >= 32 * 512) return spmv_stream_go<32, 0, true>(a, x, nullptr, y, s);
+  if (a.n >= 1024) return spmv_stream_go<16, 0, true>(a, x, nullptr, y, s);
+  return spmv_stream_go<4, 0, true>(a, x, nullptr, y, s);
 }
 
 hipError_t launch_spmv(Elem e, const DCsr& a, SpmvMode mode, const void* x,

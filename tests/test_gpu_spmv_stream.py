@@ -22,15 +22,43 @@ def _reference(rptr, cind, val, bit, x):
         return ((p[rptr[1:]] - p[rptr[:-1]]) >> bit).astype(np.int32)
 
 
-@pytest.mark.parametrize("n", [1, 15, 16, 17, 32 * 512 - 1, 32 * 512, 128 * 512, 128 * 512 + 77])
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 1023, 1024, 1041, 32 * 512 - 1, 32 * 512, 128 * 512, 128 * 512 + 77])
 def test_rows_per_workgroup(n):
-    """16, 32 and 128 rows per workgroup, by the number of rows."""
+    """4, 16, 32 and 128 rows per workgroup, by the number of rows."""
     rng = np.random.default_rng(n)
     lens = rng.integers(0, 12, n)
     lens[rng.integers(0, n, 3)] = [2047, 2048, 5001]
     lens[n // 3:n // 3 + 300] = 0
     rptr = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
     m = 3001
+    cind = rng.integers(0, m, rptr[-1]).astype(np.int32)
+    val = rng.integers(-2**31, 2**31, rptr[-1]).astype(np.int32)
+    x = rng.integers(-2**31, 2**31, m).astype(np.int32)
+    for bit in (0, 30):
+        assert np.array_equal(S.spmv_int(rptr, cind, val, bit, x),
+                              _reference(rptr, cind, val, bit, x)), bit
+
+
+@pytest.mark.parametrize("n", [1, 3, 4, 5, 1023, 1024, 32 * 512, 128 * 512 + 77])
+@pytest.mark.parametrize("kind", ["all long", "one", "every 50th", "around the bound"])
+def test_long_rows(n, kind):
+    """Rows of more than 32 entries per lane, whose workgroups share each tile's
+    products: alone, among short and empty rows, across many tiles, and rows of
+    exactly the bound and one more (64 to 2,048 entries)."""
+    rng = np.random.default_rng(n)
+    if kind == "all long":
+        lens = np.full(n, max(300, min(40000, 2000000 // n)) + n % 3)
+    else:
+        lens = rng.integers(0, 5, n)
+        if kind == "one":
+            lens[n // 2] = 100001
+        elif kind == "every 50th":
+            lens[::50] = rng.integers(300, 4000, len(lens[::50]))
+        else:
+            at = rng.permutation(n)[:64]
+            lens[at] = np.resize([64, 65, 256, 257, 512, 513, 2048, 2049], len(at))
+    rptr = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    m = 5003
     cind = rng.integers(0, m, rptr[-1]).astype(np.int32)
     val = rng.integers(-2**31, 2**31, rptr[-1]).astype(np.int32)
     x = rng.integers(-2**31, 2**31, m).astype(np.int32)
