@@ -399,6 +399,20 @@ double rp_cost_of(long long pieces, int waves, int e, double piece_cost) {
   return static_cast<double>(pieces) * std::max(piece_cost, 7.1 * waves * e);
 }
 
+// (tests) The smallest ring, at least `least` values, that holds every
+// dependency fewer than kEpFarLevels levels back: the rest are then far.
+int smallest_ring(int least, int n, const std::vector<int>& lbeg, const std::vector<int>& lpos,
+                  const std::vector<int>& lev_ptr, const std::vector<int>& lev_of) {
+  long long need = 1;
+  for (int idx = 0; idx < n; ++idx)
+    for (int q = lbeg[idx]; q < lbeg[idx + 1]; ++q)
+      if (lev_of[idx] - lev_of[lpos[q]] < dev::kEpFarLevels)
+        need = std::max(need, static_cast<long long>(lev_ptr[lev_of[idx] + 1]) - lpos[q]);
+  int r = least;
+  while (r < need) r *= 2;
+  return r;
+}
+
 // Row-parallel layout of an integer smoother factor (k_tri_chain_rp).
 //
 // A level is cut into pieces of at most 64 waves / lanes rows (rows of a level
@@ -419,13 +433,14 @@ double plan_rp(TriPlan& plan, int n, const std::vector<int>& lbeg, const std::ve
   const bool one_lane = env_rp && env_rp[0] == '1';
   const bool force_groups = env_rp && env_rp[0] == '2';  // lanes per row even for short rows
   const bool pow2 = std::getenv("SC23AD_RP_POW2") != nullptr;
-  // SC23AD_RP_LANES / SC23AD_RP_WAVES (tests): only layouts of so many lanes
-  // per row / waves
+  // SC23AD_RP_LANES / SC23AD_RP_ENTRIES / SC23AD_RP_WAVES (tests): only layouts
+  // of so many lanes per row / entries per lane / waves
   auto forced = [](const char* name) {
     const char* e = std::getenv(name);
     return e ? std::atoi(e) : 0;
   };
-  const int only_lanes = forced("SC23AD_RP_LANES"), only_waves = forced("SC23AD_RP_WAVES");
+  const int only_lanes = forced("SC23AD_RP_LANES"), only_waves = forced("SC23AD_RP_WAVES"),
+            only_entries = forced("SC23AD_RP_ENTRIES");
   const int nlev = static_cast<int>(lev_ptr.size()) - 1;
   // the kernel keeps negated values
   for (int32_t v : lval)
@@ -438,6 +453,8 @@ double plan_rp(TriPlan& plan, int n, const std::vector<int>& lbeg, const std::ve
   std::vector<int> lev_of(static_cast<size_t>(n));
   for (int Lv = 0; Lv < nlev; ++Lv)
     for (int idx = lev_ptr[Lv]; idx < lev_ptr[Lv + 1]; ++idx) lev_of[idx] = Lv;
+  if (std::getenv("SC23AD_RP_RING_FAR"))
+    ring = std::min(ring, smallest_ring(2, n, lbeg, lpos, lev_ptr, lev_of));
   auto is_far = [&](int idx, int dpos) {
     return static_cast<long long>(lev_ptr[lev_of[idx] + 1]) - dpos > ring;
   };
@@ -474,6 +491,7 @@ double plan_rp(TriPlan& plan, int n, const std::vector<int>& lbeg, const std::ve
       if (farq > 0 && g > 1 && (e < 8 || farq > dev::kRpFarSlots * g)) continue;
       if (g == 1 && force_groups && farq == 0 && md > 4) continue;
       if (only_lanes > 0 && g != only_lanes) continue;
+      if (only_entries > 0 && e != only_entries) continue;
       for (int w = 1; w <= dev::kRpMaxWaves; w = pow2 ? 2 * w : w + 1) {
         if (w > 8 && (g > 1 || e > 4)) break;
         const int cap = 64 * w / g;
@@ -529,7 +547,7 @@ double plan_rp(TriPlan& plan, int n, const std::vector<int>& lbeg, const std::ve
   L.rp_waves = best_w;
   L.rp_farq = farq;
   plan.nlaunch = 1;
-  if (env_rp || only_lanes > 0 || only_waves > 0) return 0;
+  if (env_rp || only_lanes > 0 || only_waves > 0 || only_entries > 0) return 0;
   return rp_cost_of(best_pieces, best_w, best_e, best / static_cast<double>(best_pieces));
 }
 
@@ -562,17 +580,8 @@ void plan_rpf(TriPlan& plan, int n, const std::vector<int>& lbeg, const std::vec
   // levels back, come from global memory
   int ring = 4;
   while (ring * 2 * kT <= 128 * 1024 && ring < span) ring *= 2;
-  if (std::getenv("SC23AD_FP_RING_FAR") && md > 8) {
-    // (tests) the smallest ring the far rule admits
-    long long need = 1;
-    for (int idx = 0; idx < n; ++idx)
-      for (int q = lbeg[idx]; q < lbeg[idx + 1]; ++q)
-        if (lev_of[idx] - lev_of[lpos[q]] < dev::kEpFarLevels)
-          need = std::max(need, static_cast<long long>(lev_ptr[lev_of[idx] + 1]) - lpos[q]);
-    int r = 4;
-    while (r < need) r *= 2;
-    ring = std::min(ring, r);
-  }
+  if (std::getenv("SC23AD_FP_RING_FAR"))
+    ring = std::min(ring, smallest_ring(4, n, lbeg, lpos, lev_ptr, lev_of));
   auto is_far = [&](int idx, int dpos) {
     return static_cast<long long>(lev_ptr[lev_of[idx] + 1]) - dpos > ring;
   };

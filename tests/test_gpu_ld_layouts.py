@@ -1,8 +1,9 @@
 """The row-parallel LD solves (k_tri_chain_rp, k_tri_chain_rpf) in the layouts
-that the plan picks at the ends of its range: one wave and 9-16 waves, 1-64 lanes per
-row, levels cut into pieces, a single chain with levels of more than 1,024
-rows, odd sizes.  Every LD solve equals the oracle's bit for bit (whole
-numbers: no tolerance)."""
+at the ends of the plan's range: one wave and 9-16 waves, 1-64 lanes per row,
+far dependencies over one and several lanes, levels cut into pieces, a single
+chain with levels of more than 1,024 rows, odd sizes; integer layouts on single
+vectors and on blocks.  Every LD solve equals the oracle's bit for bit (whole
+numbers, or FP sums in stored order: no tolerance)."""
 from __future__ import annotations
 
 import os
@@ -17,15 +18,22 @@ from helpers import export
 
 pytestmark = pytest.mark.gpu
 
+
 LAYOUT = re.compile(r"\[sc23ad plan\] kind 0 n (\d+) .*rp waves (\d+) entries (\d+) rows \d+ "
                     r"lanes (\d+) .*rp: pieces (\d+) far (\d+) fence \d+(.*)")
 
-def _check(a, smoother, monkeypatch, capfd, prec=S.INT):
+
+def _check(a, smoother, monkeypatch, capfd, prec=S.INT, block=0):
     """LD solves of every level against the oracle; the layouts picked: (rows,
-    waves, entries, lanes, pieces, far entries, single vectors entry-parallel)."""
-    monkeypatch.setenv("SC23AD_VERBOSE", "1")
+    waves, entries, lanes, pieces, far entries, single vectors entry-parallel).
+    block: V-cycles of so many vectors in one call too (integers)."""
     a.lmax1_scaling(np.zeros(a.n))
-    h = S.Hierarchy(a, prec, S.amg_param(smoother))
+    return _check_hierarchy(S.Hierarchy(a, prec, S.amg_param(smoother)), monkeypatch, capfd, prec,
+                            block)
+
+
+def _check_hierarchy(h, monkeypatch, capfd, prec, block):
+    monkeypatch.setenv("SC23AD_VERBOSE", "1")
     capfd.readouterr()
     amg = S.Amg(h)
     plans = [(*map(int, m.groups()[:-1]), "entry-parallel" in m.group(7))
@@ -47,6 +55,11 @@ def _check(a, smoother, monkeypatch, capfd, prec=S.INT):
             x[3::11] = 1e-310 if prec == S.FP64 else 1e-40
         y, yo = amg.level_op(lv, S.OP_TRSV_LD, x, n), oh.level_op(lv, S.OP_TRSV_LD, x, n)
         assert y.tobytes() == yo.tobytes(), lv
+    if block:
+        v = rng.integers(-2**29, 2**29, (block, oh.level_n(0))).astype(np.int32)
+        out = S.precondition_block(amg, v)
+        for k in range(block):
+            assert np.array_equal(out[k], oh.vcycle(v[k])), k
     return plans
 
 
@@ -64,19 +77,9 @@ def test_entry_parallel_where_few_rows_are_long(monkeypatch, capfd):
     """27-point SOR levels whose longest row is many times their mean: single
     vectors take the entry-parallel kernel, blocks the row-parallel one."""
     a = S.CsrMat.generate(S.GEN_DIFFUSION27, 64, 8, 1.0, 1.0, 1e-3, 2)
-    plans = _check(a, S.SOR, monkeypatch, capfd)
+    plans = _check(a, S.SOR, monkeypatch, capfd, block=2)
     assert not plans[0][6] and any(p[6] for p in plans)
     assert all(p[1] > 0 for p in plans)
-    h = S.Hierarchy(a, S.INT, S.amg_param(S.SOR))
-    path = export(h)
-    amg, oh = S.Amg(h), O.OracleHier(path)
-    os.unlink(path)
-    assert S.block_native(amg)
-    v = np.random.default_rng(3).integers(-2**29, 2**29, (2, a.n)).astype(np.int32)
-    out = S.precondition_block(amg, v)
-    for k in range(2):
-        assert np.array_equal(out[k], oh.vcycle(v[k]))
-        assert np.array_equal(out[k], amg.precondition(v[k]))
 
 
 @pytest.mark.parametrize("prec", [S.INT, S.FP64, S.FP32], ids=["int", "fp64", "fp32"])
@@ -105,15 +108,45 @@ def test_one_long_row_is_not_padded_to(prec, monkeypatch, capfd):
 def test_forced_layouts(lanes, waves, monkeypatch, capfd):
     monkeypatch.setenv("SC23AD_RP_LANES", str(lanes))
     monkeypatch.setenv("SC23AD_RP_WAVES", str(waves))
-    plans = _check(S.CsrMat.generate(S.GEN_DIFFUSION27, 17, 5, 1.0, 1.0, 1e-3, 3), S.SOR,
-                   monkeypatch, capfd)
-    assert any(p[1] == waves and p[3] == lanes for p in plans) or lanes == 1
+    a = (S.CsrMat.generate(S.GEN_POISSON2D, 67) if lanes == 1 else
+         S.CsrMat.generate(S.GEN_DIFFUSION27, 17, 5, 1.0, 1.0, 1e-3, 3))
+    plans = _check(a, S.SOR, monkeypatch, capfd, block=3)
+    assert any(p[1] == waves and p[3] == lanes for p in plans)
 
 
-def test_sixteen_waves(monkeypatch, capfd):
-    monkeypatch.setenv("SC23AD_RP_WAVES", "16")
-    plans = _check(S.CsrMat.generate(S.GEN_POISSON2D, 67), S.SOR, monkeypatch, capfd)
-    assert any(p[1] == 16 for p in plans)
+@pytest.mark.parametrize("waves", [9, 16])
+def test_sixteen_waves(waves, monkeypatch, capfd):
+    monkeypatch.setenv("SC23AD_RP_WAVES", str(waves))
+    plans = _check(S.CsrMat.generate(S.GEN_POISSON2D, 67), S.SOR, monkeypatch, capfd, block=3)
+    assert any(p[1] == waves for p in plans)
+
+
+@pytest.fixture(scope="module")
+def far_hierarchy():
+    """BlockSOR blocks of 7 1/2 grid lines: the rows of a line's second half
+    depend on the line before, up to 299 levels back.  Entries per row 2, 4,
+    10, 11, 10 on the five levels, far ones 1, 2, 5, 3, 5."""
+    a = S.CsrMat.generate(S.GEN_POISSON2D, 300)
+    a.lmax1_scaling(np.zeros(a.n))
+    return S.Hierarchy(a, S.INT, S.amg_param(S.BLOCK_SOR))
+
+
+@pytest.mark.parametrize("lanes,entries,waves", [
+    (1, 4, 1), (1, 4, 3), (1, 4, 9), (1, 4, 16), (1, 8, 2), (1, 10, 1), (1, 12, 8),
+    (2, 8, 1), (2, 10, 3), (2, 12, 8), (4, 8, 3), (4, 10, 1), (4, 12, 2), (8, 8, 8), (8, 10, 2),
+    (8, 12, 1)])
+def test_far_layouts(lanes, entries, waves, far_hierarchy, monkeypatch, capfd):
+    """Far dependencies over 1-8 lanes, single vectors and blocks (a ring of
+    only what the far rule leaves to it; factors whose rows are longer than the
+    forced layout take other kernels)."""
+    monkeypatch.setenv("SC23AD_RP_RING_FAR", "1")
+    monkeypatch.setenv("SC23AD_RP_LANES", str(lanes))
+    monkeypatch.setenv("SC23AD_RP_ENTRIES", str(entries))
+    monkeypatch.setenv("SC23AD_RP_WAVES", str(waves))
+    plans = _check_hierarchy(far_hierarchy, monkeypatch, capfd, S.INT, 5)
+    got = [p[5] for p in plans if (p[1], p[2], p[3]) == (waves, entries, lanes)]
+    assert 1 in got and 2 in got  # one far entry per row has kernels of its own
+    assert lanes * entries < 10 or 5 in got
 
 
 @pytest.mark.parametrize("prec", [S.FP64, S.FP32], ids=["fp64", "fp32"])
@@ -134,5 +167,18 @@ def test_forced_fp_layouts(lanes, waves, prec, monkeypatch, capfd):
 @pytest.mark.parametrize("smoother", [S.SOR, S.BLOCK_SOR], ids=["sor", "block"])
 def test_fp_far_dependencies_small_ring(smoother, prec, monkeypatch, capfd):
     monkeypatch.setenv("SC23AD_FP_RING_FAR", "1")
-    _check(S.CsrMat.generate(S.GEN_DIFFUSION27, 29, 5, 1.0, 1.0, 1e-3, 3), smoother, monkeypatch,
-           capfd, prec)
+    # 1.2 planes per BlockSOR block: rows in the second one depend on rows of the
+    # first many levels back, as the coarse levels of the SOR hierarchy do
+    plans = _check(S.CsrMat.generate(S.GEN_DIFFUSION27, 48 if smoother == S.BLOCK_SOR else 29, 5,
+                                     1.0, 1.0, 1e-3, 3), smoother, monkeypatch, capfd, prec)
+    assert any(p[5] > 0 for p in plans)
+
+
+@pytest.mark.parametrize("prec", [S.FP64, S.FP32], ids=["fp64", "fp32"])
+@pytest.mark.parametrize("lanes", [1, 2, 4, 8, 16])
+def test_fp_far_layouts(lanes, prec, monkeypatch, capfd):
+    monkeypatch.setenv("SC23AD_FP_RING_FAR", "1")
+    monkeypatch.setenv("SC23AD_RP_LANES", str(lanes))
+    plans = _check(S.CsrMat.generate(S.GEN_POISSON2D, 300), S.BLOCK_SOR, monkeypatch, capfd, prec)
+    got = {p[5] for p in plans if p[3] == lanes and p[1] > 0}
+    assert {1, 2} <= got and (lanes == 1 or 5 in got)
