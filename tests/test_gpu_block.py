@@ -6,11 +6,10 @@ gmres.hpp:225-271) must give every right-hand side exactly what its own
 single solve gives: every V-cycle output bit for bit against the oracle, and
 for whole solves x, the iteration count, the status, the V-cycle checksum
 trace and the residual history against both the single device solve and the
-oracle.  Cases: the 4-RHS groups padded (k = 1, 3, 5), SOR hierarchies whose
-LD solves have no block kernel (one right-hand side at a time inside the
-block V-cycle), right-hand sides that converge at different steps and
-restarts, one that overflows, and a batch of block solvers over systems of
-different sizes.
+oracle.  Cases: the 4-RHS groups padded (k = 1, 3, 5), SOR hierarchies, LD
+solves without a block kernel (one right-hand side at a time inside the block
+V-cycle), right-hand sides that converge at different steps and restarts, one
+that overflows, and a batch of block solvers over systems of different sizes.
 """
 from __future__ import annotations
 
@@ -75,6 +74,23 @@ def test_block_vcycle_matches_oracle(golden, case, smoother, k):
     # twice: no state left behind between calls
     outs2 = S.precondition_block(amg, vins[::-1].copy())
     assert np.array_equal(outs2, outs[::-1])
+
+
+@pytest.mark.parametrize("k", [1, 5])
+@pytest.mark.parametrize("smoother", [S.SOR, S.BLOCK_SOR], ids=["sor", "block"])
+def test_block_vcycle_one_vector_at_a_time(smoother, k, monkeypatch):
+    """LD solves that have no block kernel (here: the row-parallel layouts are
+    switched off) take the right-hand sides of a block one by one."""
+    monkeypatch.setenv("SC23AD_TRI_RP", "0")
+    a = _scaled(S.GEN_LAPLACE3D, (17,))
+    h = S.Hierarchy(a, S.INT, S.amg_param(smoother))
+    amg, oh = S.Amg(h), _oracle(h)
+    assert not S.block_native(amg)
+    v = np.random.default_rng(k).integers(-(2**29), 2**29, (k, a.n)).astype(np.int32)
+    for _ in range(2):
+        out = S.precondition_block(amg, v)
+        for r in range(k):
+            assert np.array_equal(out[r], oh.vcycle(v[r])), r
 
 
 def _free_mib():

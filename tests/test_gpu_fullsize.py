@@ -235,8 +235,8 @@ def test_inclusions160_matches_reference(rhs):
 def test_block_vcycle_inclusions160():
     """The block V-cycle on the 160^3 inclusions hierarchy (five right-hand
     sides) gives every right-hand side its single V-cycle; every level runs
-    on block kernels, including the ones whose rows span several lanes and
-    read far dependencies from global memory."""
+    on block kernels, some with rows over several lanes and some (one lane per
+    row) with far dependencies read from global memory."""
     a, _, amg_i, _ = _incl160()
     rng = np.random.default_rng(13)
     vins = rng.integers(-(2**29), 2**29, (5, a.n)).astype(np.int32)
