@@ -40,10 +40,14 @@ def test_gradient_at_tile_edges(batch):
     x = rng.uniform(0.0, 1.5, (batch, 8)).astype(np.float32)
     t = rng.random((batch, 2)).astype(np.float32)
     lo, go = MO.loss_grad(m.params(), x, t)
+    first = None
     for _ in range(2):  # the second call finds the first one's partial sums
         loss, g = m.grad(x, t)
         assert abs(loss - lo) <= 1e-5 * lo
         np.testing.assert_allclose(g, go, rtol=1e-4, atol=1e-5 * np.abs(go).max())
+        # every sum has a fixed order: the same bits again
+        first = first or (loss, g.tobytes())
+        assert (loss, g.tobytes()) == first
 
 
 def test_training_fits_a_smooth_target():
