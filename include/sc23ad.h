@@ -240,11 +240,11 @@ int sc23ad_solve_batch(int count, sc23ad_solver* const* solvers, const double* c
    per Restarted::Solve (Work/main.cpp:167-169).  Up to SC23AD_BLOCK_MAX_RHS
    integer solves on one hierarchy run in lockstep: every V-cycle
    (INTAMG.hpp:269-293), fine-level SpMV and Gram-Schmidt pass of the step
-   is one launch for all of them, so the matrices and level schedules are
-   read once per step and the sequential levels of the LD solves
-   (ldtri.hpp:511-525) are walked once for four right-hand sides per
-   workgroup.  Each right-hand side's results (x, iterations, statuses) are
-   those of its own sc23ad_solver_solve, bit for bit. */
+   is one launch for all of them: a matrix is read once for up to 16 of them,
+   and the sequential levels of the LD solves (ldtri.hpp:511-525) are walked
+   by a workgroup per BlockSOR block and right-hand side, side by side.  Each
+   right-hand side's results (x, iterations, statuses) are those of its own
+   sc23ad_solver_solve, bit for bit. */
 #define SC23AD_BLOCK_MAX_RHS 64
 typedef struct sc23ad_block_solver_s sc23ad_block_solver;
 /* One V-cycle on nrhs vectors in the block layout: element (row i, vector r)

@@ -1243,7 +1243,7 @@ void tune_spmv(DevMat& m, Elem e, SpmvMode mode) {
       csr.group = g;
       cands.push_back(csr);
     }
-    // streamed through LDS: one to four tiles of 2048 entries per workgroup
+    // streamed through LDS: half a tile of 2048 entries to four per workgroup
     for (int r = 16; r <= 256; r *= 2)
       if (r * avg >= 1024 && r * avg <= 8192) {
         dev::DCsr st = csr;

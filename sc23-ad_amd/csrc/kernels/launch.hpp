@@ -83,10 +83,6 @@ struct TriSegment {
   int row_begin, row_end;
   int group = 1;  // chain_kernel 0, integer factors: lanes per row (power of two <= 64)
 };
-hipError_t launch_trsv_segment(Elem e, TriKind kind, const DCsr& a,
-                               const int* perm, const int* lev_ptr,
-                               const TriSegment& seg, const void* in, void* out,
-                               hipStream_t s);
 
 // Level-ordered layout of a triangular factor (see k_tri_chain_pre): row
 // lrow[idx] at position idx, its dependency entries lcol/lval[lbeg[idx] ..
@@ -165,9 +161,6 @@ inline size_t rp_lds_bytes(int ring, int maxlev) {
   return sizeof(int32_t) * static_cast<size_t>(ring) +
          sizeof(int) * (static_cast<size_t>(maxlev) + 1 + kRpPadLevels);
 }
-// ---- block kernels (block.hip): several right-hand sides of one hierarchy --
-// A block vector of n rows and `groups` groups of four right-hand sides holds
-// element (row i, right-hand side r) at ((r / 4) * n + i) * 4 + r % 4.
 // LDS of the FP row-parallel LD solve (see k_tri_chain_rpf).
 constexpr int kRpfReadAhead = 3 * 8 * 8;  // bytes read past the last row's products
 inline size_t rpf_lds_bytes(size_t elem, int ring, int waves, int lanes, int e, int maxlev) {
@@ -178,6 +171,9 @@ inline size_t rpf_lds_bytes(size_t elem, int ring, int waves, int lanes, int e, 
   return elem * static_cast<size_t>(ring) + 16 + stage +
          2 * sizeof(int) * (static_cast<size_t>(maxlev) + 1 + kRpPadLevels);
 }
+// ---- block kernels: several right-hand sides of one hierarchy ---------------
+// A block vector of n rows and `groups` groups of four right-hand sides holds
+// element (row i, right-hand side r) at ((r / 4) * n + i) * 4 + r % 4.
 hipError_t launch_permute_blk(int n, int groups, const int* perm, const void* src, void* dst,
                               bool gather, hipStream_t s);
 hipError_t launch_copy_blk(int n, int groups, const void* src, void* dst, hipStream_t s);

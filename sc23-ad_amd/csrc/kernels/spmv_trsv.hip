@@ -503,133 +503,7 @@ hipError_t spmv_fp(const DCsr& a, const void* x, const void* z, void* y,
   return hipGetLastError();
 }
 
-// ---- triangular rows --------------------------------------------------------
-
-template <TriKind K>
-__device__ __forceinline__ int32_t tri_row_int(int i, const int* __restrict__ rptr,
-                                               const int* __restrict__ cind,
-                                               const int32_t* __restrict__ v,
-                                               int bit, int dbit,
-                                               const int32_t* __restrict__ in,
-                                               const int32_t* out) {
-  const int rb = rptr[i], re = rptr[i + 1];
-  uint64_t t = static_cast<uint64_t>(static_cast<int64_t>(in[i])) << bit;
-  if (K == TriKind::kLD) {
-    for (int p = rb; p < re - 1; ++p) t -= prod64(v[p], out[cind[p]]);
-    return low32(mul_wrap(as_i64(t) >> bit, v[re - 1]) >> dbit);
-  } else if (K == TriKind::kL) {
-    for (int p = rb; p < re; ++p) t -= prod64(v[p], out[cind[p]]);
-    return low32(as_i64(t) >> bit);
-  } else {
-    for (int p = re - 1; p >= rb + 1; --p) t -= prod64(v[p], out[cind[p]]);
-    return low32(mul_wrap(as_i64(t) >> bit, v[rb]) >> dbit);
-  }
-}
-
-template <TriKind K, typename T>
-__device__ __forceinline__ T tri_row_fp(int i, const int* __restrict__ rptr,
-                                        const int* __restrict__ cind,
-                                        const T* __restrict__ v,
-                                        const T* __restrict__ in, const T* out) {
-  const int rb = rptr[i], re = rptr[i + 1];
-  T t = in[i];
-  if (K == TriKind::kLD) {
-    int p = rb;
-    for (; p < re - 1; ++p) t -= v[p] * out[cind[p]];
-    return t * v[p];
-  } else if (K == TriKind::kL) {
-    for (int p = rb; p < re; ++p) t -= v[p] * out[cind[p]];
-    return t;
-  } else {
-    int p = re - 1;
-    for (; p >= rb + 1; --p) t -= v[p] * out[cind[p]];
-    return t * v[p];
-  }
-}
-
-template <typename T, TriKind K>
-struct Row;
-template <TriKind K>
-struct Row<int32_t, K> {
-  __device__ static int32_t eval(int i, const int* rptr, const int* cind,
-                                 const void* v, int bit, int dbit,
-                                 const int32_t* in, const int32_t* out) {
-    return tri_row_int<K>(i, rptr, cind, static_cast<const int32_t*>(v), bit,
-                          dbit, in, out);
-  }
-};
-template <TriKind K>
-struct Row<double, K> {
-  __device__ static double eval(int i, const int* rptr, const int* cind,
-                                const void* v, int, int, const double* in,
-                                const double* out) {
-    return tri_row_fp<K, double>(i, rptr, cind, static_cast<const double*>(v), in,
-                                 out);
-  }
-};
-template <TriKind K>
-struct Row<float, K> {
-  __device__ static float eval(int i, const int* rptr, const int* cind,
-                               const void* v, int, int, const float* in,
-                               const float* out) {
-    return tri_row_fp<K, float>(i, rptr, cind, static_cast<const float*>(v), in,
-                                out);
-  }
-};
-
 constexpr int kChainBlock = 512;
-
-// One workgroup per chain; levels of the chain one after another, separated
-// by a workgroup barrier (rows of a level only read rows of earlier levels).
-template <typename T, TriKind K>
-__global__ __launch_bounds__(kChainBlock) void k_tri_chain(
-    const int* __restrict__ rptr, const int* __restrict__ cind, const void* val,
-    int bit, int dbit, const int* __restrict__ perm,
-    const int* __restrict__ lev_ptr, const int* __restrict__ chain_lev,
-    const T* __restrict__ in, T* out) {
-  const int lb = chain_lev[2 * blockIdx.x], le = chain_lev[2 * blockIdx.x + 1];
-  for (int L = lb; L < le; ++L) {
-    const int s = lev_ptr[L], e = lev_ptr[L + 1];
-    for (int idx = s + threadIdx.x; idx < e; idx += kChainBlock) {
-      const int i = perm[idx];
-      out[i] = Row<T, K>::eval(i, rptr, cind, val, bit, dbit, in, out);
-    }
-    __syncthreads();
-  }
-}
-
-// All rows of one level, many workgroups.
-template <typename T, TriKind K>
-__global__ __launch_bounds__(kBlock) void k_tri_level(
-    const int* __restrict__ rptr, const int* __restrict__ cind, const void* val,
-    int bit, int dbit, const int* __restrict__ perm, int row_begin, int row_end,
-    const T* __restrict__ in, T* out) {
-  const int idx = row_begin + blockIdx.x * kBlock + threadIdx.x;
-  if (idx >= row_end) return;
-  const int i = perm[idx];
-  out[i] = Row<T, K>::eval(i, rptr, cind, val, bit, dbit, in, out);
-}
-
-template <typename T, TriKind K>
-hipError_t tri_seg(const DCsr& a, const int* perm, const int* lev_ptr,
-                   const TriSegment& seg, const void* in, void* out,
-                   hipStream_t s) {
-  if (seg.chain_kernel) {
-    if (seg.nchain <= 0) return hipSuccess;
-    hipLaunchKernelGGL((k_tri_chain<T, K>), dim3(seg.nchain), dim3(kChainBlock), 0,
-                       s, a.rptr, a.cind, a.val, a.bit, a.dbit, perm, lev_ptr,
-                       seg.chain_lev, static_cast<const T*>(in),
-                       static_cast<T*>(out));
-  } else {
-    const int rows = seg.row_end - seg.row_begin;
-    if (rows <= 0) return hipSuccess;
-    hipLaunchKernelGGL((k_tri_level<T, K>), dim3((rows + kBlock - 1) / kBlock),
-                       dim3(kBlock), 0, s, a.rptr, a.cind, a.val, a.bit, a.dbit,
-                       perm, seg.row_begin, seg.row_end, static_cast<const T*>(in),
-                       static_cast<T*>(out));
-  }
-  return hipGetLastError();
-}
 
 // ---- blocked single-workgroup solve for the coarsest grid ------------------
 //
@@ -2361,17 +2235,6 @@ hipError_t tri_pre_seg(const TriLayout& L, const TriSegment& seg, int bit, int d
   return hipGetLastError();
 }
 
-template <typename T>
-hipError_t tri_kind(TriKind kind, const DCsr& a, const int* perm,
-                    const int* lev_ptr, const TriSegment& seg, const void* in,
-                    void* out, hipStream_t s) {
-  switch (kind) {
-    case TriKind::kLD: return tri_seg<T, TriKind::kLD>(a, perm, lev_ptr, seg, in, out, s);
-    case TriKind::kL: return tri_seg<T, TriKind::kL>(a, perm, lev_ptr, seg, in, out, s);
-    default: return tri_seg<T, TriKind::kDU>(a, perm, lev_ptr, seg, in, out, s);
-  }
-}
-
 }  // namespace
 
 template <typename T, int MODE>
@@ -2604,15 +2467,6 @@ hipError_t launch_trsv_rpf(Elem e, const TriLayout& L, const void* in, void* out
   if (e == Elem::kF32)
     return tri_rpf<float>(L, static_cast<const float*>(in), static_cast<float*>(out), s);
   return hipErrorInvalidValue;
-}
-
-hipError_t launch_trsv_segment(Elem e, TriKind kind, const DCsr& a,
-                               const int* perm, const int* lev_ptr,
-                               const TriSegment& seg, const void* in, void* out,
-                               hipStream_t s) {
-  if (e == Elem::kI32) return tri_kind<int32_t>(kind, a, perm, lev_ptr, seg, in, out, s);
-  if (e == Elem::kF64) return tri_kind<double>(kind, a, perm, lev_ptr, seg, in, out, s);
-  return tri_kind<float>(kind, a, perm, lev_ptr, seg, in, out, s);
 }
 
 }  // namespace sc23ad::dev
