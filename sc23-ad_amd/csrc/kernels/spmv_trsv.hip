@@ -1445,14 +1445,15 @@ hipError_t tri_ep_launch(const TriLayout& L, const TriSegment& seg, int bit, int
 //  * shifts by bit and dbit (0..30) are single 32-bit funnel shifts, and the
 //    finish takes one 32 x 32 product and one low product.
 // Measured per solve against the form that masked ring positions and computed
-// addresses per level (128^3 BlockSOR, levels 1-4: 83 / 78 / 92 / 43 us, now
-// 80 / 64 / 62 / 29 us; level 0: 87 -> 82 us) and against the entry-parallel
-// kernel and one launch per wide level (63^3 SOR, whole V-cycle: 5.27 -> 2.61 ms).
+// addresses per level (128^3 BlockSOR, levels 0-4: 87 / 83 / 78 / 92 / 43 us,
+// now 80 / 82 / 57 / 55 / 27; with scalar offsets 82 / 80 / 64 / 62 / 29) and
+// against the entry-parallel kernel and one launch per wide level (63^3 SOR,
+// whole V-cycle: 5.27 -> 2.50 ms).
 // A block of right-hand sides runs one workgroup per chain and right-hand side
 // (a chain leaves most of the chip idle: 40 chains, 256 CUs), all of one chain
 // on one XCD when the chain count is a multiple of 8; four right-hand sides
 // per workgroup, which loads each entry once, took 1.9 ms of LD solves per
-// 16-vector V-cycle of the 96^3 inclusions system, against 1.1 ms.
+// 16-vector V-cycle of the 96^3 inclusions system, against 0.95 ms.
 using RpWord4 = __attribute__((ext_vector_type(4))) unsigned;
 template <int kE, int kFq>
 struct RpPre {
