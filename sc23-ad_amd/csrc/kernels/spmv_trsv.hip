@@ -189,8 +189,9 @@ __global__ __launch_bounds__(kBlock) void k_spmv_stream_int(
         first += __popcll(__ballot(mine && rp[r + 1] <= p0));
         last += __popcll(__ballot(mine && rp[r] - p0 < kTile));
       }
-      // 2^lg lanes for each of them (at least kLanes: there are kRows at most)
-      const int lg = 31 - __clz(kBlock / (last - first));
+      // 2^lg lanes for each of them (at least kLanes: there are kRows at most;
+      // one or more, unless the row pointers do not ascend)
+      const int lg = 31 - __clz(kBlock / max(last - first, 1));
       const int g = t >> lg, part = t & ((1 << lg) - 1);
       const int mine = min(first + g, nr - 1);
       const int lo = max(rp[mine] - p0, 0);
