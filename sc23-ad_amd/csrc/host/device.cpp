@@ -1382,8 +1382,10 @@ std::unique_ptr<DevAmg::Work> DevAmg::make_work() const {
   }
   w->err.alloc(sizeof(int));
   w->err.upload(zero.data(), sizeof(int));
-  w->tickets.alloc(4 * sizeof(unsigned));
-  w->tickets.upload(zero.data(), 4 * sizeof(unsigned));
+  // a ticket that does not start at zero names a block that does not exist
+  const unsigned tickets[4] = {0, 0, 0, 0};
+  w->tickets.alloc(sizeof(tickets));
+  w->tickets.upload(tickets, sizeof(tickets));
   return w;
 }
 

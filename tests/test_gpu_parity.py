@@ -117,6 +117,31 @@ def test_default_frac_bits(built):
             assert amg.default_frac_bits(sy.b, sy.nrm_b) == c["solves"][f"2_{smoother}"]["bit"]
 
 
+@pytest.mark.parametrize("prec", [S.INT, S.FP64, S.FP32], ids=["int", "fp64", "fp32"])
+@pytest.mark.parametrize("kind,n", [(S.GEN_POISSON2D, 2), (S.GEN_POISSON2D, 8),
+                                    (S.GEN_LAPLACE3D, 7)])
+def test_one_coarse_row(kind, n, prec):
+    """Coarsened down to one row: the coarse solves' counters start at zero
+    however small the vectors beside them are (several hierarchies, since what
+    else the counters could start at is whatever the host heap holds)."""
+    a = S.CsrMat.generate(kind, n)
+    a.lmax1_scaling(np.zeros(a.n))
+    h = S.Hierarchy(a, prec, S.amg_param(S.SOR, coarse_n=1))
+    path = export(h)
+    oh = O.OracleHier(path)
+    os.unlink(path)
+    rng = np.random.default_rng(41)
+    for _ in range(8):
+        amg = S.Amg(h)
+        assert oh.level_n(amg.depth) == 1
+        c = _rand(prec, 1, rng)
+        assert _same(amg.level_op(amg.depth, S.OP_COARSE, c, 1),
+                     oh.level_op(amg.depth, S.OP_COARSE, c, 1))
+        v = _rand(prec, a.n, rng)
+        for _ in range(2):
+            assert _same(amg.precondition(v), oh.vcycle(v))
+
+
 @pytest.mark.parametrize("fmt", ["csr", "sell", "sell16", "sellcol"])
 def test_spmv_formats_match_oracle(fmt, monkeypatch):
     """Every SpMV kernel the tuner can pick (CSR with 1-64 lanes, SELL-64,
