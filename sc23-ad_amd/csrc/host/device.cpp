@@ -383,6 +383,19 @@ bool padded_too_far(int n, int slots, size_t entries, size_t entry_bytes) {
          padded > 32.0 * static_cast<double>(entries);
 }
 
+// The least LDS ring, in values: one for every row that a kernel solves
+// between two barriers (at most `cap` of a level).  Rows a ring apart share a
+// slot, and those of one piece are written in no order; between pieces the
+// later one, which is the one still needed, is written last.
+int least_ring(const std::vector<int>& lev_ptr, int cap) {
+  int rows = 1;
+  for (size_t Lv = 0; Lv + 1 < lev_ptr.size(); ++Lv)
+    rows = std::max(rows, std::min(cap, lev_ptr[Lv + 1] - lev_ptr[Lv]));
+  int r = 4;
+  while (r < rows) r *= 2;
+  return r;
+}
+
 // What the entry-parallel kernel takes for a chain's levels, in ns, from its
 // mean entries and rows per level: fitted to its solves of 27-point 48^3, 64^3
 // and 80^3, 7-point 63^3 and 48^3-inclusions SOR hierarchies and the 27-point
@@ -450,13 +463,14 @@ double plan_rp(TriPlan& plan, int n, const std::vector<int>& lbeg, const std::ve
   // LDS ring: a dependency is read from it when no later position of its
   // level's end has overwritten it, else (at least kEpFarLevels levels back)
   // from global memory
-  int ring = 2;
+  const int least = least_ring(lev_ptr, 64 * dev::kRpMaxWaves);
+  int ring = least;
   while (ring < 32768 && ring < span) ring *= 2;
   std::vector<int> lev_of(static_cast<size_t>(n));
   for (int Lv = 0; Lv < nlev; ++Lv)
     for (int idx = lev_ptr[Lv]; idx < lev_ptr[Lv + 1]; ++idx) lev_of[idx] = Lv;
   if (std::getenv("SC23AD_RP_RING_FAR"))
-    ring = std::min(ring, smallest_ring(2, n, lbeg, lpos, lev_ptr, lev_of));
+    ring = std::min(ring, smallest_ring(least, n, lbeg, lpos, lev_ptr, lev_of));
   auto is_far = [&](int idx, int dpos) {
     return static_cast<long long>(lev_ptr[lev_of[idx] + 1]) - dpos > ring;
   };
@@ -580,10 +594,11 @@ void plan_rpf(TriPlan& plan, int n, const std::vector<int>& lbeg, const std::vec
   const int md = *std::max_element(lev_md.begin(), lev_md.end());
   // LDS ring of at most 128 KB; further dependencies, at least kEpFarLevels
   // levels back, come from global memory
-  int ring = 4;
+  const int least = least_ring(lev_ptr, 64 * dev::kRpfMaxWaves);
+  int ring = least;
   while (ring * 2 * kT <= 128 * 1024 && ring < span) ring *= 2;
   if (std::getenv("SC23AD_FP_RING_FAR"))
-    ring = std::min(ring, smallest_ring(4, n, lbeg, lpos, lev_ptr, lev_of));
+    ring = std::min(ring, smallest_ring(least, n, lbeg, lpos, lev_ptr, lev_of));
   auto is_far = [&](int idx, int dpos) {
     return static_cast<long long>(lev_ptr[lev_of[idx] + 1]) - dpos > ring;
   };
@@ -605,7 +620,7 @@ void plan_rpf(TriPlan& plan, int n, const std::vector<int>& lbeg, const std::vec
           static_cast<uint64_t>(n) * g * e * kT > dev::kRpMaxBytes ||
           padded_too_far(n, g * e, lpos.size(), 4 + kT))
         continue;
-      for (int w = 1; w <= 8; ++w) {
+      for (int w = 1; w <= dev::kRpfMaxWaves; ++w) {
         if (only_waves > 0 && w != only_waves) continue;
         const int cap = 64 * w / g;
         if (cap == 0) continue;
@@ -862,14 +877,14 @@ void build_plan(TriPlan& plan, TriKind kind, int n, const std::vector<int>& rptr
   // Entry-parallel mode (integer factors): a dependency is read from the LDS
   // ring when the ring holds it, else from global memory, which needs it at
   // least kEpFarLevels levels back.  The ring is the smallest power of two
-  // that holds every dependency, at most 32768 values.
+  // that holds every dependency and a level's rows, at most 32768 values.
   size_t maxlev_rows = 0;
   for (size_t Lv = 0; Lv + 1 < lev_ptr.size(); ++Lv)
     maxlev_rows = std::max<size_t>(maxlev_rows, lev_ptr[Lv + 1] - lev_ptr[Lv]);
   int maxlev_chain = 0;
   for (size_t c = 0; c + 1 < all_chain_lev.size(); c += 2)
     maxlev_chain = std::max(maxlev_chain, all_chain_lev[c + 1] - all_chain_lev[c]);
-  int ep_ring = 2;
+  int ep_ring = least_ring(lev_ptr, dev::kEpMaxRows);
   while (ep_ring < 32768 && ep_ring < span) ep_ring *= 2;
   // Accumulator copies (LD factors only) where one instruction's lanes pile
   // onto few rows: rows averaging at least 8 dependency entries and levels

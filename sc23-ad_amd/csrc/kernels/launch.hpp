@@ -147,6 +147,7 @@ hipError_t launch_trsv_ep(TriKind kind, const TriLayout& L, const TriSegment& se
 // Row-parallel integer LD solve (one workgroup per chain, 1-64 lanes per row).
 constexpr int kRpMaxLanes = 64;   // lanes per row, 4 to 12 entries each
 constexpr int kRpMaxWaves = 16;   // more than 8: one lane of 4 entries per row
+constexpr int kRpfMaxWaves = 8;   // FP
 constexpr int kRpFarSlots = 4;    // far entries per lane of layouts over several lanes
 constexpr int kRpMaxAhead = 4;    // far values are loaded at most this many levels ahead
 constexpr int kRpPadLevels = 12;  // level offsets past a chain's last one

@@ -2121,7 +2121,7 @@ hipError_t tri_rpf_layout(const TriLayout& L, const T* in, T* out, hipStream_t s
 
 template <typename T>
 hipError_t tri_rpf(const TriLayout& L, const T* in, T* out, hipStream_t s) {
-  if (L.rp_waves < 1 || L.rp_waves > 8) return hipErrorInvalidValue;
+  if (L.rp_waves < 1 || L.rp_waves > kRpfMaxWaves) return hipErrorInvalidValue;
   if (L.rp_lanes > 1)
     return L.rp_waves == 1 ? tri_rpf_layout<T, 1, true>(L, in, out, s)
                            : tri_rpf_layout<T, 8, true>(L, in, out, s);

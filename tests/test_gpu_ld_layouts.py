@@ -82,6 +82,49 @@ def test_entry_parallel_where_few_rows_are_long(monkeypatch, capfd):
     assert all(p[1] > 0 for p in plans)
 
 
+def _wide_level_short_reach(n=1000, first=970, reach=25):
+    """`first` rows without dependencies, then rows that depend on the last
+    `reach` of them: a level many times wider than any dependency reaches."""
+    rng = np.random.default_rng(5)
+    at = [(k, int(d)) for k in range(first, n)
+          for d in rng.choice(np.arange(first - reach, first), 3, replace=False)]
+    m = np.zeros((n, n))
+    for k, d in at:
+        m[k, d] = m[d, k] = -rng.uniform(0.5, 1.0)
+    m[np.arange(n), np.arange(n)] = 1.0 - m.sum(1)
+    i, j = np.nonzero(m)
+    rptr = np.searchsorted(i, np.arange(n + 1)).astype(np.int32)
+    return S.CsrMat.from_arrays(n, rptr, j.astype(np.int32), m[i, j])
+
+
+@pytest.mark.parametrize("prec", [S.INT, S.FP64, S.FP32], ids=["int", "fp64", "fp32"])
+@pytest.mark.parametrize("knobs", [{}, {"SC23AD_TRI_RP": "0"}, {"SC23AD_RP_WAVES": "1"},
+                                   {"SC23AD_RP_WAVES": "8"}, {"SC23AD_RP_RING_FAR": "1",
+                                                              "SC23AD_FP_RING_FAR": "1"}],
+                         ids=["plan", "other-kernels", "one-wave", "eight-waves", "least-ring"])
+def test_level_wider_than_the_reach(knobs, prec, monkeypatch, capfd):
+    """The ring holds at least the rows that are solved between two barriers,
+    also where the dependencies need less: rows a ring apart share a slot."""
+    for k, v in knobs.items():
+        monkeypatch.setenv(k, v)
+    a = _wide_level_short_reach()
+    a.lmax1_scaling(np.zeros(a.n))
+    h = S.Hierarchy(a, prec, S.amg_param(S.SOR, coarse_n=64))
+    for _ in range(4):
+        _check_hierarchy(h, monkeypatch, capfd, prec, 3 if prec == S.INT else 0)
+
+
+@pytest.mark.parametrize("prec", [S.INT, S.FP64, S.FP32], ids=["int", "fp64", "fp32"])
+def test_jacobi_sor_levels_wider_than_the_reach(prec, monkeypatch, capfd):
+    """JacobiSOR blocks of 1,200 rows: two levels, the second of 31 rows that
+    depend on the last of the first."""
+    a = S.CsrMat.generate(S.GEN_CONVDIFF2D, 94, 24.14150207068065, 5.948711626198889)
+    a.lmax1_scaling(np.zeros(a.n))
+    h = S.Hierarchy(a, prec, S.amg_param(S.JACOBI_SOR, coarse_n=300))
+    for _ in range(4):
+        _check_hierarchy(h, monkeypatch, capfd, prec, 0)
+
+
 @pytest.mark.parametrize("prec", [S.INT, S.FP64, S.FP32], ids=["int", "fp64", "fp32"])
 def test_one_long_row_is_not_padded_to(prec, monkeypatch, capfd):
     """A 5-point system of 48,400 rows whose last row has 400 entries more (in
