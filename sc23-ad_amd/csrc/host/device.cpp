@@ -567,6 +567,24 @@ double plan_rp(TriPlan& plan, int n, const std::vector<int>& lbeg, const std::ve
   return rp_cost_of(best_pieces, best_w, best_e, best / static_cast<double>(best_pieces));
 }
 
+// What the level-pipelined kernel (k_tri_chain_pre, a thread per row) takes for
+// its longest chain, in ns: 700 per level, 115 per entry of the level's longest
+// row past the 8 that are loaded ahead, and 2,500 where the level's rows need
+// a second round.  7-point 63^3 SOR in FP64, levels of longest rows 9 / 28 / 80
+// / 127 / 284: 2.1 / 4.7 / 8.1 / 7.1 / 15.9 us per level.
+double pre_cost(const std::vector<int>& lev_ptr, const std::vector<int>& lev_md,
+                const std::vector<int>& chain_lev) {
+  double most = 0;
+  for (size_t c = 0; c + 1 < chain_lev.size(); c += 2) {
+    double t = 0;
+    for (int Lv = chain_lev[c]; Lv < chain_lev[c + 1]; ++Lv)
+      t += 700 + 115.0 * std::max(0, lev_md[Lv] - 8) +
+           (lev_ptr[Lv + 1] - lev_ptr[Lv] > 512 ? 2500 : 0);
+    most = std::max(most, t);
+  }
+  return most;
+}
+
 // Row-parallel layout of an FP smoother factor (k_tri_chain_rpf): as plan_rp,
 // with the row's ordered subtractions in the cost of a piece,
 //   70 + 10 e + (waves - 1) (2 + 4.5 e elem / 4)                 one lane
@@ -575,7 +593,8 @@ double plan_rp(TriPlan& plan, int n, const std::vector<int>& lbeg, const std::ve
 template <typename V>
 void plan_rpf(TriPlan& plan, int n, const std::vector<int>& lbeg, const std::vector<int>& lpos,
               const std::vector<V>& lval, const std::vector<int>& lev_ptr,
-              const std::vector<int>& chain_lev, long long span, int single_wg_max) {
+              const std::vector<int>& chain_lev, long long span, int single_wg_max,
+              bool one_launch) {
   const char* env_rp = std::getenv("SC23AD_TRI_RP");
   if ((env_rp && env_rp[0] == '0') || n <= 0 || n >= (1 << 27)) return;
   auto forced = [](const char* name) {
@@ -653,6 +672,12 @@ void plan_rpf(TriPlan& plan, int n, const std::vector<int>& lbeg, const std::vec
       }
     }
   if (best_w == 0 || (nchain == 1 && segmented_wins(lev_ptr, single_wg_max, best))) return;
+  // the level-pipelined kernel, whose work does not grow with the factor's
+  // longest row, where it is clearly faster (13,795 rows of 11 entries and one
+  // of 160: 32 lanes per row, 1,445 pieces, 1,155 us against 555)
+  if (one_launch && !env_rp && only_lanes <= 0 && only_waves <= 0 &&
+      pre_cost(lev_ptr, lev_md, chain_lev) < 0.8 * best)
+    return;
   const std::vector<int> ptr = put_pieces(plan, lev_ptr, chain_lev, 64 * best_w / best_g);
   std::vector<int> steps(std::max<size_t>(ptr.size() - 1, 1), 8);
   for (size_t p = 0; p + 1 < ptr.size(); ++p)
@@ -983,7 +1008,8 @@ void build_plan(TriPlan& plan, TriKind kind, int n, const std::vector<int>& rptr
   // the level-pipelined kernel.
   if constexpr (!std::is_same_v<V, int32_t>) {
     if (kind == TriKind::kLD && plan.identity)
-      plan_rpf(plan, n, lbeg, lpos, lval, lev_ptr, chain_lev, span, single_wg_max);
+      plan_rpf(plan, n, lbeg, lpos, lval, lev_ptr, chain_lev, span, single_wg_max,
+               one_launch_chains);
   }
   int maxdeps = 0;
   for (int idx = 0; idx < n; ++idx) maxdeps = std::max(maxdeps, lbeg[idx + 1] - lbeg[idx]);

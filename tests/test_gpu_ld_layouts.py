@@ -146,6 +146,26 @@ def test_one_long_row_is_not_padded_to(prec, monkeypatch, capfd):
     assert plans[0][0] == n and plans[0][1] == 0
 
 
+@pytest.mark.parametrize("prec", [S.FP64, S.FP32], ids=["fp64", "fp32"])
+def test_fp_level_pipelined_where_few_rows_are_long(prec, monkeypatch, capfd):
+    """Short rows in levels of about 100 and one row of 150 entries: a thread per
+    row beats 32 lanes per row, which would cut every level into ten pieces."""
+    n = 120
+    rptr, cind, val = S.CsrMat.generate(S.GEN_POISSON2D, n).arrays()
+    old = cind[rptr[-2]:]
+    extra = np.setdiff1d(np.arange(n * n - 200, n * n - 50), old).astype(np.int32)
+    cols = np.concatenate([old, extra])
+    order = np.argsort(cols)
+    vals = np.concatenate([val[rptr[-2]:], np.full(len(extra), -2.0**-9)])[order]
+    rptr = rptr.copy()
+    rptr[-1] += len(extra)
+    cut = len(cind) - len(old)
+    a = S.CsrMat.from_arrays(n * n, rptr, np.concatenate([cind[:cut], cols[order]]),
+                             np.concatenate([val[:cut], vals]))
+    plans = _check(a, S.SOR, monkeypatch, capfd, prec)
+    assert plans[0][0] == n * n and plans[0][1] == 0
+
+
 @pytest.mark.parametrize("lanes", [1, 2, 4, 8, 16, 32, 64])
 @pytest.mark.parametrize("waves", [1, 3])
 def test_forced_layouts(lanes, waves, monkeypatch, capfd):
